@@ -348,6 +348,15 @@ int mc3d_diag_stream(mc3d_ctx *ctx, size_t bytes, int32_t write, double *ms);
  * counterpart in the reference; it checks the library's own culling. */
 int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked, uint64_t *mismatches);
 
+/* Diagnostics (host only, no GPU): random spheres, boxes, capsules and
+ * cylinders (aligned, grazed, degenerate, far away, huge) on random lines of
+ * corners and of edge midpoints -- every point that the row form of an atom
+ * calls certainly inside or certainly outside is compared with the atom's
+ * float64 Contains; differing points are counted (must be 0), and the points
+ * it leaves open.  No counterpart in the reference; it checks the interval
+ * bounds the corner and bisection kernels decide whole rows by. */
+int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_t *open, uint64_t *mismatches);
+
 const char *mc3d_last_error(void);
 const char *mc3d_version(void);
 

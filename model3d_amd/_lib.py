@@ -195,6 +195,9 @@ SIGNATURES = {
     "mc3d_selftest_plan_fold": (
         ctypes.c_int, [ctypes.c_uint64, ctypes.c_uint32, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]
     ),
+    "mc3d_selftest_rows": (
+        ctypes.c_int, [ctypes.c_uint64, ctypes.c_uint32] + [ctypes.POINTER(ctypes.c_uint64)] * 3
+    ),
     "mc3d_last_error": (ctypes.c_char_p, []),
     "mc3d_version": (ctypes.c_char_p, []),
 }

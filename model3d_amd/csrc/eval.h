@@ -222,7 +222,7 @@ __device__ __forceinline__ void apply_frame(F64P f64, Frame fr, double &x, doubl
 // Constants that do not depend on the point were computed on the host with
 // the reference's operation order (solid.cpp).
 template <class F64P>
-__device__ __forceinline__ bool atom64(uint32_t kind, F64P a, double x, double y, double z) {
+MC3D_HD inline bool atom64(uint32_t kind, F64P a, double x, double y, double z) {
     switch (kind) {
     case A_SPHERE: {  // Sphere.Contains: coord.Dist(center) <= r, shapes.go:29-31
         double d1 = x - a[0], d2 = y - a[1], d3 = z - a[2];

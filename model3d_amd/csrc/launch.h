@@ -48,6 +48,8 @@ struct Pipe {
     uint32_t plan_gsz = 64;  // bricks per plan wave
     bool plan_tile = false;  // plan waves take compact tiles of bricks (one solid)
     bool scan_one_pass = false;  // classify scans its counts itself (at most SCAN_ONE_PASS blocks)
+    bool rows = false;  // every atom has a row form: corners and bisection decide lines, not points
+    int stack = 1;      // boolean stack entries of the call's programs
     uint32_t emit_div = 1024;  // emit blocks: occupancy words / emit_div, in [512, 4096]
 };
 
@@ -63,7 +65,9 @@ template <>
 hipError_t launch_corners_ms<1, false>(const Pipe &p, const Bufs &b, hipStream_t st);
 template <>
 hipError_t launch_corners_ms<1, true>(const Pipe &p, const Bufs &b, hipStream_t st);
+hipError_t launch_rows(const Pipe &p, const Bufs &b, hipStream_t st);
 inline hipError_t launch_corners(const Pipe &p, const Bufs &b, hipStream_t st) {
+    if (p.rows) return launch_rows(p, b, st);
     if (p.mode == 0) return p.stats ? launch_corners_ms<0, true>(p, b, st) : launch_corners_ms<0, false>(p, b, st);
     return p.stats ? launch_corners_ms<1, true>(p, b, st) : launch_corners_ms<1, false>(p, b, st);
 }

@@ -39,6 +39,7 @@
 #include "launch.h"
 #include "mc3d_internal.h"
 #include "plan.h"
+#include "rows.h"
 
 using namespace mc3d;
 
@@ -532,6 +533,13 @@ int lowered(const mc3d_solid *s, std::shared_ptr<const Lowered> &out) {
             return MC3D_E_UNSUPPORTED;
         }
         L->host = !L->P.host_atoms.empty();
+        L->rows = true;
+        for (uint32_t pc : L->P.atom_pc) {
+            const uint32_t x = L->P.code[pc].x, kind = insn_kind(x);
+            if (insn_frame(x) != 0 ||
+                !(kind == A_SPHERE || kind == A_RECT || kind == A_CAPSULE || kind == A_CYLINDER))
+                L->rows = false;
+        }
         L->frames = host_frames(L->P);
         job_nodes(L->P, L->nodes);
         s->low = std::move(L);
@@ -548,6 +556,11 @@ int layout_job(Job &j, const mc3d_options &o, bool check) {
     g.nx = (int)j.ax[0].size(), g.ny = (int)j.ax[1].size(), g.nz = (int)j.ax[2].size();
     g.W = (g.nx + 63) / 64;
     j.nwords = (uint64_t)g.W * g.ny * g.nz;
+    g.inv_h = 1 / j.delta;
+    g.mag = 0;
+    for (int a = 0; a < 3; a++) g.mag = std::max({g.mag, fabs(j.ax[a].front()), fabs(j.ax[a].back())});
+    // 64 additions of delta, each rounded to half an ulp of the coordinate
+    g.eta = 1e-6 + 1e-11 * g.mag * g.inv_h;
     if (check && j.nwords >= (1ull << 32)) {
         set_error("grid too large: more than 2^32 occupancy words");
         return MC3D_E_UNSUPPORTED;
@@ -989,6 +1002,8 @@ struct Call {
     bool stats = false;
     bool interior = false;  // a call of one MarchingCubesInterior solid
     bool host = false;      // a call of one solid with host-evaluated atoms
+    bool rows = false;      // corners and bisection by rows (every atom has a row form, no statistics)
+    int stack = 1;          // boolean stack entries of the call's programs
     bool bm = false;        // the scan takes the words in brick-major order (one culled solid)
     uint64_t nscan = 0;     // scan positions: words, or brick-major positions
     size_t plan_lds = 0;
@@ -1040,6 +1055,13 @@ int plan_call(std::vector<Job> &jobs, const mc3d_options &o, Call &c) {
         }
     } else {
         for (Job &j : jobs) j.pos0 = j.word0, j.npos = 0;
+    }
+    // Row forms need evenly spaced corners (eta) and finite coordinates;
+    // statistics runs count the evaluations of single points.
+    c.rows = !c.stats && !c.host;
+    for (const Job &j : jobs) {
+        c.rows = c.rows && j.low->rows && j.g.eta < 0.01 && std::isfinite(j.g.inv_h);
+        c.stack = std::max(c.stack, j.low->P.max_stack);
     }
     c.plan_lds = PLAN_STACK_BYTES;
     if (c.cull)
@@ -1106,6 +1128,8 @@ Pipe make_pipe(const Call &c, const Upload &U) {
     p.mode = c.mode;
     p.rows_per_walk = c.rows_per_walk;
     p.wpb = c.wpb;
+    p.rows = c.rows;
+    p.stack = c.stack;
     p.plan_lds = c.plan_lds;
     // Launch shapes measured on MI355X: a single solid's plan waves take
     // compact tiles, 16 bricks for programs that stage in LDS and 64 for the
@@ -2720,6 +2744,96 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
             }
         }
         if (checked) *checked = nchecked;
+        if (mismatches) *mismatches = nbad;
+        return MC3D_OK;
+    });
+}
+
+int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_t *open, uint64_t *mismatches) {
+    for (uint64_t *p : {checked, open, mismatches})
+        if (p) *p = 0;
+    return guarded([&]() -> int {
+        uint64_t state = seed, nchecked = 0, nopen = 0, nbad = 0;
+        auto next = [&]() {  // splitmix64
+            uint64_t z = (state += 0x9E3779B97F4A7C15ull);
+            z = (z ^ (z >> 30)) * 0xBF58476D1CE4E5B9ull;
+            z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
+            return z ^ (z >> 31);
+        };
+        auto uni = [&](double lo, double hi) { return lo + (hi - lo) * (double)(next() >> 11) * 0x1.0p-53; };
+        auto mag10 = [&](double lo, double hi) { return pow(10.0, uni(lo, hi)); };
+        for (uint32_t l = 0; l < lines; l++) {
+            // spacing, and coordinates up to 10^6 spacings from the origin
+            const double h = next() % 4 ? mag10(-4, 0) : pow(2.0, -(double)(next() % 8)), far = h * mag10(0, 6);
+            double c[3], d[3], p[3];
+            for (int a = 0; a < 3; a++) c[a] = uni(-far, far), d[a] = uni(-1, 1);
+            const int k = (int)(next() % 3);
+            const uint64_t tilt = next() % 4;  // along the line, nearly so, or anyhow
+            if (tilt < 2)
+                for (int a = 0; a < 3; a++) d[a] = a == k ? (next() & 1 ? 1 : -1) : (tilt ? uni(-1, 1) * mag10(-12, -2) : 0);
+            const double r = h * mag10(-1, 3), len = next() % 16 ? h * mag10(-1, 3) : 0;
+            const double e[3] = {c[0] + d[0] * len, c[1] + d[1] * len, c[2] + d[2] * len};
+            const uint32_t what = (uint32_t)(next() % 4);
+            const double lo[3] = {std::min(c[0], e[0]), std::min(c[1], e[1]), std::min(c[2], e[2])};
+            const double hi[3] = {std::max(c[0], e[0]), std::max(c[1], e[1]), std::max(c[2], e[2])};
+            mc3d_solid *s = what == 0   ? mc3d_sphere(c, r)
+                            : what == 1 ? mc3d_rect(lo, hi)
+                            : what == 2 ? mc3d_capsule(c, e, r)
+                                        : mc3d_cylinder(c, e, r);
+            if (!s) return MC3D_E_OOM;
+            std::unique_ptr<mc3d_solid, void (*)(mc3d_solid *)> hold(s, mc3d_solid_release);
+            Program P;
+            std::string msg;
+            if (!lower_solid(*s->ptr, P, msg)) {
+                set_error(msg);
+                return MC3D_E_INTERNAL;
+            }
+            const uint32_t kind = insn_kind(P.code[0].x);
+            const double *a = P.f64.data() + P.code[0].y;
+            // a line near the atom, often grazing it or starting on its face
+            for (int q = 0; q < 3; q++) p[q] = uni(lo[q] - r, hi[q] + r);
+            const int o = (k + 1 + (int)(next() & 1)) % 3;
+            if (next() % 4 == 0) p[(k + 1) % 3] = c[(k + 1) % 3], p[(k + 2) % 3] = c[(k + 2) % 3];
+            if (next() % 3 == 0) p[o] = c[o] + r * (1 + (next() & 1 ? 0 : uni(-1, 1) * mag10(-16, -6)));
+            if (next() % 4 == 0) p[k] = (next() & 1 ? lo[k] : hi[k]) - (double)(next() % 60) * h;
+            else p[k] -= uni(0, 64) * h;
+            const bool edge = next() & 1;
+            double pts[64];
+            int last = 63;
+            double scale = 1 / h, smax = 64 * h, mag = 0;
+            if (edge) {  // the 32 dyadic points of one edge, as halvings reach them
+                const double t1 = p[k] + h;
+                last = 31, scale = 32 / (t1 - p[k]), smax = t1 - p[k];
+                pts[0] = p[k];
+                for (int i = 1; i < 32; i++) {
+                    double f = p[k], t = t1, m = 0;
+                    for (int bit = 16, at = 0; bit; bit >>= 1) {
+                        m = (f + t) / 2;
+                        if (at + bit == i) break;
+                        if (i > at + bit) f = m, at += bit;
+                        else t = m;
+                    }
+                    pts[i] = m;
+                }
+            } else {
+                double x = p[k];
+                for (int i = 0; i < 64; i++, x += h) pts[i] = x;
+            }
+            for (int q = 0; q < 3; q++) mag = std::max(mag, fabs(p[q]));
+            mag = std::max(mag, fabs(pts[last]));
+            uint64_t sure, maybe;
+            row_mask(atom_span(kind, a, k, p[0], p[1], p[2], smax, mag), scale, 1e-6 + 1e-11 * mag / h, last, sure,
+                     maybe);
+            for (int i = 0; i <= last; i++) {
+                p[k] = pts[i];
+                const bool in = atom64(kind, a, p[0], p[1], p[2]), yes = sure >> i & 1, may = maybe >> i & 1;
+                nchecked++;
+                nopen += may && !yes;
+                nbad += (yes && !in) || (!may && in);
+            }
+        }
+        if (checked) *checked = nchecked;
+        if (open) *open = nopen;
         if (mismatches) *mismatches = nbad;
         return MC3D_OK;
     });

@@ -224,6 +224,7 @@ struct Lowered {
     std::vector<uint32_t> frames;  // frame of each host-evaluated atom
     std::vector<PlanNode> nodes;   // the brick plan's node records of P (plan_nodes)
     bool host = false;             // some atom is evaluated on the host
+    bool rows = false;             // every atom is an untransformed sphere, box, capsule or cylinder
 };
 }  // namespace mc3d
 

@@ -106,3 +106,17 @@ def test_plan_fold_skip_equals_serial_fold():
     assert L.mc3d_selftest_plan_fold(20240607, 20000, ctypes.byref(checked), ctypes.byref(bad)) == 0
     assert checked.value == 20000 * 16
     assert bad.value == 0
+
+
+def test_row_bounds_match_contains():
+    """The interval bounds by which the row kernels decide whole rows of
+    corners and the midpoints of an edge, against each atom's float64
+    Contains, on the host: no point they call certain may differ."""
+    import ctypes
+
+    L = _lib.lib()
+    checked, opened, bad = ctypes.c_uint64(), ctypes.c_uint64(), ctypes.c_uint64()
+    assert L.mc3d_selftest_rows(77, 300000, ctypes.byref(checked), ctypes.byref(opened), ctypes.byref(bad)) == 0
+    assert checked.value > 300000 * 32
+    assert bad.value == 0
+    assert opened.value < checked.value // 2  # (most points are decided)
