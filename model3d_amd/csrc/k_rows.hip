@@ -20,14 +20,20 @@
 namespace mc3d {
 namespace {
 
+__device__ __forceinline__ RowScale row_scale(const Grid &g) {
+    const auto p = scalar_ptr(g.zs + g.nz);
+    return RowScale{p[0], p[1], p[2], p[3]};
+}
+
 // The corners of one word (from x0, in row (y, z)) that a program holds for.
 template <bool UNI, class CodeP, class F64P>
 __device__ __forceinline__ uint64_t word_bits(CodeP code, uint32_t n, F64P f64, const Grid &g, int x0, int y, int z,
                                               uint64_t *stack) {
+    const RowScale rs = row_scale(g);
     const int last = min(63, g.nx - 1 - x0);
     const double *xs = g.xs + x0;
-    const uint64_t m = row_program<UNI, uint64_t>(code, n, f64, 0, xs[0], g.ys[y], g.zs[z], 64 / g.inv_h, g.mag, g.inv_h,
-                                                  g.eta, last, ~0ull, stack, 64, [&](int i) { return xs[i]; });
+    const uint64_t m = row_program<UNI, uint64_t>(code, n, f64, LineAxis<true>(0), xs[0], g.ys[y], g.zs[z], 64 * rs.h, rs.mag,
+                                                  rs.inv_h, rs.eta, last, ~0ull, stack, 64, [&](int i) { return xs[i]; });
     return m & (~0ull >> (63 - last));
 }
 
@@ -107,7 +113,148 @@ __global__ __launch_bounds__(256) void k_rows_all(const Seg *__restrict__ segs, 
     }
 }
 
+// The program as a mask over the dyadic points of the bracket [lo, hi] on
+// axis k of the line through p: bit i is the point that halving the bracket
+// reaches at i / 2^levels.
+template <bool UNI, class CodeP, class F64P>
+__device__ __forceinline__ uint64_t bracket_bits(CodeP code, uint32_t n, F64P f64, const Grid &g,
+                                                 const LineAxis<false> &ax, double lo, double hi, double x, double y,
+                                                 double z, int levels, uint64_t *stack) {
+    const int k = ax.k;
+    const double scale = (double)(1 << levels) * recip(hi - lo);
+    // (the points' rounding, in steps between them)
+    const double mag = row_scale(g).mag, eta = 1e-6 + 1e-15 * mag * scale;
+    const int last = (1 << levels) - 1;
+    return row_program<UNI, uint64_t>(code, n, f64, ax, k == 0 ? lo : x, k == 1 ? lo : y, k == 2 ? lo : z, hi - lo, mag,
+                                      scale, eta, last, ~1ull, stack, 256, [&](int i) {
+                                          double a = lo, b = hi, m = lo;
+                                          for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
+                                              m = (a + b) / 2;
+                                              if (at + bit == i) break;
+                                              if (i > at + bit) a = m, at += bit;
+                                              else b = m;
+                                          }
+                                          return m;
+                                      });
+}
+
+// mcSearchPoint (mc.go:223-258) of one vertex: up to six halvings are
+// decided at a time by the program's mask over the points they can reach,
+// the last one or two by evaluating it (a second mask costs more than two
+// evaluations, the last of three or more would not: 8 halvings as 6 + 2
+// took 31.6 -> 28.4 us, 573 -> 531 us against two masks).
+//
+// Evaluating every halving is a chain of `iters` dependent program walks,
+// bound by the latency of its loads where few waves run (a small part) and by
+// the walks' scalar and vector issue where many do; one walk decides six
+// halvings here.  Bound by vector issue now (57% of the cycles at 4 waves per
+// SIMD; 115 registers).  Measured (kernel trace, MI355X, 8 halvings): 1,100
+// vertices 23 -> 12 us, 411k vertices of 64 primitives 43 -> 28 us (with the
+// float32 guard 64 -> 31 us), a batch of 32 solids 173 -> 103 us, 10.1M
+// vertices of 512 primitives 819 -> 531 us.
+__device__ __forceinline__ void bisect_rows(const Seg &sg, const uint64_t *__restrict__ bits_all, const uint64_t key,
+                                            double *__restrict__ verts, double *__restrict__ interior, uint64_t v,
+                                            uint64_t *stack) {
+    const DevProg &P = sg.P;
+    const Grid &g = sg.g;
+    const Bricks &B = sg.B;
+    const uint64_t *bits = bits_all + sg.word0;
+    const int k = (int)(key & 3);
+    const int x = (int)((key >> 2) & 0xfffff), y = (int)((key >> 22) & 0xfffff), z = (int)((key >> 42) & 0xfffff);
+    const double px = g.xs[x], py = g.ys[y], pz = g.zs[z];
+    double lo = sel3(k, px, py, pz), hi = *(k == 0 ? g.xs + x + 1 : (k == 1 ? g.ys + y + 1 : g.zs + z + 1));
+    // the high corner decides which end is inside
+    const bool up = corner_bit(g, bits, x + (k == 0), y + (k == 1), z + (k == 2));
+    if (sg.iters > 0) {
+        // the edge's brick program (a crossed edge lies in a brick that is
+        // evaluated: the boxes of constant bricks hold their +1 corners)
+        uint2 bi = make_uint2(BRICK_FULL, P.ncode);
+        if (B.info) bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
+        const uint2 b0 = make_uint2((uint32_t)__builtin_amdgcn_readfirstlane((int)bi.x),
+                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bi.y));
+        const bool uni = __ballot(bi.x != b0.x || bi.y != b0.y) == 0;  // one program for the wave: scalar loads
+        const Insn *code = brick_code(P, B, bi), *code0 = brick_code(P, B, b0);
+        const LineAxis<false> ax(k);
+        int left = sg.iters;
+        while (left > 2) {
+            const int levels = min(left, 6);
+            const uint64_t m = uni ? bracket_bits<true>(scalar_ptr(code0), b0.y, scalar_ptr(P.f64), g, ax, lo, hi, px, py,
+                                                        pz, levels, stack)
+                                   : bracket_bits<false>(code, bi.y, P.f64, g, ax, lo, hi, px, py, pz, levels, stack);
+            for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
+                const double mid = (lo + hi) / 2;
+                const bool in = (m >> (at + bit)) & 1;
+                if (in == up) hi = mid;  // the inside end moves
+                else lo = mid, at += bit;
+            }
+            left -= levels;
+        }
+        for (; left > 0; left--) {
+            const double mid = (lo + hi) / 2;
+            const double qx = k == 0 ? mid : px, qy = k == 1 ? mid : py, qz = k == 2 ? mid : pz;
+            GStats gs;
+            const bool in = uni ? eval_code<0, false, true>(code0, b0.y, P, qx, qy, qz, gs)
+                                : eval_code<0, false, false>(code, bi.y, P, qx, qy, qz, gs);
+            if (in == up) hi = mid;
+            else lo = mid;
+        }
+    }
+    const double res = (lo + hi) / 2;
+    verts[3 * v] = k == 0 ? res : px;
+    verts[3 * v + 1] = k == 1 ? res : py;
+    verts[3 * v + 2] = k == 2 ? res : pz;
+    if (interior) {
+        const double in = up ? hi : lo;  // the bracket's inside end (mc.go:252-255)
+        interior[3 * v] = k == 0 ? in : px;
+        interior[3 * v + 1] = k == 1 ? in : py;
+        interior[3 * v + 2] = k == 2 ? in : pz;
+    }
+}
+
+template <bool MULTI>
+__global__ __launch_bounds__(256) void k_bisect_rows(const Seg *__restrict__ segs, const Seg seg0,
+                                                     const uint32_t *__restrict__ vseg,
+                                                     const uint64_t *__restrict__ bits_all,
+                                                     const uint64_t *__restrict__ vkeys, double *__restrict__ verts,
+                                                     double *__restrict__ interior, const Ctl *__restrict__ ctl,
+                                                     uint64_t vcap) {
+    extern __shared__ __align__(16) uint64_t row_stack[];
+    uint64_t *stack = row_stack + threadIdx.x;
+    // the first vertex's key (and solid) loaded beside the vertex count: the
+    // arrays hold vcap entries, so the loads stay in bounds
+    const uint64_t v0 = (uint64_t)blockIdx.x * 256 + threadIdx.x;
+    const uint64_t key0 = v0 < vcap ? vkeys[v0] : 0;
+    const uint32_t mine0 = MULTI && v0 < vcap ? vseg[v0] : 0u;
+    const uint64_t nv = min((uint64_t)ctl->totals[0], vcap);
+    for (uint64_t v = v0; v < nv; v += (uint64_t)gridDim.x * 256) {
+        const uint64_t key = v == v0 ? key0 : vkeys[v];
+        // lanes may belong to different solids: one solid at a time (every
+        // lane stays in the loop, so the solid is one for the wave in it)
+        const uint32_t mine = MULTI ? (v == v0 ? mine0 : vseg[v]) : 0u;
+        for (uint64_t todo = __ballot(true); todo;) {
+            const uint32_t si =
+                MULTI ? (uint32_t)__builtin_amdgcn_readlane((int)mine, __ffsll((unsigned long long)todo) - 1) : 0u;
+            const bool here = !MULTI || mine == si;
+            if (here) bisect_rows(pick_seg<MULTI>(segs, seg0, si), bits_all, key, verts, interior, v, stack);
+            todo &= ~__ballot(here);
+        }
+    }
+}
+
 }  // namespace
+
+hipError_t launch_bisect_rows(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
+                              hipStream_t st) {
+    const int depth = p.stack > 1 ? p.stack - 1 : 1;
+    const size_t lds = (size_t)depth * 256 * sizeof(uint64_t);
+    const unsigned grid = grid_for(vcap, 256, 1u << 14);
+    if (p.nsegs > 1)
+        k_bisect_rows<true><<<grid, 256, lds, st>>>(p.segs, p.seg0, b.vseg, b.bits, b.vkeys, verts, interior, p.ctl, vcap);
+    else
+        k_bisect_rows<false><<<grid, 256, lds, st>>>(p.segs, p.seg0, nullptr, b.bits, b.vkeys, verts, interior, p.ctl,
+                                                     vcap);
+    return hipGetLastError();
+}
 
 hipError_t launch_rows(const Pipe &p, const Bufs &b, hipStream_t st) {
     const int depth = p.stack > 1 ? p.stack - 1 : 1;  // masks below the top

@@ -78,6 +78,8 @@ hipError_t launch_classify(const Pipe &p, const Bufs &b, hipStream_t st);
 // several solids) each solid's output ranges
 hipError_t launch_scan(const Pipe &p, const Bufs &b, hipStream_t st);
 hipError_t launch_emit(const Pipe &p, const Bufs &b, uint32_t *tris, uint64_t vcap, uint64_t tcap, hipStream_t st);
+hipError_t launch_bisect_rows(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
+                              hipStream_t st);
 hipError_t launch_bisect(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
                          hipStream_t st);
 hipError_t launch_bisect_host(int mode, const DevProg &P, const Grid &g, const uint64_t *bits,

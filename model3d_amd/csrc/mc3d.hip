@@ -487,6 +487,7 @@ struct Job {
     std::shared_ptr<const Lowered> low;  // the solid's (shared with its handle)
     std::vector<double> ax[3];
     Grid g{};    // sizes; axis pointers set by the upload
+    RowScale scale{};
     Bricks B{};  // shape; array pointers set by the upload
     uint64_t nwords = 0, nbricks = 0, word0 = 0, brick0 = 0;
     uint64_t pos0 = 0, npos = 0;  // scan positions (npos 0: the scan takes the words, pos0 = word0)
@@ -556,11 +557,11 @@ int layout_job(Job &j, const mc3d_options &o, bool check) {
     g.nx = (int)j.ax[0].size(), g.ny = (int)j.ax[1].size(), g.nz = (int)j.ax[2].size();
     g.W = (g.nx + 63) / 64;
     j.nwords = (uint64_t)g.W * g.ny * g.nz;
-    g.inv_h = 1 / j.delta;
-    g.mag = 0;
-    for (int a = 0; a < 3; a++) g.mag = std::max({g.mag, fabs(j.ax[a].front()), fabs(j.ax[a].back())});
+    RowScale &rs = j.scale;
+    rs = RowScale{j.delta, 1 / j.delta, 0, 0};
+    for (int a = 0; a < 3; a++) rs.mag = std::max({rs.mag, fabs(j.ax[a].front()), fabs(j.ax[a].back())});
     // 64 additions of delta, each rounded to half an ulp of the coordinate
-    g.eta = 1e-6 + 1e-11 * g.mag * g.inv_h;
+    rs.eta = 1e-6 + 1e-11 * rs.mag * rs.inv_h;
     if (check && j.nwords >= (1ull << 32)) {
         set_error("grid too large: more than 2^32 occupancy words");
         return MC3D_E_UNSUPPORTED;
@@ -808,7 +809,7 @@ void layout_upload(const std::vector<Job> &jobs, uint64_t nwords_all, uint64_t n
         po.fr = place(P.frames.size() * sizeof(Frame));
         po.nodes = place(nodes.size() * sizeof(PlanNode));
         po.col = place(P.colliders.size() * sizeof(DevCollider));
-        po.ax = place((jobs[s].ax[0].size() + jobs[s].ax[1].size() + jobs[s].ax[2].size()) * sizeof(double));
+        po.ax = place((jobs[s].ax[0].size() + jobs[s].ax[1].size() + jobs[s].ax[2].size()) * sizeof(double) + sizeof(RowScale));
     }
     U.total = off;
 }
@@ -850,6 +851,7 @@ void fill_upload(std::vector<Job> &jobs, uint64_t nwords_all, uint64_t nbricks_a
         if (!U.cols[s].empty()) memcpy(h + po.col, U.cols[s].data(), U.cols[s].size() * sizeof(DevCollider));
         double *d = (double *)(h + po.ax);
         for (int a = 0; a < 3; a++) d = std::copy(j.ax[a].begin(), j.ax[a].end(), d);
+        memcpy(d, &j.scale, sizeof(RowScale));
         Seg &sg = U.hsegs[s];
         sg.P.code = (const Insn *)(dv + po.code);
         sg.P.f64 = (const double *)(dv + po.f64);
@@ -1060,7 +1062,7 @@ int plan_call(std::vector<Job> &jobs, const mc3d_options &o, Call &c) {
     // statistics runs count the evaluations of single points.
     c.rows = !c.stats && !c.host;
     for (const Job &j : jobs) {
-        c.rows = c.rows && j.low->rows && j.g.eta < 0.01 && std::isfinite(j.g.inv_h);
+        c.rows = c.rows && j.low->rows && j.scale.eta < 0.01 && std::isfinite(j.scale.inv_h);
         c.stack = std::max(c.stack, j.low->P.max_stack);
     }
     c.plan_lds = PLAN_STACK_BYTES;
@@ -2822,8 +2824,9 @@ int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_
             for (int q = 0; q < 3; q++) mag = std::max(mag, fabs(p[q]));
             mag = std::max(mag, fabs(pts[last]));
             uint64_t sure, maybe;
-            row_mask(atom_span(kind, a, k, p[0], p[1], p[2], smax, mag), scale, 1e-6 + 1e-11 * mag / h, last, sure,
-                     maybe);
+            const Span sp = k == 0 && (next() & 1) ? atom_span(kind, a, LineAxis<true>(0), p[0], p[1], p[2], smax, mag)
+                                                   : atom_span(kind, a, LineAxis<false>(k), p[0], p[1], p[2], smax, mag);
+            row_mask(sp, scale, 1e-6 + 1e-11 * mag / h, last, sure, maybe);
             for (int i = 0; i <= last; i++) {
                 p[k] = pts[i];
                 const bool in = atom64(kind, a, p[0], p[1], p[2]), yes = sure >> i & 1, may = maybe >> i & 1;

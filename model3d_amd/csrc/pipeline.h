@@ -51,9 +51,14 @@ struct Grid {
     // a z slab of a larger grid: its first / last plane is shared with the
     // slab below / above, not a face of the grid
     int zlo_open, zhi_open;
-    // for the row kernels (rows.h): 1 / spacing, the largest |coordinate|, and
-    // a bound, in spacings, of how far 64 corners stray from even spacing
-    double inv_h, mag, eta;
+};
+
+// For the row kernels (rows.h): the spacing and its inverse, the largest
+// |coordinate|, and a bound, in spacings, of how far 64 corners stray from
+// even spacing.  They follow the z axis in memory (a solid moved by the same
+// grid keeps its kernel arguments, and so its captured launches).
+struct RowScale {
+    double h, inv_h, mag, eta;
 };
 
 // Plane z is a face of the whole grid (where panic("solid is true outside

@@ -36,6 +36,17 @@ MC3D_HD inline double rsq_estimate(double w) {
 #endif
 }
 
+// 1 / x to the last digit or two (the bounds it goes into carry far more).
+MC3D_HD inline double recip(double x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y = __builtin_amdgcn_rcp(x);
+    y = __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+    return __builtin_fma(y, __builtin_fma(-x, y, 1.0), y);
+#else
+    return 1 / x;
+#endif
+}
+
 // ro >= sqrt(w') >= ri for every w' in [w - D, w + D] (w >= -D), with e0
 // more on each side; ri < 0: w' may be below zero.
 MC3D_HD inline void span_root(double w, double D, double e0, double &ro, double &ri) {
@@ -56,12 +67,31 @@ MC3D_HD inline void span_root(double w, double D, double e0, double &ro, double 
 // product of two leaves the float64 range.
 MC3D_HD inline bool span_range(double M) { return M > 1e-100 && M < 1e100; }
 
-// Sphere about c with threshold T (s <= T), M bounding every coordinate and
-// length: the line's squared distance is q, and s - T = x^2 + q - T.
-// Rounding moves s by far less than 1e-13 M^2.
-MC3D_HD inline Span sphere_span(double ck, double c1, double c2, double T, double pk, double p1, double p2, double M) {
-    const double d1 = p1 - c1, d2 = p2 - c2, D = 1e-13 * M * M;
-    const double w = T - (d1 * d1 + d2 * d2), m = ck - pk;
+// The axis of a line: known when the code is compiled (KX: the x axis), or
+// a lane's own, then as the unit vector e_k and 1 - e_k, so that picking a
+// component is three multiply-adds instead of selects of scalar operands.
+template <bool KX>
+struct LineAxis {
+    int k = 0;
+    double v[3] = {1, 0, 0}, u[3] = {0, 1, 1};
+    MC3D_HD explicit LineAxis(int axis) : k(axis) {
+        for (int a = 0; a < 3; a++) v[a] = a == axis ? 1.0 : 0.0, u[a] = a == axis ? 0.0 : 1.0;
+    }
+    MC3D_HD double along(double x, double y, double z) const {
+        if (KX) return x;
+        return __builtin_fma(z, v[2], __builtin_fma(y, v[1], x * v[0]));
+    }
+    MC3D_HD double across2(double x, double y, double z) const {  // the other components' squares
+        if (KX) return __builtin_fma(z, z, y * y);
+        return __builtin_fma(z * z, u[2], __builtin_fma(y * y, u[1], x * x * u[0]));
+    }
+};
+
+// Sphere with threshold T (s <= T) whose centre is p - d, M bounding every
+// coordinate and length.  Rounding moves s by far less than 1e-13 M^2.
+template <bool KX>
+MC3D_HD inline Span sphere_span(const LineAxis<KX> &ax, double dx, double dy, double dz, double T, double M) {
+    const double D = 1e-13 * M * M, w = T - ax.across2(dx, dy, dz), m = -ax.along(dx, dy, dz);
     if (w < -D) return span_none();
     double ro, ri;
     span_root(w, D, 1e-14 * M, ro, ri);
@@ -70,28 +100,29 @@ MC3D_HD inline Span sphere_span(double ck, double c1, double c2, double T, doubl
     return s;
 }
 
-// Cylinder from q along the unit vector d, length L, threshold T: with
-// v = p - q, c = v.d and n = v - c d, the squared distance from its axis is
-// |n|^2 + 2 s n_k + s^2 (1 - d_k^2), the position along it c + s d_k.  smax:
-// the largest |s| asked about (nearly parallel lines, where the roots or the
-// end planes are ill-defined, are bounded over that range instead).
-MC3D_HD inline Span cylinder_span(double qk, double q1, double q2, double dk, double d1, double d2, double L, double T,
-                                  double pk, double p1, double p2, double smax, double M) {
-    const double vk = pk - qk, v1 = p1 - q1, v2 = p2 - q2;
-    const double c = vk * dk + v1 * d1 + v2 * d2;
-    const double nk = vk - dk * c, n1 = v1 - d1 * c, n2 = v2 - d2 * c;
-    const double w = T - (nk * nk + n1 * n1 + n2 * n2), A = d1 * d1 + d2 * d2, D = 1e-13 * M * M;
+// Cylinder from p - v along the unit vector d, length L, threshold T: with
+// c = v.d and n = v - c d, the squared distance from its axis is |n|^2 +
+// 2 s n_k + s^2 (1 - d_k^2), the position along it c + s d_k.  smax: the
+// largest |s| asked about (nearly parallel lines, where the roots or the end
+// planes are ill-defined, are bounded over that range instead).
+template <bool KX>
+MC3D_HD inline Span cylinder_span(const LineAxis<KX> &ax, double vx, double vy, double vz, double dx, double dy, double dz,
+                                  double L, double T, double smax, double M) {
+    const double c = __builtin_fma(vz, dz, __builtin_fma(vy, dy, vx * dx));
+    const double nx = __builtin_fma(-dx, c, vx), ny = __builtin_fma(-dy, c, vy), nz = __builtin_fma(-dz, c, vz);
+    const double nk = ax.along(nx, ny, nz), dk = ax.along(dx, dy, dz), A = ax.across2(dx, dy, dz);
+    const double w = T - __builtin_fma(nz, nz, __builtin_fma(ny, ny, nx * nx)), D = 1e-13 * M * M;
     Span s;
     if (A < 1e-6) {  // along the axis: the distance hardly changes
         const double D2 = D + 2 * fabs(nk) * smax + A * smax * smax;
         if (w < -D2) return span_none();
         s = w > D2 ? span_all() : span_unsure();
     } else {
-        const double disc = nk * nk + A * w, DD = A * D + 1e-14 * nk * nk;
+        const double disc = __builtin_fma(A, w, nk * nk), DD = A * D + 1e-14 * nk * nk;
         if (disc < -DD) return span_none();
         double ro, ri;
         span_root(disc, DD, 0, ro, ri);
-        const double iA = 1 / A, e = (1e-12 * (fabs(nk) + ro) + 1e-14 * M) * iA;
+        const double iA = recip(A), e = (1e-12 * (fabs(nk) + ro) + 1e-14 * M) * iA;
         s = Span{(-nk - ro) * iA - e, (-nk + ro) * iA + e, INFINITY, -INFINITY};
         if (ri > 0) s.ai = (-nk - ri) * iA + e, s.bi = (-nk + ri) * iA - e;
     }
@@ -101,7 +132,7 @@ MC3D_HD inline Span cylinder_span(double qk, double q1, double q2, double dk, do
         if (c < -f2 || c > L + f2) return span_none();
         if (!(c > f2 && c < L - f2)) s.ai = INFINITY, s.bi = -INFINITY;
     } else {
-        const double i = 1 / dk;
+        const double i = recip(dk);
         const double t0 = (-f - c) * i, t1 = (L + f - c) * i, u0 = (f - c) * i, u1 = (L - f - c) * i;
         s.ao = fmax(s.ao, fmin(t0, t1)), s.bo = fmin(s.bo, fmax(t0, t1));
         s.ai = fmax(s.ai, dk > 0 ? u0 : u1), s.bi = fmin(s.bi, dk > 0 ? u1 : u0);
@@ -110,40 +141,42 @@ MC3D_HD inline Span cylinder_span(double qk, double q1, double q2, double dk, do
 }
 
 // Where an untransformed sphere, box, capsule or cylinder (params a, the
-// layouts of AtomKind) is true on the line through (x, y, z) along axis k.
+// layouts of AtomKind) is true on the line through (x, y, z) along the axis.
 // mag: a bound of |x|, |y|, |z| and of the coordinates asked about.
-template <class F64P>
-MC3D_HD inline Span atom_span(uint32_t kind, F64P a, int k, double x, double y, double z, double smax, double mag) {
-    const double pk = sel3(k, x, y, z), p1 = sel3(k, y, x, x), p2 = sel3(k, z, z, y);
-    auto along = [&](int o) { return sel3(k, a[o], a[o + 1], a[o + 2]); };
-    auto first = [&](int o) { return sel3(k, a[o + 1], a[o], a[o]); };
-    auto second = [&](int o) { return sel3(k, a[o + 2], a[o + 2], a[o + 1]); };
+template <bool KX, class F64P>
+MC3D_HD inline Span atom_span(uint32_t kind, F64P a, const LineAxis<KX> &ax, double x, double y, double z, double smax,
+                              double mag) {
     auto size = [&](int o) { return fabs(a[o]) + fabs(a[o + 1]) + fabs(a[o + 2]); };
     if (kind == A_RECT) {  // exact comparisons off the line's axis
-        if (!(in_lo(p1, first(0)) && in_hi(p1, first(3)) && in_lo(p2, second(0)) && in_hi(p2, second(3))))
-            return span_none();
-        const double lo = along(0) - pk, hi = along(3) - pk;
-        return Span{lo, hi, lo, hi};
+        const int k = KX ? 0 : ax.k;
+        const bool in = (int)(k == 0 || ((int)in_lo(x, a[0]) & (int)in_hi(x, a[3]))) &
+                        (int)(k == 1 || ((int)in_lo(y, a[1]) & (int)in_hi(y, a[4]))) &
+                        (int)(k == 2 || ((int)in_lo(z, a[2]) & (int)in_hi(z, a[5])));
+        if (!in) return span_none();
+        const double p = sel3(k, x, y, z), a0 = sel3(k, a[0], a[1], a[2]), a1 = sel3(k, a[3], a[4], a[5]);
+        const double lo = a0 - p, hi = a1 - p;
+        // (rounding of the differences; an infinite face has none)
+        const double el = fabs(lo) < INFINITY ? 1e-15 * (mag + fabs(a0)) : 0;
+        const double eh = fabs(hi) < INFINITY ? 1e-15 * (mag + fabs(a1)) : 0;
+        return Span{lo - el, hi + eh, lo + el, hi - eh};
     }
     if (kind == A_SPHERE) {
         const double M = 3 * mag + size(0) + a[3];
         if (!span_range(M)) return span_unsure();
-        return sphere_span(along(0), first(0), second(0), a[4], pk, p1, p2, M);
+        return sphere_span(ax, x - a[0], y - a[1], z - a[2], a[4], M);
     }
     if (kind == A_CYLINDER) {
         const double M = 3 * mag + size(0) + a[6] + a[7];
         if (!(span_range(M) && size(3) < 2)) return span_unsure();
-        return cylinder_span(along(0), first(0), second(0), along(3), first(3), second(3), a[6], a[8], pk, p1, p2,
-                             smax, M);
+        return cylinder_span(ax, x - a[0], y - a[1], z - a[2], a[3], a[4], a[5], a[6], a[8], smax, M);
     }
     // capsule: the cylinder between two spheres; it is convex, so the hull
     // of their intervals (and of the certain parts of those) is its own
     const double M = 3 * mag + size(0) + size(3) + a[9] + a[10];
     if (!(span_range(M) && size(6) < 2)) return span_unsure();
-    const Span u = sphere_span(along(0), first(0), second(0), a[11], pk, p1, p2, M);
-    const Span v = sphere_span(along(3), first(3), second(3), a[11], pk, p1, p2, M);
-    Span s = cylinder_span(along(0), first(0), second(0), along(6), first(6), second(6), a[9], a[11], pk, p1, p2, smax,
-                           M);
+    const Span u = sphere_span(ax, x - a[0], y - a[1], z - a[2], a[11], M);
+    const Span v = sphere_span(ax, x - a[3], y - a[4], z - a[5], a[11], M);
+    Span s = cylinder_span(ax, x - a[0], y - a[1], z - a[2], a[6], a[7], a[8], a[9], a[11], smax, M);
     if (!(s.ao <= s.bo)) s = span_none();
     if (!(s.ai <= s.bi)) s.ai = INFINITY, s.bi = -INFINITY;
     s.ao = fmin(s.ao, fmin(u.ao, v.ao)), s.bo = fmax(s.bo, fmax(u.bo, v.bo));
@@ -171,14 +204,15 @@ MC3D_HD inline void row_mask(const Span &s, double scale, double eta, int last, 
 // The atom's mask over the points: sure ones, and those of the rest at
 // which atom64 is true (point(i): the i-th point's coordinate along axis k).
 // Only the points of `want` matter.
-template <class F64P, class Point>
-__device__ __forceinline__ uint64_t atom_mask(uint32_t kind, F64P a, int k, double x, double y, double z, double smax,
+template <bool KX, class F64P, class Point>
+__device__ __forceinline__ uint64_t atom_mask(uint32_t kind, F64P a, const LineAxis<KX> &ax, double x, double y, double z, double smax,
                                               double mag, double scale, double eta, int last, uint64_t want,
                                               Point &&point) {
     uint64_t sure, maybe;
-    row_mask(atom_span(kind, a, k, x, y, z, smax, mag), scale, eta, last, sure, maybe);
+    row_mask(atom_span(kind, a, ax, x, y, z, smax, mag), scale, eta, last, sure, maybe);
     for (uint64_t open = maybe & ~sure & want; open; open &= open - 1) {
         const int i = __ffsll((unsigned long long)open) - 1;
+        const int k = KX ? 0 : ax.k;
         const double p = point(i);
         if (atom64(kind, a, k == 0 ? p : x, k == 1 ? p : y, k == 2 ? p : z)) sure |= 1ull << i;
     }
@@ -196,8 +230,8 @@ __device__ __forceinline__ M mask_op(uint32_t op, M a, M b) {
 
 // A program over such atoms as a mask over the points of a line; the stack
 // below its top lies in LDS (slot i of this lane: stack[i * stride]).
-template <bool UNI, class M, class CodeP, class F64P, class Point>
-__device__ __forceinline__ M row_program(CodeP code, uint32_t n, F64P f64, int k, double x, double y, double z,
+template <bool UNI, class M, bool KX, class CodeP, class F64P, class Point>
+__device__ __forceinline__ M row_program(CodeP code, uint32_t n, F64P f64, const LineAxis<KX> &ax, double x, double y, double z,
                                          double smax, double mag, double scale, double eta, int last, M want,
                                          M *stack, int stride, Point &&point) {
     M top = 0;
@@ -210,7 +244,7 @@ __device__ __forceinline__ M row_program(CodeP code, uint32_t n, F64P f64, int k
         if (op == OP_ATOM || op == OP_TRUE || op == OP_FALSE) {
             if (sp > 0) stack[(sp - 1) * stride] = top;
             sp++;
-            top = op == OP_ATOM ? (M)atom_mask(insn_kind(in.x), f64 + in.y, k, x, y, z, smax, mag, scale, eta, last,
+            top = op == OP_ATOM ? (M)atom_mask(insn_kind(in.x), f64 + in.y, ax, x, y, z, smax, mag, scale, eta, last,
                                                (uint64_t)want, point)
                                 : (op == OP_TRUE ? ~(M)0 : (M)0);
         } else if (op == OP_NOT) {
