@@ -11,25 +11,33 @@
 // a rect's answer is the OR over the triangles of the cells it overlaps of
 // "the triangle's box overlaps the rect and Triangle.RectCollision" -- the
 // answer the collider's tree gives, whose every node box contains the boxes
-// of the triangles below it.  The recursion runs level by level: one wave
-// per block asks the filter; an accepted block whose volume / 2 is below 64
-// sets its cubes in the cube mask, a larger one pushes its two halves to the
-// next level.  The reference's two-stage recursion (first down to
-// max(volume / 4096, 64), then each queued block down to 64) asks the same
-// deterministic filter of the same blocks, so its accepted leaves are these.
+// of the triangles below it.
+//
+// A leaf of the recursion (volume / 2 below 64) is accepted when it and
+// every block above it are.  The splits do not depend on the filter, so a
+// leaf is a path of halvings from the root, and all leaves are asked at once,
+// a lane each: most are decided by summed-volume tables (no triangle listed
+// in the rect's cells: rejected; a segment origin in a cell inside it:
+// accepted, and with it every block above, whose rects contain the leaf's).
+// The few left open are asked with Triangle.RectCollision, a wave each, and
+// where the leaf is hit without an origin in it the blocks above it too.  The
+// reference's two-stage recursion (first down to max(volume / 4096, 64), then
+// each queued block down to 64) asks the same deterministic filter of the
+// same blocks, so its accepted leaves are these.
+//
+// Level by level (a kernel per level, each waiting for the one above, four
+// blocks a wave so that open ones did not wait for each other) a grid of
+// 402^3 corners with 51k triangles took 1,660 us; here the leaves take 117
+// us (the mask's atomics) and the open ones 390 us, bound by the chain of
+// loads to each batch of 64 listed triangles (list, box, triangle).  Cells of
+// one coarse spacing instead of two list fewer triangles per rect (open 610
+// -> 460 us); the boxes kept from the binning reject most of a batch with six
+// comparisons (460 -> 372 us).
 #include "launch.h"
 #include "rect_collide.h"
 
-// Blocks per wave in the recursion's level kernel.
-#ifndef MC3D_FILTER_GROUP
-#define MC3D_FILTER_GROUP 4
-#endif
-
 namespace mc3d {
 namespace {
-
-constexpr int FGROUP = MC3D_FILTER_GROUP;
-static_assert(FGROUP >= 1 && FGROUP <= 64, "blocks per wave: 1 to 64");
 
 __device__ __forceinline__ void cell_range(double lo, double hi, double o, double inv, int n, int &c0, int &c1) {
     // clamped to the grid (a NaN bound: cell 0; such a rect overlaps no box)
@@ -40,12 +48,10 @@ __device__ __forceinline__ void cell_range(double lo, double hi, double o, doubl
 
 // The cells of a triangle's box; false for a box with NaN bounds (such a
 // triangle's box overlaps no rect).
-__device__ __forceinline__ bool tri_cells(const RectGridDev &R, const double *p, int *c0, int *c1) {
-    double tmn[3], tmx[3];
-    rc::tri_box(p, tmn, tmx);
+__device__ __forceinline__ bool tri_cells(const RectGridDev &R, const GroupBox &b, int *c0, int *c1) {
     for (int a = 0; a < 3; a++) {
-        if (isnan(tmn[a]) || isnan(tmx[a])) return false;
-        cell_range(tmn[a], tmx[a], R.o[a], R.inv, R.n[a], c0[a], c1[a]);
+        if (isnan(b.mn[a]) || isnan(b.mx[a])) return false;
+        cell_range(b.mn[a], b.mx[a], R.o[a], R.inv, R.n[a], c0[a], c1[a]);
     }
     return true;
 }
@@ -60,10 +66,14 @@ __global__ __launch_bounds__(256) void k_rgrid_gather(const double *__restrict__
     }
 }
 
-__global__ __launch_bounds__(256) void k_rgrid_count(RectGridDev R, uint32_t *__restrict__ counts) {
+__global__ __launch_bounds__(256) void k_rgrid_count(RectGridDev R, GroupBox *__restrict__ box,
+                                                     uint32_t *__restrict__ counts) {
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < R.ntris; t += gridDim.x * blockDim.x) {
         int c0[3], c1[3];
-        if (!tri_cells(R, R.tris + 9 * (size_t)t, c0, c1)) continue;
+        GroupBox b;
+        rc::tri_box(R.tris + 9 * (size_t)t, b.mn, b.mx);
+        box[t] = b;
+        if (!tri_cells(R, b, c0, c1)) continue;
         for (int z = c0[2]; z <= c1[2]; z++)
             for (int y = c0[1]; y <= c1[1]; y++)
                 for (int x = c0[0]; x <= c1[0]; x++) atomicAdd(&counts[((size_t)z * R.n[1] + y) * R.n[0] + x], 1u);
@@ -74,7 +84,7 @@ __global__ __launch_bounds__(256) void k_rgrid_fill(RectGridDev R, uint32_t *__r
                                                     uint32_t *__restrict__ cell_tris) {
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < R.ntris; t += gridDim.x * blockDim.x) {
         int c0[3], c1[3];
-        if (!tri_cells(R, R.tris + 9 * (size_t)t, c0, c1)) continue;
+        if (!tri_cells(R, R.box[t], c0, c1)) continue;
         for (int z = c0[2]; z <= c1[2]; z++)
             for (int y = c0[1]; y <= c1[1]; y++)
                 for (int x = c0[0]; x <= c1[0]; x++)
@@ -123,7 +133,7 @@ __global__ __launch_bounds__(256) void k_vsat_x(uint32_t *__restrict__ v, int n0
     }
 }
 
-__global__ __launch_bounds__(256) void k_vsat_yz(uint32_t *__restrict__ v, int n0, int n1, int n2, int axis) {
+__global__ __launch_bounds__(64) void k_vsat_yz(uint32_t *__restrict__ v, int n0, int n1, int n2, int axis) {
     // axis 1: columns (x, z) along y; axis 2: columns (x, y) along z
     const uint32_t ncol = (uint32_t)n0 * (axis == 1 ? n2 : n1);
     for (uint32_t c = blockIdx.x * blockDim.x + threadIdx.x; c < ncol; c += gridDim.x * blockDim.x) {
@@ -132,8 +142,17 @@ __global__ __launch_bounds__(256) void k_vsat_yz(uint32_t *__restrict__ v, int n
         int len;
         if (axis == 1) i = (size_t)w * n1 * n0 + x, step = n0, len = n1;
         else i = (size_t)w * n0 + x, step = (size_t)n0 * n1, len = n2;
+        // eight loads in flight (a column is a chain of dependent additions,
+        // and few columns run at once: one load at a time took 31 us for
+        // 100^3 cells)
         uint32_t s = 0;
-        for (int k = 0; k < len; k++, i += step) v[i] = s += v[i];
+        int k = 0;
+        for (; k + 8 <= len; k += 8, i += 8 * step) {
+            uint32_t t[8];
+            for (int j = 0; j < 8; j++) t[j] = v[i + j * step];
+            for (int j = 0; j < 8; j++) v[i + j * step] = s += t[j];
+        }
+        for (; k < len; k++, i += step) v[i] = s += v[i];
     }
 }
 
@@ -189,15 +208,20 @@ __global__ __launch_bounds__(RSCAN) void k_rscan_down(const uint32_t *__restrict
     if (i == n - 1) start[n] = s;
 }
 
-__global__ void k_filter_root(FBlock root, FBlock *__restrict__ front, uint32_t *__restrict__ level_counts,
-                              uint32_t nlevels) {
-    for (uint32_t i = threadIdx.x; i <= nlevels; i += blockDim.x) level_counts[i] = i == 0 ? 1u : 0u;
-    if (threadIdx.x == 0) front[0] = root;
-}
-
 // Candidate k of n in a scattered order (P prime and above n: a bijection),
 // so that the first 64 lanes sample the whole rect, not its first rows.
 __device__ __forceinline__ uint32_t scatter(uint32_t k, uint32_t n, uint64_t P) { return (uint32_t)(k * P % n); }
+
+// Sum of the cells [lo, hi] from a summed-volume table of n[0] x n[1] x n[2].
+__device__ __forceinline__ uint32_t table_sum(const uint32_t *__restrict__ t, const int *n, const int *lo, const int *hi) {
+    auto S = [&](int x, int y, int z) -> uint32_t {
+        if (x < 0 || y < 0 || z < 0) return 0u;
+        return t[((size_t)z * n[1] + y) * n[0] + x];
+    };
+    const int x0 = lo[0] - 1, y0 = lo[1] - 1, z0 = lo[2] - 1, x1 = hi[0], y1 = hi[1], z1 = hi[2];
+    return S(x1, y1, z1) - S(x0, y1, z1) - S(x1, y0, z1) - S(x1, y1, z0) + S(x0, y0, z1) + S(x0, y1, z0) + S(x1, y0, z0) -
+           S(x0, y0, z0);
+}
 
 // A sure hit from the vertex table: a segment origin in a cell strictly
 // inside the rect's cell range.  For such a vertex v in cell k on an axis,
@@ -214,42 +238,59 @@ __device__ __forceinline__ bool sure_hit(const RectGridDev &R, const double *mn,
         lo[a] = c0 + 1, hi[a] = c1 - 1;  // (clamping only narrows the range)
         if (hi[a] < lo[a]) return false;
     }
-    auto S = [&](int x, int y, int z) -> uint32_t {
-        if (x < 0 || y < 0 || z < 0) return 0u;
-        return R.vsat[((size_t)z * R.vn[1] + y) * R.vn[0] + x];
-    };
-    const int x0 = lo[0] - 1, y0 = lo[1] - 1, z0 = lo[2] - 1, x1 = hi[0], y1 = hi[1], z1 = hi[2];
-    const uint32_t n = S(x1, y1, z1) - S(x0, y1, z1) - S(x1, y0, z1) - S(x1, y1, z0) + S(x0, y0, z1) + S(x0, y1, z0) +
-                       S(x1, y0, z0) - S(x0, y0, z0);
-    return n != 0;
+    return table_sum(R.vsat, R.vn, lo, hi) != 0;
+}
+
+// No triangle is listed in the rect's cells: the rect overlaps no triangle's
+// box (cell_range is monotone, so overlapping boxes share a cell).
+__device__ __forceinline__ bool sure_miss(const RectGridDev &R, const double *mn, const double *mx) {
+    int c0[3], c1[3];
+    for (int a = 0; a < 3; a++) {
+        cell_range(mn[a], mx[a], R.o[a], R.inv, R.n[a], c0[a], c1[a]);
+        if (c1[a] < c0[a]) return true;  // min above max: the rect overlaps no box
+    }
+    return table_sum(R.csat, R.n, c0, c1) == 0;
+}
+
+// rc::box_overlap for boxes without NaN (none else is listed; a NaN on
+// either side compares false, which is its answer too).
+__device__ __forceinline__ bool boxes_overlap(const double *mn, const double *mx, const GroupBox &b) {
+    return mn[0] <= b.mx[0] && b.mn[0] <= mx[0] && mn[1] <= b.mx[1] && b.mn[1] <= mx[1] && mn[2] <= b.mx[2] &&
+           b.mn[2] <= mx[2] && mn[0] <= mx[0] && mn[1] <= mx[1] && mn[2] <= mx[2];
 }
 
 // RectCollision of the mesh for [mn, mx] where the vertex table gave no sure
-// hit, asked by a whole wave (the answer is wave-uniform): every candidate
+// hit, asked by a whole wave (the answer is wave-uniform: 0 no, 1 yes, 2 yes
+// by a segment origin inside, which is inside every larger rect too): every
+// candidate
 // triangle tested once -- the triangles binned in the cells the rect
 // overlaps, taken 64 at a time (each (y, z) row of those cells is one run
 // of the cell lists; a triangle listed in several of the rect's cells is
 // tested at the first of them), or, for a rect over more cells than half
 // the triangles, all triangles in a scattered order.
-__device__ bool rect_hits(const RectGridDev &R, const double *mn, const double *mx) {
+__device__ int rect_hits(const RectGridDev &R, const double *mn, const double *mx) {
     const int lane = threadIdx.x & 63;
     int c0[3], c1[3];
     for (int a = 0; a < 3; a++) {
         cell_range(mn[a], mx[a], R.o[a], R.inv, R.n[a], c0[a], c1[a]);
-        if (c1[a] < c0[a]) return false;  // min above max: the rect overlaps no box
+        if (c1[a] < c0[a]) return 0;  // min above max: the rect overlaps no box
     }
     const uint32_t lx = c1[0] - c0[0] + 1, ly = c1[1] - c0[1] + 1, lz = c1[2] - c0[2] + 1;
     const uint64_t ncell = (uint64_t)lx * ly * lz;
     if (2 * ncell > R.ntris) {
         for (uint32_t t0 = 0; t0 < R.ntris; t0 += 64) {
-            bool h = false;
+            int h = 0;
             if (t0 + lane < R.ntris) {
-                const double *p = R.tris + 9 * (size_t)scatter(t0 + lane, R.ntris, 4294967291ull);
-                h = rc::vertex_inside(p, mn, mx) || rc::triangle_hits_rect(p, mn, mx);
+                const uint32_t t = scatter(t0 + lane, R.ntris, 4294967291ull);
+                const double *p = R.tris + 9 * (size_t)t;
+                if (boxes_overlap(mn, mx, R.box[t])) {
+                    const rc::V v[3] = {rc::mk(p[0], p[1], p[2]), rc::mk(p[3], p[4], p[5]), rc::mk(p[6], p[7], p[8])};
+                    h = rc::vertex_inside(p, mn, mx) ? 2 : (rc::tri_rect(v, mn, mx) ? 1 : 0);
+                }
             }
-            if (__ballot(h)) return true;
+            if (__ballot(h != 0)) return __ballot(h == 2) ? 2 : 1;
         }
-        return false;
+        return 0;
     }
     const uint32_t nrows = ly * lz;
     for (uint32_t r0 = 0; r0 < nrows; r0 += 64) {
@@ -280,31 +321,31 @@ __device__ bool rect_hits(const RectGridDev &R, const double *mn, const double *
             }
             const uint32_t aj = __shfl(a, lo, 64), xj = __shfl(excl, lo, 64);
             const int yj = __shfl(ry, lo, 64), zj = __shfl(rz, lo, 64);
-            bool h = false;
+            int h = 0;
             if (e < total) {
                 const uint32_t idx = aj + (e - xj);
-                const double *p = R.tris + 9 * (size_t)R.cell_tris[idx];
-                double tmn[3], tmx[3];
-                rc::tri_box(p, tmn, tmx);
-                if (rc::box_overlap(mn, mx, tmn, tmx)) {
+                const uint32_t tri = R.cell_tris[idx];
+                const double *p = R.tris + 9 * (size_t)tri;
+                const GroupBox tb = R.box[tri];
+                if (boxes_overlap(mn, mx, tb)) {
                     // the first of the rect's cells that list it: row (y, z)
                     // at max(its first cell, the rect's), then the cell's run
                     int t0[3], t1[3];
-                    for (int ax = 0; ax < 3; ax++) cell_range(tmn[ax], tmx[ax], R.o[ax], R.inv, R.n[ax], t0[ax], t1[ax]);
+                    for (int ax = 0; ax < 3; ax++) cell_range(tb.mn[ax], tb.mx[ax], R.o[ax], R.inv, R.n[ax], t0[ax], t1[ax]);
                     if (yj == max(t0[1], c0[1]) && zj == max(t0[2], c0[2])) {
                         const size_t cf = ((size_t)zj * R.n[1] + yj) * R.n[0] + max(t0[0], c0[0]);
                         if (idx >= R.cell_start[cf] && idx < R.cell_start[cf + 1]) {
                             const rc::V t[3] = {rc::mk(p[0], p[1], p[2]), rc::mk(p[3], p[4], p[5]),
                                                 rc::mk(p[6], p[7], p[8])};
-                            h = rc::vertex_inside(p, mn, mx) || rc::tri_rect(t, mn, mx);
+                            h = rc::vertex_inside(p, mn, mx) ? 2 : (rc::tri_rect(t, mn, mx) ? 1 : 0);
                         }
                     }
                 }
             }
-            if (__ballot(h)) return true;
+            if (__ballot(h != 0)) return __ballot(h == 2) ? 2 : 1;
         }
     }
-    return false;
+    return 0;
 }
 
 template <class T>
@@ -312,77 +353,162 @@ __device__ __forceinline__ T lane_value(T v, int j) {
     return __shfl(v, j, 64);
 }
 
-// One level of the recursion: wave w takes blocks FGROUP w .. FGROUP w +
-// FGROUP - 1 of `in` (then strides), one per lane.  Each lane asks the vertex
-// table; the blocks it leaves open get the wave-cooperative full test one
-// at a time; the accepted ones split into `out` (one counter update per
-// wave) or set their cubes (a leaf: the wave takes its rows).
-__global__ __launch_bounds__(256) void k_filter_level(BlockFilter F, const FBlock *__restrict__ in,
-                                                      const uint32_t *__restrict__ nin, FBlock *__restrict__ out,
-                                                      uint32_t *__restrict__ nout, uint32_t cap) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
-    const uint32_t n = min(*nin, cap);  // (never above: the lists hold every block of a level)
-    const double *ax[3] = {F.xs, F.ys, F.zs};
-    for (uint32_t base = wave * FGROUP; base < n; base += nw * FGROUP) {
-        const uint32_t i = base + lane;
-        const bool valid = lane < FGROUP && i < n;
-        FBlock b = valid ? in[i] : FBlock{{0, 0, 0}, {0, 0, 0}};
-        // mcBlock.Bounds(epsilon) (mc.go:736-740), then the filter's
-        // Rect.Expand(extra) (shapes.go:339-344; extra 0: the rect itself)
-        double mn[3], mx[3];
-        for (int a = 0; a < 3; a++) {
-            mn[a] = (ax[a][b.mn[a]] + -F.eps) + -F.extra;
-            mx[a] = (ax[a][b.mx[a]] + F.eps) + F.extra;
+// mcBlock.Pieces(64, ...) stops at this block (mc.go:760-775).
+__device__ __forceinline__ bool is_leaf(const FBlock &b) {
+    return (int64_t)(b.mx[0] - b.mn[0]) * (b.mx[1] - b.mn[1]) * (b.mx[2] - b.mn[2]) / 2 < 64;
+}
+
+// mcBlock.Split (mc.go:777-797): a half of the longest axis (y, then z on
+// ties with x).
+__device__ __forceinline__ void halve(FBlock &b, bool second) {
+    const int lx = b.mx[0] - b.mn[0], ly = b.mx[1] - b.mn[1], lz = b.mx[2] - b.mn[2];
+    int axis = 0;
+    if (ly >= lx && ly >= lz) axis = 1;
+    else if (lz >= lx && lz >= ly) axis = 2;
+    for (int a = 0; a < 3; a++)
+        if (a == axis) {
+            const int mid = (b.mx[a] + b.mn[a]) / 2;
+            if (second) b.mn[a] = mid;
+            else b.mx[a] = mid;
         }
-        bool acc = valid && sure_hit(F.R, mn, mx);
-        for (uint64_t open = __ballot(valid && !acc); open; open &= open - 1) {
-            const int j = __ffsll((unsigned long long)open) - 1;
+}
+
+// mcBlock.Bounds(epsilon) (mc.go:736-740), then the filter's
+// Rect.Expand(extra) (shapes.go:339-344; extra 0: the rect itself).
+__device__ __forceinline__ void block_rect(const BlockFilter &F, const FBlock &b, double *mn, double *mx) {
+    const double *ax[3] = {F.xs, F.ys, F.zs};
+    for (int a = 0; a < 3; a++) {
+        mn[a] = (ax[a][b.mn[a]] + -F.eps) + -F.extra;
+        mx[a] = (ax[a][b.mx[a]] + F.eps) + F.extra;
+    }
+}
+
+// Cubes [x0, x1) of a row into the mask.
+__device__ __forceinline__ void set_cubes(unsigned long long *row, int x0, int x1) {
+    for (int x = x0; x < x1;) {
+        const int w = x >> 6, lo = x & 63, hi = min(64, x1 - (w << 6));
+        const uint64_t m = (hi >= 64 ? ~0ull : ((1ull << hi) - 1)) & (~0ull << lo);
+        atomicOr(&row[w], (unsigned long long)m);
+        x = (w << 6) + hi;
+    }
+}
+
+__device__ __forceinline__ unsigned long long *keep_row(const BlockFilter &F, int y, int z) {
+    return (unsigned long long *)F.keep + ((size_t)z * F.ny + y) * F.W;
+}
+
+// The leaf at the end of `path` (bit depth - 1 first; one path for the
+// wave), asked by the whole wave.
+__device__ void open_leaf(const BlockFilter &F, const FBlock &root, int depth, uint64_t path) {
+    const int lane = threadIdx.x & 63;
+    path = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)path) |
+           ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(path >> 32)) << 32);
+    FBlock b = root;
+    int leaf = 0;  // its depth
+    for (; leaf < depth && !is_leaf(b); leaf++) halve(b, (path >> (depth - 1 - leaf)) & 1);
+    double mn[3], mx[3];
+    block_rect(F, b, mn, mx);
+    int hit = rect_hits(F.R, mn, mx);
+    if (!hit) return;
+    if (hit == 1) {  // the blocks above (lane i: i halvings down), up to one that certainly is hit
+        FBlock u = root;
+        for (int d = 0; d < min(lane, leaf); d++) halve(u, (path >> (depth - 1 - d)) & 1);
+        block_rect(F, u, mn, mx);
+        const uint64_t sure = __ballot(lane < leaf && sure_hit(F.R, mn, mx));
+        for (int j = leaf - 1; j >= 0 && hit != 2 && !((sure >> j) & 1); j--) {
             double jmn[3], jmx[3];
             for (int a = 0; a < 3; a++) jmn[a] = lane_value(mn[a], j), jmx[a] = lane_value(mx[a], j);
-            const bool hit = rect_hits(F.R, jmn, jmx);
-            if (lane == j) acc = hit;
-        }
-        const int lx = b.mx[0] - b.mn[0], ly = b.mx[1] - b.mn[1], lz = b.mx[2] - b.mn[2];
-        const bool leaf = acc && (int64_t)lx * ly * lz / 2 < 64;  // mcBlock.Pieces(64, ...), mc.go:760-775
-        const bool split = acc && !leaf;
-        // mcBlock.Split (mc.go:777-797): halve the longest axis (y, then z
-        // on ties with x); the halves go to out[k + 2 r], r: the lane's rank
-        const uint64_t sm = __ballot(split);
-        if (sm) {
-            uint32_t k = 0;
-            if (lane == 0) k = atomicAdd(nout, 2u * (uint32_t)__popcll(sm));
-            k = lane_value(k, 0);
-            if (split) {
-                const uint32_t r = (uint32_t)__popcll(sm & ((1ull << lane) - 1));
-                int axis = 0;
-                if (ly >= lx && ly >= lz) axis = 1;
-                else if (lz >= lx && lz >= ly) axis = 2;
-                FBlock b1 = b, b2 = b;
-                b1.mx[axis] = (b.mx[axis] + b.mn[axis]) / 2;
-                b2.mn[axis] = b1.mx[axis];
-                if (k + 2 * r + 2 <= cap) out[k + 2 * r] = b1, out[k + 2 * r + 1] = b2;
-                else atomicOr(&F.ctl->filter_overflow, 1u);
-            }
-        }
-        // the leaves' cubes, one leaf at a time, its rows across the lanes
-        for (uint64_t lm = __ballot(leaf); lm; lm &= lm - 1) {
-            const int j = __ffsll((unsigned long long)lm) - 1;
-            int m0[3], m1[3];
-            for (int a = 0; a < 3; a++) m0[a] = lane_value(b.mn[a], j), m1[a] = lane_value(b.mx[a], j);
-            const int jy = m1[1] - m0[1], rows = jy * (m1[2] - m0[2]);
-            for (int r = lane; r < rows; r += 64) {
-                const int y = m0[1] + r % jy, z = m0[2] + r / jy;
-                unsigned long long *row = (unsigned long long *)F.keep + ((size_t)z * F.ny + y) * F.W;
-                for (int x = m0[0]; x < m1[0];) {
-                    const int w = x >> 6, lo = x & 63, hi = min(64, m1[0] - (w << 6));
-                    const uint64_t m = (hi >= 64 ? ~0ull : ((1ull << hi) - 1)) & (~0ull << lo);
-                    atomicOr(&row[w], (unsigned long long)m);
-                    x = (w << 6) + hi;
-                }
-            }
+            if (!(hit = rect_hits(F.R, jmn, jmx))) return;
         }
     }
+    const int jy = b.mx[1] - b.mn[1], rows = jy * (b.mx[2] - b.mn[2]);
+    for (int r = lane; r < rows; r += 64) set_cubes(keep_row(F, b.mn[1] + r % jy, b.mn[2] + r / jy), b.mn[0], b.mx[0]);
+}
+
+// Rows of a wave's common block whose cubes are gathered in LDS.
+constexpr int LEAF_ROWS = 640;
+
+// A lane per leaf; a wave's 64 leaves share the block 6 halvings up, which is
+// asked first, and whose cubes are gathered row by row before they go out.
+// The leaves left open go to the list, or where it is full are asked here.
+__global__ __launch_bounds__(256) void k_filter_leaves(BlockFilter F, FBlock root, int depth, uint64_t npath,
+                                                       uint64_t *__restrict__ open, uint32_t *__restrict__ nopen,
+                                                       uint32_t ocap) {
+    __shared__ unsigned long long rows_all[4][LEAF_ROWS];
+    const int lane = threadIdx.x & 63;
+    const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // (scalar: so is the walk to the common block)
+    unsigned long long *rows = rows_all[wid];
+    const uint64_t wave = blockIdx.x * 4ull + wid, nw = gridDim.x * 4ull;
+    const int above = depth > 6 ? depth - 6 : 0;
+    for (uint64_t base = wave * 64; base < npath; base += nw * 64) {
+        FBlock b = root;
+        int d = 0;
+        for (; d < above && !is_leaf(b); d++) halve(b, (base >> (depth - 1 - d)) & 1);
+        double mn[3], mx[3];
+        block_rect(F, b, mn, mx);
+        const bool single = d < above;  // a leaf this far up: its first path stands for it
+        if ((single && (base & ((1ull << (depth - d)) - 1))) || sure_miss(F.R, mn, mx)) continue;
+        const uint64_t path = base + lane;
+        FBlock l = b;
+        bool valid = path < npath && (!single || lane == 0);
+        if (!single) {
+            for (; d < depth && !is_leaf(l); d++) halve(l, (path >> (depth - 1 - d)) & 1);
+            valid = valid && (path & ((1ull << (depth - d)) - 1)) == 0;
+        }
+        bool acc = false, ask = false;
+        if (valid) {
+            block_rect(F, l, mn, mx);
+            if (!sure_miss(F.R, mn, mx)) acc = sure_hit(F.R, mn, mx), ask = !acc;
+        }
+        const uint64_t am = __ballot(ask);
+        if (am) {
+            uint32_t at = 0;
+            if (lane == 0) {  // (a full list's count stops growing)
+                at = __hip_atomic_load(nopen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (at < ocap) at = atomicAdd(nopen, (uint32_t)__popcll(am));
+            }
+            at = lane_value(at, 0);
+            const uint32_t mine = at + (uint32_t)__popcll(am & ((1ull << lane) - 1));
+            const bool fits = at < ocap && mine < ocap;
+            if (ask && fits) open[mine] = path;
+            for (uint64_t left = __ballot(ask && !fits); left; left &= left - 1)
+                open_leaf(F, root, depth, base + (uint64_t)(__ffsll((unsigned long long)left) - 1));
+        }
+        if (!__ballot(acc)) continue;
+        const int bx = b.mx[0] - b.mn[0], by = b.mx[1] - b.mn[1], nrows = by * (b.mx[2] - b.mn[2]);
+        const int jy = l.mx[1] - l.mn[1], lrows = acc ? jy * (l.mx[2] - l.mn[2]) : 0;
+        if (nrows <= LEAF_ROWS && bx <= 64) {
+            for (int r = lane; r < nrows; r += 64) rows[r] = 0;
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int lx = l.mx[0] - l.mn[0];
+            const uint64_t m = (lx >= 64 ? ~0ull : ((1ull << lx) - 1)) << (l.mn[0] - b.mn[0]);
+            for (int r = 0; r < lrows; r++)
+                atomicOr(&rows[(l.mn[2] + r / jy - b.mn[2]) * by + (l.mn[1] + r % jy - b.mn[1])], (unsigned long long)m);
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            const int w = b.mn[0] >> 6, sh = b.mn[0] & 63;
+            for (int r = lane; r < nrows; r += 64) {
+                const uint64_t v = rows[r];
+                if (!v) continue;
+                unsigned long long *row = keep_row(F, b.mn[1] + r % by, b.mn[2] + r / by);
+                atomicOr(&row[w], (unsigned long long)(v << sh));
+                if (sh && (v >> (64 - sh))) atomicOr(&row[w + 1], (unsigned long long)(v >> (64 - sh)));
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            for (int r = 0; r < lrows; r++) set_cubes(keep_row(F, l.mn[1] + r % jy, l.mn[2] + r / jy), l.mn[0], l.mx[0]);
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void k_filter_open(BlockFilter F, FBlock root, int depth,
+                                                     const uint64_t *__restrict__ open,
+                                                     const uint32_t *__restrict__ nopen, uint32_t ocap) {
+    const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
+    const uint32_t n = min(*nopen, ocap);
+    for (uint32_t i = wave; i < n; i += nw) open_leaf(F, root, depth, open[i]);
 }
 
 }  // namespace
@@ -393,9 +519,9 @@ hipError_t launch_rgrid_gather(const double *verts, const uint32_t *tris, uint64
     return hipGetLastError();
 }
 
-hipError_t launch_rgrid_count(const RectGridDev &R, uint32_t *counts, hipStream_t st) {
+hipError_t launch_rgrid_count(const RectGridDev &R, GroupBox *box, uint32_t *counts, hipStream_t st) {
     if (!R.ntris) return hipSuccess;
-    k_rgrid_count<<<grid_for(R.ntris, 256, 4096), 256, 0, st>>>(R, counts);
+    k_rgrid_count<<<grid_for(R.ntris, 256, 4096), 256, 0, st>>>(R, box, counts);
     return hipGetLastError();
 }
 
@@ -417,26 +543,22 @@ hipError_t launch_rgrid_fill(const RectGridDev &R, uint32_t *cursor, uint32_t *c
 
 hipError_t launch_vgrid(const RectGridDev &R, uint32_t *vsat, hipStream_t st) {
     if (R.ntris) k_vgrid_count<<<grid_for(R.ntris, 256, 4096), 256, 0, st>>>(R, vsat);
-    const uint32_t rows = (uint32_t)R.vn[1] * R.vn[2];
-    k_vsat_x<<<grid_for(rows, 4, 4096), 256, 0, st>>>(vsat, R.vn[0], rows);
-    k_vsat_yz<<<grid_for((uint64_t)R.vn[0] * R.vn[2], 256, 4096), 256, 0, st>>>(vsat, R.vn[0], R.vn[1], R.vn[2], 1);
-    k_vsat_yz<<<grid_for((uint64_t)R.vn[0] * R.vn[1], 256, 4096), 256, 0, st>>>(vsat, R.vn[0], R.vn[1], R.vn[2], 2);
+    return launch_table(vsat, R.vn, st);
+}
+
+hipError_t launch_table(uint32_t *t, const int *n, hipStream_t st) {
+    const uint32_t rows = (uint32_t)n[1] * n[2];
+    k_vsat_x<<<grid_for(rows, 4, 4096), 256, 0, st>>>(t, n[0], rows);
+    k_vsat_yz<<<grid_for((uint64_t)n[0] * n[2], 64, 4096), 64, 0, st>>>(t, n[0], n[1], n[2], 1);
+    k_vsat_yz<<<grid_for((uint64_t)n[0] * n[1], 64, 4096), 64, 0, st>>>(t, n[0], n[1], n[2], 2);
     return hipGetLastError();
 }
 
-hipError_t launch_filter_root(const FBlock &root, FBlock *front, uint32_t *level_counts, uint32_t nlevels,
-                              hipStream_t st) {
-    k_filter_root<<<1, 256, 0, st>>>(root, front, level_counts, nlevels);
-    return hipGetLastError();
-}
-
-hipError_t launch_filter_level(const BlockFilter &F, const FBlock *in, const uint32_t *nin, FBlock *out,
-                               uint32_t *nout, uint32_t cap, uint64_t max_in, hipStream_t st) {
-    // one wave per FGROUP blocks of the level (at most max_in of them), 4
-    // waves per workgroup, at most 16384 waves (they stride over the rest)
-    const uint32_t waves =
-        (uint32_t)std::min<uint64_t>(std::max<uint64_t>((max_in + FGROUP - 1) / FGROUP, 1), 16384);
-    k_filter_level<<<(waves + 3) / 4, 256, 0, st>>>(F, in, nin, out, nout, cap);
+hipError_t launch_block_filter(const BlockFilter &F, const FBlock &root, int depth, uint64_t *open, uint32_t *nopen,
+                               uint32_t ocap, hipStream_t st) {
+    const uint64_t npath = 1ull << depth;
+    k_filter_leaves<<<grid_for(npath, 256, 1u << 16), 256, 0, st>>>(F, root, depth, npath, open, nopen, ocap);
+    k_filter_open<<<grid_for(std::min<uint64_t>(npath, ocap), 4, 2048), 256, 0, st>>>(F, root, depth, open, nopen, ocap);
     return hipGetLastError();
 }
 

@@ -32,6 +32,7 @@
 #include <memory>
 #include <mutex>
 #include <new>
+#include <set>
 #include <string>
 #include <thread>
 #include <vector>
@@ -434,8 +435,8 @@ struct mc3d_ctx {
     DevBuf keep;                         // block filter: cube mask
     // z slabs: a plane's vertex list and the stitch's per-vertex arrays
     DevBuf s_flags, s_scan, s_keys, s_idx, s_count, s_keep, s_rank, s_newidx, s_bad;
-    // device block filter: triangles, their grid, the recursion's block lists
-    DevBuf rf_tris, rf_counts, rf_start, rf_cursor, rf_cells, rf_tiles, rf_front[2], rf_levels, rf_vsat;
+    // device block filter: triangles, their grid, the open leaves
+    DevBuf rf_tris, rf_box, rf_counts, rf_start, rf_cursor, rf_cells, rf_tiles, rf_open, rf_nopen, rf_vsat;
     HostBuf rf_total;
     std::shared_ptr<Pool<DevBuf>> pool = std::make_shared<Pool<DevBuf>>();
     std::shared_ptr<Pool<HostBuf>> hpool = std::make_shared<Pool<HostBuf>>();
@@ -1352,39 +1353,32 @@ int graph_launch(mc3d_ctx *ctx, const Pipe &p, const Bufs &b, const Upload &U, d
     return MC3D_OK;
 }
 
-// Blocks at each level of mcBlock.Pieces(64, ...) (mc.go:760-797) from a
-// root of l[0] x l[1] x l[2] cubes when every block is accepted: the sizes
-// the level lists need.  The halves of a split are floor and ceil of the
-// longest axis, so few distinct shapes occur per level.
-std::vector<uint64_t> filter_level_sizes(int lx, int ly, int lz) {
-    std::map<std::array<int, 3>, uint64_t> cur{{{lx, ly, lz}, 1}};
-    std::vector<uint64_t> sizes;
-    while (!cur.empty()) {
-        uint64_t total = 0;
-        std::map<std::array<int, 3>, uint64_t> next;
-        for (const auto &e : cur) {
-            total += e.second;
-            const std::array<int, 3> &d = e.first;
+// Halvings from a root of lx x ly x lz cubes to the deepest leaf of
+// mcBlock.Pieces(64, ...) (mc.go:760-797).  The halves of a split are floor
+// and ceil of the longest axis, so few distinct shapes occur per level.
+int filter_depth(int lx, int ly, int lz) {
+    std::set<std::array<int, 3>> cur{{lx, ly, lz}};
+    for (int depth = 0;; depth++) {
+        std::set<std::array<int, 3>> next;
+        for (const std::array<int, 3> &d : cur) {
             if ((int64_t)d[0] * d[1] * d[2] / 2 < 64) continue;
             int axis = 0;
             if (d[1] >= d[0] && d[1] >= d[2]) axis = 1;
             else if (d[2] >= d[0] && d[2] >= d[1]) axis = 2;
             std::array<int, 3> a = d, b = d;
             a[axis] = d[axis] / 2, b[axis] = d[axis] - d[axis] / 2;
-            next[a] += e.second;
-            next[b] += e.second;
+            next.insert(a), next.insert(b);
         }
-        sizes.push_back(total);
+        if (next.empty()) return depth;
         cur.swap(next);
     }
-    return sizes;
 }
 
 // The block filter of job j on the device, into the cube mask `keep`
 // (after the upload: it reads the grid's axes there).  The collider's
 // triangles are binned in a grid over the search grid's bounds (cells of
 // about F.cell, at most 2^20 of them; triangles outside fall in the edge
-// cells), then the recursion runs one launch per level.
+// cells), then all leaves of the recursion are asked.
 int enqueue_block_filter(mc3d_ctx *ctx, const Job &j, const Upload &U, uint64_t *keep) {
     const DeviceRectFilter &F = *j.dfilter;
     hipStream_t st = ctx->stream;
@@ -1394,7 +1388,7 @@ int enqueue_block_filter(mc3d_ctx *ctx, const Job &j, const Upload &U, uint64_t 
     }
     int rc;
     const size_t tbytes = F.ntris * 9 * sizeof(double);
-    if ((rc = ctx->rf_tris.ensure(tbytes + 8))) return rc;
+    if ((rc = ctx->rf_tris.ensure(tbytes + 8)) || (rc = ctx->rf_box.ensure(F.ntris * sizeof(GroupBox) + 8))) return rc;
     if (F.host_tris) {
         if (tbytes) HIP_TRY(hipMemcpyAsync(ctx->rf_tris.p, F.host_tris, tbytes, hipMemcpyHostToDevice, st));
     } else {
@@ -1402,6 +1396,7 @@ int enqueue_block_filter(mc3d_ctx *ctx, const Job &j, const Upload &U, uint64_t 
     }
     RectGridDev R;
     R.tris = ctx->rf_tris.as<double>();
+    R.box = ctx->rf_box.as<GroupBox>();
     R.ntris = (uint32_t)F.ntris;
     double ext[3], emax = 0;
     for (int a = 0; a < 3; a++) {
@@ -1428,7 +1423,7 @@ int enqueue_block_filter(mc3d_ctx *ctx, const Job &j, const Upload &U, uint64_t 
         (rc = ctx->rf_total.ensure(4)))
         return rc;
     HIP_TRY(hipMemsetAsync(ctx->rf_counts.p, 0, ncell * 4, st));
-    HIP_TRY(launch_rgrid_count(R, ctx->rf_counts.as<uint32_t>(), st));
+    HIP_TRY(launch_rgrid_count(R, ctx->rf_box.as<GroupBox>(), ctx->rf_counts.as<uint32_t>(), st));
     HIP_TRY(launch_rgrid_scan(ctx->rf_counts.as<uint32_t>(), (uint32_t)ncell, ctx->rf_tiles.as<uint32_t>(),
                               ctx->rf_start.as<uint32_t>(), ctx->rf_cursor.as<uint32_t>(), st));
     HIP_TRY(hipMemcpyAsync(ctx->rf_total.p, ctx->rf_start.as<uint32_t>() + ncell, 4, hipMemcpyDeviceToHost, st));
@@ -1457,27 +1452,22 @@ int enqueue_block_filter(mc3d_ctx *ctx, const Job &j, const Upload &U, uint64_t 
     HIP_TRY(launch_vgrid(R, ctx->rf_vsat.as<uint32_t>(), st));
     R.vsat = ctx->rf_vsat.as<uint32_t>();
 
-    // the recursion from the root block (mc.go:712-716), level by level
+    // (the list lengths are in cell_start: their counts become the table)
+    HIP_TRY(launch_table(ctx->rf_counts.as<uint32_t>(), R.n, st));
+    R.csat = ctx->rf_counts.as<uint32_t>();
+
+    // the recursion from the root block (mc.go:712-716)
     const FBlock root{{0, 0, 0}, {j.g.nx - 1, j.g.ny - 1, j.g.nz - 1}};
-    const std::vector<uint64_t> sizes = filter_level_sizes(root.mx[0], root.mx[1], root.mx[2]);
-    const uint64_t cap = *std::max_element(sizes.begin(), sizes.end());
-    if (cap >= (1ull << 32)) {
-        set_error("block filter: too many blocks");
-        return MC3D_E_UNSUPPORTED;
-    }
-    const uint32_t nlevels = (uint32_t)sizes.size();
-    if ((rc = ctx->rf_front[0].ensure(cap * sizeof(FBlock))) || (rc = ctx->rf_front[1].ensure(cap * sizeof(FBlock))) ||
-        (rc = ctx->rf_levels.ensure((nlevels + 1) * 4)))
-        return rc;
+    const int depth = filter_depth(root.mx[0], root.mx[1], root.mx[2]);
+    // room for a quarter of the leaves, at most 32 MiB (where the list is
+    // full, leaves are asked by the wave that found them)
+    const uint32_t ocap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>((1ull << depth) / 4, 1024), 1u << 22);
+    if ((rc = ctx->rf_open.ensure(ocap * sizeof(uint64_t))) || (rc = ctx->rf_nopen.ensure(16))) return rc;
     HIP_TRY(hipMemsetAsync(keep, 0, j.nwords * 8, st));
-    uint32_t *counts = ctx->rf_levels.as<uint32_t>();
-    FBlock *front[2] = {ctx->rf_front[0].as<FBlock>(), ctx->rf_front[1].as<FBlock>()};
-    HIP_TRY(launch_filter_root(root, front[0], counts, nlevels, st));
+    HIP_TRY(hipMemsetAsync(ctx->rf_nopen.p, 0, 4, st));
     const Grid &g = U.hsegs[0].g;
-    const BlockFilter BF{R, g.xs, g.ys, g.zs, j.delta * 1e-3, F.extra, keep, g.W, g.ny, U.ctl};
-    for (uint32_t L = 0; L < nlevels; L++)
-        HIP_TRY(launch_filter_level(BF, front[L & 1], counts + L, front[(L + 1) & 1], counts + L + 1, (uint32_t)cap,
-                                    sizes[L], st));
+    const BlockFilter BF{R, g.xs, g.ys, g.zs, j.delta * 1e-3, F.extra, keep, g.W, g.ny};
+    HIP_TRY(launch_block_filter(BF, root, depth, ctx->rf_open.as<uint64_t>(), ctx->rf_nopen.as<uint32_t>(), ocap, st));
     return MC3D_OK;
 }
 
@@ -1619,10 +1609,6 @@ int run_call(mc3d_ctx *ctx, std::vector<Job> &jobs, const mc3d_options &o, std::
             HIP_TRY(hipStreamSynchronize(ctx->copy));
             ms_d2h = ms_since(t0);
         }
-    }
-    if (hc->filter_overflow) {  // the level lists are sized for every block accepted
-        set_error("internal error: block filter level list overflow");
-        return MC3D_E_INTERNAL;
     }
     const uint64_t nv = hc->totals[0], nt = hc->totals[1];
     if (!to_host && (rc = fit_outputs(ctx, *mb, nv, nt))) return rc;
@@ -2227,7 +2213,7 @@ int mc3d_marching_cubes_c2f(mc3d_ctx *ctx, const mc3d_solid *s, double big_delta
         if ((rc = mc3d_mesh_device_ptrs(coarse, &df.dev_verts, &df.dev_tris))) return rc;
         df.ntris = coarse->nt;
         df.extra = extra;
-        df.cell = 2 * big_delta;
+        df.cell = big_delta;
         if (df.ntris && (!df.dev_verts || !df.dev_tris)) {
             set_error("internal error: coarse mesh not on the device");
             return MC3D_E_INTERNAL;
