@@ -160,21 +160,29 @@ struct GroupLevel {
     uint8_t *axis = nullptr;
     uint8_t *flag = nullptr;
 };
-// boxes and the three midpoint key arrays of triangles (verts + tris, or 9
-// doubles each when tris is null); iota[t] = t
-hipError_t launch_grp_boxes(const double *verts, const uint32_t *tris, uint32_t n, GroupBox *box, uint64_t *keys[3],
-                            uint32_t *iota, hipStream_t st);
+// boxes and midpoint keys of triangles (verts + tris, or 9 doubles each when
+// tris is null): keys[a * n + t] with vals[a * n + t] = a * step + t
+hipError_t launch_grp_boxes(const double *verts, const uint32_t *tris, uint32_t n, GroupBox *box, uint64_t *keys,
+                            uint32_t *vals, uint32_t step, hipStream_t st);
+// 3 n sorted values axis * n + triangle into the three orders, out[axis * n]
+// on (counts: 3 * grp_tiles(3 n) entries of scratch)
+hipError_t launch_grp_split(const uint32_t *vals, uint32_t n, uint32_t *counts, uint32_t *out, hipStream_t st);
 // stable radix sort of (key, value) pairs / exclusive sum (hipCUB; a null
 // tmp asks for the temporary bytes)
 hipError_t grp_sort(void *tmp, size_t &bytes, const uint64_t *keys_in, uint64_t *keys_out, const uint32_t *vals_in,
                     uint32_t *vals_out, uint32_t n, hipStream_t st);
 hipError_t grp_scan(void *tmp, size_t &bytes, const uint32_t *in, uint32_t *out, uint32_t n, hipStream_t st);
-// the axis of every node (slots: 36 keys per node of a level whose nodes
-// hold more than 64 triangles)
+// the axis of every node (slots: 36 keys per node)
 hipError_t launch_grp_axis(const GroupLevel &G, unsigned long long *slots, hipStream_t st);
 hipError_t launch_grp_flags(const GroupLevel &G, hipStream_t st);
-hipError_t launch_grp_gather_flags(const GroupLevel &G, int a, uint32_t *f, hipStream_t st);
-hipError_t launch_grp_scatter(const GroupLevel &G, int a, const uint32_t *scan, uint32_t *out, hipStream_t st);
+// the three orders partitioned by the flags into out (counts: 3 *
+// grp_tiles(n) entries of scratch)
+uint32_t grp_tiles(uint32_t n);
+hipError_t launch_grp_partition(const GroupLevel &G, uint32_t *counts, uint32_t *const out[3], hipStream_t st);
+// all further levels of nodes of at most GROUP_LOCAL triangles: the x order
+// into out (inv: n entries of scratch)
+constexpr int GROUP_LOCAL = 1024;
+hipError_t launch_grp_local(const GroupLevel &G, uint32_t *inv, uint32_t *out, hipStream_t st);
 // out[k] = the three indices of triangle perm[k]
 hipError_t launch_grp_apply(const uint32_t *tris, const uint32_t *perm, uint32_t n, uint32_t *out, hipStream_t st);
 

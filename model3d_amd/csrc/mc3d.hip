@@ -429,9 +429,9 @@ struct mc3d_ctx {
     DevBuf hvals, hpts, hstate, hprobe;  // host-evaluated atoms: answers, points, bisection state
     HostBuf hstage;                      // pinned points / answers of one callback batch
     DevBuf stl, stl_in;                  // STL encoding: body bytes; uploaded host triangles
-    // GroupTriangles: boxes, keys, the three orders (and a spare), flags,
+    // GroupTriangles: boxes, keys, the three orders (and indices), flags,
     // scans, node axes and slots, hipCUB's temporary storage
-    DevBuf g_box, g_keys[4], g_perm[4], g_flag, g_f, g_scan, g_axis, g_slots, g_tmp, g_tris;
+    DevBuf g_box, g_keys[2], g_perm[2], g_flag, g_f, g_scan, g_axis, g_slots, g_tmp, g_tris;
     DevBuf keep;                         // block filter: cube mask
     // z slabs: a plane's vertex list and the stitch's per-vertex arrays
     DevBuf s_flags, s_scan, s_keys, s_idx, s_count, s_keep, s_rank, s_newidx, s_bad;
@@ -2398,54 +2398,57 @@ int group_order(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, uint64
     }
     hipStream_t st = ctx->stream;
     int rc;
-    const size_t n4 = n * 4 + 16, n8 = n * 8 + 16;
     if ((rc = ctx->g_box.ensure(n * sizeof(GroupBox) + 16)) || (rc = ctx->g_flag.ensure(n + 16)) ||
-        (rc = ctx->g_f.ensure(n4)) || (rc = ctx->g_scan.ensure(n4)) || (rc = ctx->g_axis.ensure(n + 16)))
+        (rc = ctx->g_f.ensure(n * 4 + 16)) || (rc = ctx->g_axis.ensure(n + 16)))
         return rc;
-    for (int a = 0; a < 4; a++)
-        if ((rc = ctx->g_keys[a].ensure(n8)) || (rc = ctx->g_perm[a].ensure(n4))) return rc;
+    for (int i = 0; i < 2; i++)
+        if ((rc = ctx->g_keys[i].ensure(3 * n * 8 + 16)) || (rc = ctx->g_perm[i].ensure(3 * n * 4 + 16))) return rc;
     if (n == 0) {
         *perm = ctx->g_perm[0].as<uint32_t>();
         return MC3D_OK;
     }
     const uint32_t n32 = (uint32_t)n;
-    // the hipCUB temporary storage for the sorts and the scans
-    size_t sort_bytes = 0, scan_bytes = 0;
-    HIP_TRY(grp_sort(nullptr, sort_bytes, nullptr, nullptr, nullptr, nullptr, n32, st));
-    HIP_TRY(grp_scan(nullptr, scan_bytes, nullptr, nullptr, n32, st));
-    if ((rc = ctx->g_tmp.ensure(std::max(sort_bytes, scan_bytes) + 16))) return rc;
-    uint64_t *keys[3] = {ctx->g_keys[0].as<uint64_t>(), ctx->g_keys[1].as<uint64_t>(), ctx->g_keys[2].as<uint64_t>()};
-    uint32_t *iota = ctx->g_perm[3].as<uint32_t>();
-    HIP_TRY(launch_grp_boxes(verts, tris, n32, ctx->g_box.as<GroupBox>(), keys, iota, st));
-    uint32_t *P[4] = {ctx->g_perm[0].as<uint32_t>(), ctx->g_perm[1].as<uint32_t>(), ctx->g_perm[2].as<uint32_t>(),
-                      iota};
-    for (int a = 0; a < 3; a++) {
+    // One sort of the three axes' keys, then each axis's own out of it: a sort
+    // of a few hundred thousand keys is bound by its launches (203k triangles:
+    // 253 us, split included, for 574 us in three).  Past the sort's 2^31 entries
+    // there are three.
+    const bool one = 3 * n < (1ull << 31);
+    const uint32_t entries = one ? 3 * n32 : n32;
+    size_t sort_bytes = 0;
+    HIP_TRY(grp_sort(nullptr, sort_bytes, nullptr, nullptr, nullptr, nullptr, entries, st));
+    if ((rc = ctx->g_tmp.ensure(sort_bytes + 16)) || (rc = ctx->g_scan.ensure(3 * (size_t)grp_tiles(entries) * 4 + 16)))
+        return rc;
+    uint64_t *k_in = ctx->g_keys[0].as<uint64_t>(), *k_out = ctx->g_keys[1].as<uint64_t>();
+    uint32_t *orders = ctx->g_perm[0].as<uint32_t>(), *other = ctx->g_perm[1].as<uint32_t>();
+    HIP_TRY(launch_grp_boxes(verts, tris, n32, ctx->g_box.as<GroupBox>(), k_in, orders, one ? n32 : 0, st));
+    for (uint64_t at = 0; at < 3 * n; at += entries) {
         size_t bytes = ctx->g_tmp.cap;
-        HIP_TRY(grp_sort(ctx->g_tmp.p, bytes, keys[a], ctx->g_keys[3].as<uint64_t>(), iota, P[a], n32, st));
+        HIP_TRY(grp_sort(ctx->g_tmp.p, bytes, k_in + at, k_out + at, orders + at, other + at, entries, st));
     }
-    // the levels, until every node holds at most one triangle
+    if (one) HIP_TRY(launch_grp_split(other, n32, ctx->g_scan.as<uint32_t>(), orders, st));
+    else std::swap(orders, other);
+    uint32_t *P[3] = {orders, orders + n, orders + 2 * n}, *Q[3] = {other, other + n, other + 2 * n};
+    // the levels above nodes that a block takes whole, then the rest at once
     int levels = 0;
-    while ((n32 + (1u << levels) - 1) >> levels > 1) levels++;
-    const uint32_t big_nodes = std::max<uint32_t>(1, n32 / 64 + 1);  // nodes of a level of nodes above 64
-    if ((rc = ctx->g_slots.ensure((size_t)big_nodes * 36 * 8 + 16))) return rc;
+    while ((n32 + (1u << levels) - 1) >> levels > GROUP_LOCAL) levels++;
+    if ((rc = ctx->g_slots.ensure(((size_t)1 << levels) * 36 * 8 + 16))) return rc;
     GroupLevel G;
     G.n = n32;
     G.box = ctx->g_box.as<GroupBox>();
     G.axis = ctx->g_axis.as<uint8_t>();
     G.flag = ctx->g_flag.as<uint8_t>();
-    uint32_t *spare = P[3];
-    for (int L = 0; L < levels; L++) {
+    for (int L = 0; L <= levels; L++) {
         G.L = L;
         for (int a = 0; a < 3; a++) G.perm[a] = P[a];
+        if (L == levels) {
+            HIP_TRY(launch_grp_local(G, ctx->g_f.as<uint32_t>(), Q[0], st));
+            std::swap(P[0], Q[0]);
+            break;
+        }
         HIP_TRY(launch_grp_axis(G, ctx->g_slots.as<unsigned long long>(), st));
         HIP_TRY(launch_grp_flags(G, st));
-        for (int a = 0; a < 3; a++) {
-            HIP_TRY(launch_grp_gather_flags(G, a, ctx->g_f.as<uint32_t>(), st));
-            size_t bytes = ctx->g_tmp.cap;
-            HIP_TRY(grp_scan(ctx->g_tmp.p, bytes, ctx->g_f.as<uint32_t>(), ctx->g_scan.as<uint32_t>(), n32, st));
-            HIP_TRY(launch_grp_scatter(G, a, ctx->g_scan.as<uint32_t>(), spare, st));
-            std::swap(P[a], spare);
-        }
+        HIP_TRY(launch_grp_partition(G, ctx->g_scan.as<uint32_t>(), Q, st));
+        for (int a = 0; a < 3; a++) std::swap(P[a], Q[a]);
     }
     *perm = P[0];
     return MC3D_OK;
