@@ -583,10 +583,6 @@ hipError_t grp_sort(void *tmp, size_t &bytes, const uint64_t *keys_in, uint64_t 
     return hipcub::DeviceRadixSort::SortPairs(tmp, bytes, keys_in, keys_out, vals_in, vals_out, (int)n, 0, 64, st);
 }
 
-hipError_t grp_scan(void *tmp, size_t &bytes, const uint32_t *in, uint32_t *out, uint32_t n, hipStream_t st) {
-    return hipcub::DeviceScan::ExclusiveSum(tmp, bytes, in, out, (int)n, st);
-}
-
 hipError_t launch_grp_axis(const GroupLevel &G, unsigned long long *slots, hipStream_t st) {
     const uint32_t nodes = 1u << G.L;
     k_grp_slots_init<<<grid_for((uint64_t)nodes * 36, 256, 4096), 256, 0, st>>>(slots, nodes);

@@ -167,11 +167,10 @@ hipError_t launch_grp_boxes(const double *verts, const uint32_t *tris, uint32_t 
 // 3 n sorted values axis * n + triangle into the three orders, out[axis * n]
 // on (counts: 3 * grp_tiles(3 n) entries of scratch)
 hipError_t launch_grp_split(const uint32_t *vals, uint32_t n, uint32_t *counts, uint32_t *out, hipStream_t st);
-// stable radix sort of (key, value) pairs / exclusive sum (hipCUB; a null
-// tmp asks for the temporary bytes)
+// stable radix sort of (key, value) pairs (hipCUB; a null tmp asks for the
+// temporary bytes)
 hipError_t grp_sort(void *tmp, size_t &bytes, const uint64_t *keys_in, uint64_t *keys_out, const uint32_t *vals_in,
                     uint32_t *vals_out, uint32_t n, hipStream_t st);
-hipError_t grp_scan(void *tmp, size_t &bytes, const uint32_t *in, uint32_t *out, uint32_t n, hipStream_t st);
 // the axis of every node (slots: 36 keys per node)
 hipError_t launch_grp_axis(const GroupLevel &G, unsigned long long *slots, hipStream_t st);
 hipError_t launch_grp_flags(const GroupLevel &G, hipStream_t st);
@@ -186,28 +185,44 @@ hipError_t launch_grp_local(const GroupLevel &G, uint32_t *inv, uint32_t *out, h
 // out[k] = the three indices of triangle perm[k]
 hipError_t launch_grp_apply(const uint32_t *tris, const uint32_t *perm, uint32_t n, uint32_t *out, hipStream_t st);
 
-// z-slab stitching (k_slab.hip).  The x and y edges of plane z among a
-// slab's vertices (keys vkeys): keys without z and vertex indices, in
-// vertex order, *count of them (flags, scan: nv entries of scratch; tmp:
-// grp_scan's temporary storage).
-hipError_t launch_plane_list(const uint64_t *vkeys, uint32_t nv, uint32_t z, uint32_t *flags, uint32_t *scan,
-                             void *tmp, size_t tmp_bytes, uint64_t *keys, uint32_t *idx, uint32_t *count,
-                             hipStream_t st);
-// keep[i] = 1, then 0 at the ndrop indices of drop
-hipError_t launch_stitch_keep(uint32_t *keep, uint32_t nv, const uint32_t *drop, uint32_t ndrop, hipStream_t st);
-// kept vertex i (rank: exclusive sums of keep) to fv[vbase + rank[i]] (and
-// its interior point to fin); newidx[i] = its index in the mesh
-hipError_t launch_stitch_verts(const double *v, const double *in, uint32_t nv, const uint32_t *keep,
-                               const uint32_t *rank, uint32_t vbase, double *fv, double *fin, uint32_t *newidx,
-                               hipStream_t st);
-// newidx[up_idx[j]] = lo_global[j] (both lists sorted by key; a key
-// mismatch sets *bad)
-hipError_t launch_stitch_pairs(const uint64_t *lo_keys, const uint32_t *lo_global, const uint64_t *up_keys,
-                               const uint32_t *up_idx, uint32_t m, uint32_t *newidx, uint32_t *bad, hipStream_t st);
-hipError_t launch_stitch_tris(const uint32_t *t, uint64_t nt, const uint32_t *newidx, uint32_t *ft, hipStream_t st);
-// global[j] = newidx[idx[j]]
-hipError_t launch_stitch_globals(const uint32_t *idx, uint32_t m, const uint32_t *newidx, uint32_t *global,
-                                 hipStream_t st);
+// z-slab stitching (k_slab.hip).  What a slab's rank pass leaves: the
+// vertices on its bottom and its top plane, its own vertices, and whether a
+// bottom vertex was missing below.
+struct SlabEnd {
+    uint32_t bottom, top, kept, bad;
+};
+// One slab's rank pass.  Vertices with keys vkeys; plane zbot is shared with
+// the slab below and plane ztop with the one above (-1: none).  The slab's
+// top plane goes into a table of 2^top_bits slots, at least twice the plane's
+// vertices; the slab below left its own.  counts: slab_tiles(nv) entries of
+// scratch.
+struct SlabPart {
+    const uint64_t *vkeys = nullptr;
+    uint64_t nv = 0;
+    uint32_t ntiles = 0;
+    bool scanned = false;
+    int zbot = -1, ztop = -1;
+    uint64_t *top_keys = nullptr;
+    uint32_t *top_vals = nullptr;
+    int top_bits = 1;
+    const uint64_t *below_keys = nullptr;
+    const uint32_t *below_vals = nullptr;
+    int below_bits = 1;
+    const SlabEnd *below_end = nullptr;
+    SlabEnd *end = nullptr;
+    uint32_t *counts = nullptr, *rank = nullptr;
+};
+uint32_t slab_tiles(uint64_t nv);
+hipError_t launch_slab_rank(SlabPart S, hipStream_t st);
+// A slab's mesh and its place in the stitched one.
+struct StitchPiece {
+    const double *v, *in;
+    const uint32_t *t, *rank;
+    uint64_t nv, nt, tbase;
+    uint32_t vbase, pad;
+};
+hipError_t launch_stitch(const StitchPiece *pieces, uint32_t npieces, uint64_t nv_max, uint64_t nt_max, double *fv,
+                         double *fin, uint32_t *ft, hipStream_t st);
 
 inline unsigned grid_for(uint64_t n, unsigned block, unsigned cap = 1u << 20) {
     uint64_t b = (n + block - 1) / block;

@@ -434,7 +434,7 @@ struct mc3d_ctx {
     DevBuf g_box, g_keys[2], g_perm[2], g_flag, g_f, g_scan, g_axis, g_slots, g_tmp, g_tris;
     DevBuf keep;                         // block filter: cube mask
     // z slabs: a plane's vertex list and the stitch's per-vertex arrays
-    DevBuf s_flags, s_scan, s_keys, s_idx, s_count, s_keep, s_rank, s_newidx, s_bad;
+    DevBuf s_counts, s_keys[2], s_vals[2], s_ends, s_pieces;
     // device block filter: triangles, their grid, the open leaves
     DevBuf rf_tris, rf_box, rf_counts, rf_start, rf_cursor, rf_cells, rf_tiles, rf_open, rf_nopen, rf_vsat;
     HostBuf rf_total;
@@ -1882,43 +1882,6 @@ namespace {
 // (MarchingCubesConj).
 using RectFilter = std::function<bool(const double *, const double *)>;
 
-// The x and y edges of slab plane z among the last call's nv vertices
-// (ctx->vkeys): their keys without z and the slab's vertex indices, sorted
-// by key; `global` is left for their indices in the stitched mesh.
-struct PlaneList {
-    std::unique_ptr<DevBuf> keys{new DevBuf}, idx{new DevBuf}, global{new DevBuf};
-    uint32_t n = 0;
-};
-
-int plane_list(mc3d_ctx *ctx, uint32_t nv, uint32_t z, PlaneList &out) {
-    hipStream_t st = ctx->stream;
-    int rc;
-    size_t scan_bytes = 0, sort_bytes = 0;
-    HIP_TRY(grp_scan(nullptr, scan_bytes, nullptr, nullptr, std::max<uint32_t>(nv, 1), st));
-    HIP_TRY(grp_sort(nullptr, sort_bytes, nullptr, nullptr, nullptr, nullptr, std::max<uint32_t>(nv, 1), st));
-    if ((rc = ctx->s_flags.ensure(nv * 4 + 16)) || (rc = ctx->s_scan.ensure(nv * 4 + 16)) ||
-        (rc = ctx->s_keys.ensure(nv * 8 + 16)) || (rc = ctx->s_idx.ensure(nv * 4 + 16)) ||
-        (rc = ctx->s_count.ensure(16)) || (rc = ctx->rf_total.ensure(4)) ||
-        (rc = ctx->g_tmp.ensure(std::max(scan_bytes, sort_bytes) + 16)))
-        return rc;
-    HIP_TRY(launch_plane_list(ctx->vkeys.as<uint64_t>(), nv, z, ctx->s_flags.as<uint32_t>(),
-                              ctx->s_scan.as<uint32_t>(), ctx->g_tmp.p, ctx->g_tmp.cap, ctx->s_keys.as<uint64_t>(),
-                              ctx->s_idx.as<uint32_t>(), ctx->s_count.as<uint32_t>(), st));
-    HIP_TRY(hipMemcpyAsync(ctx->rf_total.p, ctx->s_count.p, 4, hipMemcpyDeviceToHost, st));
-    HIP_TRY(hipStreamSynchronize(st));
-    const uint32_t m = *ctx->rf_total.as<uint32_t>();
-    if ((rc = out.keys->ensure((size_t)m * 8 + 16)) || (rc = out.idx->ensure((size_t)m * 4 + 16)) ||
-        (rc = out.global->ensure((size_t)m * 4 + 16)))
-        return rc;
-    if (m) {
-        size_t bytes = ctx->g_tmp.cap;
-        HIP_TRY(grp_sort(ctx->g_tmp.p, bytes, ctx->s_keys.as<uint64_t>(), out.keys->as<uint64_t>(),
-                         ctx->s_idx.as<uint32_t>(), out.idx->as<uint32_t>(), m, st));
-    }
-    out.n = m;
-    return MC3D_OK;
-}
-
 // MarchingCubesSearch of one solid in z slabs of `planes` cube layers
 // (mc.go:614-645 keeps only a few planes alive; here device memory for the
 // grid is bounded by one slab): each slab runs the pipeline on corner planes
@@ -1937,10 +1900,21 @@ int search_slabs(mc3d_ctx *ctx, Job &base, const mc3d_options &o, int planes, mc
     so.no_graph = 1;
     struct Piece {
         std::unique_ptr<mc3d_mesh, void (*)(mc3d_mesh *)> m{nullptr, mc3d_mesh_free};
-        PlaneList top, bot;
+        std::unique_ptr<DevBuf> rank;
     };
+    const size_t npieces = (size_t)(ncube + planes - 1) / planes;
     std::vector<Piece> pieces;
-    pieces.reserve((size_t)(ncube + planes - 1) / planes);
+    pieces.reserve(npieces);
+    int table_bits[2] = {1, 1};  // of the top planes' edges, slabs in turn
+    // (the ranks' buffers go back to the pool however the call ends)
+    struct Return {
+        mc3d_ctx *ctx;
+        std::vector<Piece> &pieces;
+        ~Return() {
+            (void)hipStreamSynchronize(ctx->stream);
+            for (Piece &p : pieces) ctx->pool->give(std::move(p.rank));
+        }
+    } on_return{ctx, pieces};
     int rc;
     for (int c0 = 0; c0 < ncube; c0 += planes) {
         const int c1 = std::min(ncube, c0 + planes);
@@ -1962,20 +1936,54 @@ int search_slabs(mc3d_ctx *ctx, Job &base, const mc3d_options &o, int planes, mc
             set_error("mesh too large for 32-bit vertex indices");
             return MC3D_E_UNSUPPORTED;
         }
-        const uint32_t nv = (uint32_t)pc.m->nv;
-        if (c0 > 0 && (rc = plane_list(ctx, nv, 0, pc.bot))) return rc;
-        if (c1 < ncube && (rc = plane_list(ctx, nv, (uint32_t)(c1 - c0), pc.top))) return rc;
+        const uint64_t nv = pc.m->nv;
+        const size_t k = pieces.size() - 1, cur = k & 1;
+        SlabPart S;
+        S.vkeys = ctx->vkeys.as<uint64_t>();
+        S.nv = nv;
+        pc.rank = ctx->pool->take(nv * 4 + 16);
+        if ((rc = pc.rank->ensure(nv * 4 + 16)) || (rc = ctx->s_counts.ensure((size_t)slab_tiles(nv) * 4)) ||
+            (rc = ctx->s_ends.ensure(npieces * sizeof(SlabEnd))))
+            return rc;
+        S.rank = pc.rank->as<uint32_t>();
+        S.counts = ctx->s_counts.as<uint32_t>();
+        S.end = ctx->s_ends.as<SlabEnd>() + k;
+        if (c0 > 0) {
+            S.zbot = 0;
+            S.below_keys = ctx->s_keys[cur ^ 1].as<uint64_t>(), S.below_vals = ctx->s_vals[cur ^ 1].as<uint32_t>();
+            S.below_bits = table_bits[cur ^ 1];
+            S.below_end = S.end - 1;
+        }
+        if (c1 < ncube) {
+            const uint64_t most = std::min<uint64_t>(nv, 2ull * j.g.nx * j.g.ny);  // vertices of a plane
+            int bits = 6;
+            while ((1ull << bits) < 2 * most) bits++;
+            S.ztop = c1 - c0;
+            if ((rc = ctx->s_keys[cur].ensure(8ull << bits)) || (rc = ctx->s_vals[cur].ensure(4ull << bits))) return rc;
+            S.top_keys = ctx->s_keys[cur].as<uint64_t>(), S.top_vals = ctx->s_vals[cur].as<uint32_t>();
+            S.top_bits = table_bits[cur] = bits;
+        }
+        HIP_TRY(launch_slab_rank(S, ctx->stream));
     }
     // the stitched mesh's sizes and buffers
-    uint64_t nv_all = 0, nt_all = 0, nv_max = 0;
-    for (size_t k = 0; k < pieces.size(); k++) {
-        if (k && pieces[k].bot.n != pieces[k - 1].top.n) {
+    hipStream_t st = ctx->stream;
+    const size_t ends_bytes = npieces * sizeof(SlabEnd), table_bytes = npieces * sizeof(StitchPiece);
+    if ((rc = ctx->rf_total.ensure(std::max(ends_bytes, table_bytes))) || (rc = ctx->s_pieces.ensure(table_bytes)))
+        return rc;
+    HIP_TRY(hipMemcpyAsync(ctx->rf_total.p, ctx->s_ends.p, ends_bytes, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    std::vector<SlabEnd> ends(npieces);
+    memcpy(ends.data(), ctx->rf_total.p, ends_bytes);
+    uint64_t nv_all = 0, nt_all = 0, nv_max = 0, nt_max = 0;
+    for (size_t k = 0; k < npieces; k++) {
+        if (k && (ends[k].bottom != ends[k - 1].top || ends[k].bad)) {
             set_error("internal error: z slabs disagree on a shared plane's vertices");
             return MC3D_E_INTERNAL;
         }
-        nv_all += pieces[k].m->nv - pieces[k].bot.n;
+        nv_all += pieces[k].m->nv - ends[k].bottom;
         nt_all += pieces[k].m->nt;
         nv_max = std::max<uint64_t>(nv_max, pieces[k].m->nv);
+        nt_max = std::max<uint64_t>(nt_max, pieces[k].m->nt);
     }
     if (nv_all >= (1ull << 32) || nt_all >= (1ull << 32)) {
         set_error("mesh too large for 32-bit vertex indices");
@@ -1992,53 +2000,28 @@ int search_slabs(mc3d_ctx *ctx, Job &base, const mc3d_options &o, int planes, mc
         mb->interior = ctx->pool->take(nv_all * 24 + 16);
         if ((rc = mb->interior->ensure(nv_all * 24 + 16))) return rc;
     }
-    size_t scan_bytes = 0;
-    hipStream_t st = ctx->stream;
-    HIP_TRY(grp_scan(nullptr, scan_bytes, nullptr, nullptr, (uint32_t)std::max<uint64_t>(nv_max, 1), st));
-    if ((rc = ctx->s_keep.ensure(nv_max * 4 + 16)) || (rc = ctx->s_rank.ensure(nv_max * 4 + 16)) ||
-        (rc = ctx->s_newidx.ensure(nv_max * 4 + 16)) || (rc = ctx->s_bad.ensure(16)) ||
-        (rc = ctx->g_tmp.ensure(scan_bytes + 16)) || (rc = ctx->rf_total.ensure(4)))
-        return rc;
-    HIP_TRY(hipMemsetAsync(ctx->s_bad.p, 0, 4, st));
-    uint32_t vbase = 0;
-    uint64_t tbase = 0;
-    uint32_t *keep = ctx->s_keep.as<uint32_t>(), *rank = ctx->s_rank.as<uint32_t>();
-    uint32_t *newidx = ctx->s_newidx.as<uint32_t>();
-    for (size_t k = 0; k < pieces.size(); k++) {
+    StitchPiece *table = ctx->rf_total.as<StitchPiece>();
+    uint64_t vbase = 0, tbase = 0;
+    for (size_t k = 0; k < npieces; k++) {
         const mc3d_mesh &m = *pieces[k].m;
-        const uint32_t nv = (uint32_t)m.nv;
-        const PlaneList &bot = pieces[k].bot;
-        const double *v = m.buf->verts->as<double>() + 3 * m.voff;
-        const double *in = interior ? m.buf->interior->as<double>() + 3 * m.voff : nullptr;
-        const uint32_t *t = m.buf->tris->as<uint32_t>() + 3 * m.toff;
-        HIP_TRY(launch_stitch_keep(keep, nv, bot.idx->as<uint32_t>(), bot.n, st));
-        if (nv) {
-            size_t bytes = ctx->g_tmp.cap;
-            HIP_TRY(grp_scan(ctx->g_tmp.p, bytes, keep, rank, nv, st));
-        }
-        HIP_TRY(launch_stitch_verts(v, in, nv, keep, rank, vbase, mb->verts->as<double>(),
-                                    interior ? mb->interior->as<double>() : nullptr, newidx, st));
-        if (k)
-            HIP_TRY(launch_stitch_pairs(pieces[k - 1].top.keys->as<uint64_t>(), pieces[k - 1].top.global->as<uint32_t>(),
-                                        bot.keys->as<uint64_t>(), bot.idx->as<uint32_t>(), bot.n, newidx,
-                                        ctx->s_bad.as<uint32_t>(), st));
-        HIP_TRY(launch_stitch_tris(t, m.nt, newidx, mb->tris->as<uint32_t>() + 3 * tbase, st));
-        const PlaneList &top = pieces[k].top;
-        HIP_TRY(launch_stitch_globals(top.idx->as<uint32_t>(), top.n, newidx, top.global->as<uint32_t>(), st));
-        vbase += nv - bot.n;
+        StitchPiece &P = table[k];
+        P.v = m.buf->verts->as<double>() + 3 * m.voff;
+        P.in = interior ? m.buf->interior->as<double>() + 3 * m.voff : nullptr;
+        P.t = m.buf->tris->as<uint32_t>() + 3 * m.toff;
+        P.rank = pieces[k].rank->as<uint32_t>();
+        P.nv = m.nv, P.nt = m.nt, P.tbase = tbase;
+        P.vbase = (uint32_t)vbase, P.pad = 0;
+        vbase += m.nv - ends[k].bottom;
         tbase += m.nt;
     }
-    HIP_TRY(hipMemcpyAsync(ctx->rf_total.p, ctx->s_bad.p, 4, hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(ctx->s_pieces.p, table, table_bytes, hipMemcpyHostToDevice, st));
+    HIP_TRY(launch_stitch(ctx->s_pieces.as<StitchPiece>(), (uint32_t)npieces, nv_max, nt_max, mb->verts->as<double>(),
+                          interior ? mb->interior->as<double>() : nullptr, mb->tris->as<uint32_t>(), st));
     HIP_TRY(hipEventRecord(ctx->ev[EV_EMIT1], st));
     HIP_TRY(hipEventRecord(ctx->ev[EV_OUT], st));
     const bool to_host = !o.device_only;
     if (to_host && (rc = enqueue_host_copy(ctx, *mb, nv_all, nt_all, interior))) return rc;
     HIP_TRY(hipStreamSynchronize(st));
-    if (*ctx->rf_total.as<uint32_t>()) {
-        if (to_host) (void)hipStreamSynchronize(ctx->copy);
-        set_error("internal error: z slabs disagree on a shared plane's edges");
-        return MC3D_E_INTERNAL;
-    }
     double ms_d2h = 0;
     if (to_host) {
         const auto t0 = std::chrono::steady_clock::now();
