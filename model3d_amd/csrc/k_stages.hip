@@ -231,14 +231,16 @@ hipError_t launch_plan(const Pipe &p, const Bufs &b, hipStream_t st) {
         units = (uint64_t)p.seg0.g.W * ((p.seg0.B.nby + ty - 1) / ty) * ((p.seg0.B.nbz + tz - 1) / tz);
     }
     const unsigned pgrid = grid_for(units, PLAN_BLOCK / 64, 1u << 16);
+    const uint32_t wave_lds = (uint32_t)plan_wave_bytes(p.plan_blocks, p.stack);
+    const size_t lds = PLAN_BLOCK / 64 * wave_lds;
     if (p.nsegs > 1)
-        k_plan<true><<<pgrid, PLAN_BLOCK, p.plan_lds, st>>>(p.segs, p.nsegs, p.seg0, p.brick_seg, p.nbricks, p.cap,
+        k_plan<true><<<pgrid, PLAN_BLOCK, lds, st>>>(p.segs, p.nsegs, p.seg0, p.brick_seg, p.nbricks, p.cap,
                                                             b.binfo, b.bcode, b.actb, b.bits, p.ctl, p.sout,
-                                                            p.plan_gsz, false);
+                                                            p.plan_gsz, false, p.plan_blocks, wave_lds);
     else
-        k_plan<false><<<pgrid, PLAN_BLOCK, p.plan_lds, st>>>(p.segs, p.nsegs, p.seg0, p.brick_seg, p.nbricks, p.cap,
+        k_plan<false><<<pgrid, PLAN_BLOCK, lds, st>>>(p.segs, p.nsegs, p.seg0, p.brick_seg, p.nbricks, p.cap,
                                                              b.binfo, b.bcode, b.actb, b.bits, p.ctl, p.sout,
-                                                             p.plan_gsz, p.plan_tile);
+                                                             p.plan_gsz, p.plan_tile, p.plan_blocks, wave_lds);
     return hipGetLastError();
 }
 

@@ -124,18 +124,23 @@ __device__ __forceinline__ void wave_sync() {
 // ---------------------------------------------------------------------------
 // plan
 // ---------------------------------------------------------------------------
-// One thread per brick folds the postfix program (plan_fold_skip: a subtree
-// whose atoms miss every brick of the wave is replaced by its constant
-// without a walk, so the walk stays the same for the whole wave; a wave's
-// bricks are consecutive, so its constant bricks' words are written row by
-// row) and writes
-// the folded program into the brick's slot of `cap` instructions.  A brick
-// whose folded code ever needs more than `cap` slots uses the unfolded
-// program.  A brick where the solid is constant gets its occupancy words
-// here (all false, or every valid corner true, with the check that no
-// boundary corner is inside: panic("solid is true outside of bounds"),
-// mc.go:687-689).  With `stage`, the program's node records are first copied
-// to LDS; otherwise the uniform walk reads them with scalar loads.  The per-brick statistics are reduced per wave.
+// One thread per brick folds the postfix program into the brick's slot of
+// `cap` instructions.  A brick whose folded code ever needs more than `cap`
+// slots uses the unfolded program.  A brick where the solid is constant gets
+// its occupancy words here (all false, or every valid corner true, with the
+// check that no boundary corner is inside: panic("solid is true outside of
+// bounds"), mc.go:687-689).  The per-brick statistics are reduced per wave.
+//
+// The fold's walk is a serial chain, so what counts is how few nodes a wave
+// walks: of a large program most atoms miss the wave's bricks.  A lane per
+// node tests 64 atoms at once against the bricks' common box; from the counts
+// of atoms that meet it, each node says for itself whether it has to be walked
+// (plan_step_of), and the wave walks that list, PLAN_CHUNK node records at a
+// time in LDS.  (A walk over all nodes that skipped a missing subtree on its
+// way, its program whole in LDS or read by scalar loads, took 70 us
+// for one slab of the 512-atom solid at spacing 0.003 and 52 us for the
+// 64-atom one at 0.005 in bricks of 4; the lists take 34 and 20 us.)  Programs of
+// more than PLAN_LIST_MAX nodes, whose masks would fill the LDS, keep that walk.
 // Bricks a plan wave takes at once: its first `gsz` lanes (a power of two
 // <= 64) hold `gsz` consecutive bricks, or with `tile` (a call of one
 // solid) a tile of one word column by ty brick rows by gsz / ty brick
@@ -149,17 +154,28 @@ __device__ __forceinline__ uint64_t plan_units(const Seg &s0, uint64_t nbricks_a
     return (uint64_t)s0.g.W * ((s0.B.nby + ty - 1) / ty) * ((s0.B.nbz + tz - 1) / tz);
 }
 
+// A lane's stack, entries a wave apart (no two lanes in a bank).
+struct LaneStack {
+    uint32_t *p;
+    __device__ __forceinline__ uint32_t &operator[](int i) const { return p[i * 64]; }
+};
+
 template <bool MULTI>
 __global__ __launch_bounds__(PLAN_BLOCK) void k_plan(const Seg *__restrict__ segs, uint32_t nsegs, const Seg seg0,
                                                      const uint32_t *__restrict__ brick_seg, uint64_t nbricks_all,
                                                      uint32_t cap, uint2 *__restrict__ info, Insn *__restrict__ out,
                                                      uint32_t *__restrict__ act_list, uint64_t *__restrict__ bits_all,
                                                      Ctl *__restrict__ ctl, SegOut *__restrict__ sout, uint32_t gsz,
-                                                     bool tile) {
+                                                     bool tile, uint32_t blocks64, uint32_t wave_lds) {
     extern __shared__ __align__(16) char plan_smem[];
-    uint32_t *S = (uint32_t *)plan_smem + threadIdx.x * PLAN_STACK;
-    uint32_t staged = ~0u;  // segment whose program is in LDS
     const int lane = threadIdx.x & 63, wave = wave_id();
+    // the wave's own LDS (plan_wave_bytes)
+    char *const mem = plan_smem + (size_t)wave * wave_lds;
+    PlanNode *const recs = (PlanNode *)mem;
+    uint64_t *const masks = (uint64_t *)(mem + PLAN_CHUNK * sizeof(PlanNode));
+    uint32_t *const ring = (uint32_t *)(masks + blocks64);
+    uint32_t *const before = ring + PLAN_RING;
+    const LaneStack S{before + blocks64 + lane};
     constexpr int WPB = PLAN_BLOCK / 64;
     tile = tile && !MULTI;
     const uint64_t nunits = plan_units<MULTI>(seg0, nbricks_all, gsz, tile);
@@ -202,35 +218,71 @@ __global__ __launch_bounds__(PLAN_BLOCK) void k_plan(const Seg *__restrict__ seg
         const int x1 = min(x0 + 64, g.nx - 1), y1 = min(y0 + B.BY, g.ny - 1), z1 = min(z0 + B.BZ, g.nz - 1);
         const double lo[3] = {g.xs[x0], g.ys[y0], g.zs[z0]};
         const double hi[3] = {g.xs[x1], g.ys[y1], g.zs[z1]};
-        // a staged program's node records in LDS
-        PlanNode *sn = (PlanNode *)(plan_smem + PLAN_STACK_BYTES);
-        if (sg.stage) {  // block-uniform
-            if (staged != si) {
-                __syncthreads();  // the previous segment's walks are done with the LDS copy
-                const uint4 *src = (const uint4 *)P.plan;
-                uint4 *dst = (uint4 *)sn;
-                // copied by the LDS DMA (16 bytes a lane, 1 KiB a wave per
-                // load, no registers), all loads in flight before the wait
-                const uint32_t nq = P.ncode * (uint32_t)(sizeof(PlanNode) / 16);
-                for (uint32_t c = (uint32_t)wave; c * 64 < nq; c += WPB)
-                    if (c * 64 + (uint32_t)lane < nq)
-                        __builtin_amdgcn_global_load_lds(
-                            (const void __attribute__((address_space(1))) *)(src + c * 64 + lane),
-                            (void __attribute__((address_space(3))) *)(dst + c * 64), 16, 0, 0);
-                __builtin_amdgcn_s_waitcnt(VMCNT0);
-                __syncthreads();
-                staged = si;
-            }
-        }
         Insn *o = out + (valid ? gb * cap : 0);
         const uint32_t ocap = valid ? cap : 0u;
         uint32_t n = 0;
         bool over = false;
-        // two copies of the fold, so that each reads with typed
-        // instructions: LDS, or scalar loads for programs too large to stage
-        if (sg.stage) {
-            auto miss = [&](const PlanNode &t) { return __ballot(valid && !node_misses(t, lo, hi)) == 0; };
-            plan_fold_nodes((const PlanNode *)sn, P.ncode, S, lo, hi, o, ocap, n, over, miss);
+        if (sg.listed) {
+            // the bricks' common box, rounded outwards
+            float ulo[3], uhi[3];
+            for (int k = 0; k < 3; k++) {
+                ulo[k] = valid ? __double2float_rd(lo[k]) : INFINITY;
+                uhi[k] = valid ? __double2float_ru(hi[k]) : -INFINITY;
+            }
+            for (int d = 32; d; d >>= 1)
+                for (int k = 0; k < 3; k++) {
+                    ulo[k] = fminf(ulo[k], __shfl_xor(ulo[k], d));
+                    uhi[k] = fmaxf(uhi[k], __shfl_xor(uhi[k], d));
+                }
+            const PlanNode *nodes = P.plan;
+            const PlanTest *tests = (const PlanTest *)(nodes + P.ncode);
+            const uint32_t nb = (P.ncode + 63) / 64;
+            uint32_t live = 0, head = 0, tail = 0;  // atoms that meet the box; the ring's ends
+            int sp = 0;
+            PlanTest next = tests[min((uint32_t)lane, P.ncode - 1)];
+            for (uint32_t c = 0; c < nb; c++) {
+                const uint32_t i = c * 64 + lane;
+                const PlanTest t = next;
+                if (c + 1 < nb) next = tests[min(i + 64, P.ncode - 1)];
+                const bool in = i < P.ncode, self = in && t.op == OP_ATOM && !test_misses(t, ulo, uhi);
+                const uint64_t m = __ballot(self);
+                if (lane == 0) masks[c] = m, before[c] = live;
+                wave_sync();
+                auto atoms_before = [&](uint32_t p) {
+                    return before[p >> 6] + (uint32_t)__popcll(masks[p >> 6] & ((1ull << (p & 63)) - 1));
+                };
+                uint32_t step = STEP_SKIP;
+                if (in && (live || m)) {
+                    const uint32_t at = atoms_before(t.mid);
+                    const bool right = live + (uint32_t)__popcll(m & ((1ull << lane) - 1)) > at;
+                    const bool left = at > atoms_before(t.start);
+                    step = plan_step_of(t, self, left, right);
+                }
+                live += (uint32_t)__popcll(m);
+                const uint64_t listed = __ballot(step != STEP_SKIP);
+                if (step != STEP_SKIP)
+                    ring[(tail + (uint32_t)__popcll(listed & ((1ull << lane) - 1))) & (PLAN_RING - 1)] = i | (step << 16);
+                tail += (uint32_t)__popcll(listed);
+                const uint32_t least = c + 1 < nb ? PLAN_CHUNK : 1;
+                while (tail - head >= least) {
+                    const uint32_t cnt = min(tail - head, (uint32_t)PLAN_CHUNK);
+                    wave_sync();
+                    uint4 q[PLAN_CHUNK / 8];  // 8 records a load
+                    for (int j = 0; j < PLAN_CHUNK / 8; j++) {
+                        const uint32_t e = min((uint32_t)(j * 8 + (lane >> 3)), cnt - 1);
+                        q[j] = ((const uint4 *)(nodes + (ring[(head + e) & (PLAN_RING - 1)] & 0xffffu)))[lane & 7];
+                    }
+                    for (int j = 0; j < PLAN_CHUNK / 8; j++) ((uint4 *)recs)[j * 64 + lane] = q[j];
+                    wave_sync();
+                    for (uint32_t e = 0; e < cnt; e++) {
+                        const uint32_t st = MC3D_UNIFORM(ring[(head + e) & (PLAN_RING - 1)]) >> 16;
+                        plan_step(st, fetch_node((const PlanNode *)recs, e), S, sp, lo, hi, o, ocap, n, over);
+                    }
+                    head += cnt;
+                    wave_sync();
+                }
+            }
+            if (tail == 0) S[0] = scalar_ptr(nodes)[P.ncode - 1].cfalse ? TAG_TRUE : TAG_FALSE;
         } else {
             auto miss = [&](const PlanNode &t) { return __ballot(valid && !node_misses(t, lo, hi)) == 0; };
             plan_fold_nodes(scalar_ptr(P.plan), P.ncode, S, lo, hi, o, ocap, n, over, miss);

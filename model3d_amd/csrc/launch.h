@@ -44,7 +44,7 @@ struct Pipe {
     uint32_t cap = 0;
     bool cull = false, bm = false, stats = false;
     int mode = 0, rows_per_walk = 1, wpb = 4;
-    size_t plan_lds = 0;  // dynamic LDS of the plan (its stacks, the staged program)
+    uint32_t plan_blocks = 0;  // 64-node blocks of the longest program that the plan lists
     uint32_t plan_gsz = 64;  // bricks per plan wave
     bool plan_tile = false;  // plan waves take compact tiles of bricks (one solid)
     bool scan_one_pass = false;  // classify scans its counts itself (at most SCAN_ONE_PASS blocks)

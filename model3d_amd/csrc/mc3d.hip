@@ -677,16 +677,12 @@ int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> 
     return MC3D_OK;
 }
 
-// Bytes of LDS the plan needs to stage a program: instructions, their atom
-// boxes and the float64 params.
-size_t plan_stage_bytes(const Program &P) { return PLAN_STACK_BYTES + P.code.size() * sizeof(PlanNode); }
-constexpr size_t PLAN_STAGE_LIMIT = 64 * 1024;
-
 // The node records of a postfix program for the brick plan (PlanNode): per
 // node its instruction, link, all-false value, box (atoms: their own;
 // operators: the union of their atoms'; constants: empty; a NaN bound makes
 // the union unbounded on that axis) and the params of the "certainly true"
-// tests.  boxes: each atom's box, by pc.
+// tests; behind them, for programs of up to PLAN_LIST_MAX nodes, their
+// PlanTest records.  boxes: each atom's box, by pc.
 void plan_nodes(const Program &P, const std::vector<AtomBox> &boxes, std::vector<PlanNode> &nodes) {
     const size_t n = P.code.size();
     nodes.assign(n, PlanNode{});
@@ -739,6 +735,28 @@ void plan_nodes(const Program &P, const std::vector<AtomBox> &boxes, std::vector
     // each leaf links to the outermost node starting at it (the last in postfix order)
     for (size_t i = 0; i < n; i++)
         if (start[i] != i) nodes[start[i]].link = (uint32_t)i;
+    if (n > PLAN_LIST_MAX) return;
+    nodes.resize(n + (n * sizeof(PlanTest) + sizeof(PlanNode) - 1) / sizeof(PlanNode));
+    PlanTest *tests = (PlanTest *)(nodes.data() + n);
+    auto below = [](double x) { const float f = (float)x; return f > x ? nextafterf(f, -INFINITY) : f; };
+    auto above = [](double x) { const float f = (float)x; return f < x ? nextafterf(f, INFINITY) : f; };
+    for (size_t i = 0; i < n; i++) {
+        PlanTest &t = tests[i];
+        const uint32_t op = insn_op(nodes[i].x);
+        t.op = (uint8_t)op;
+        t.start = (uint16_t)start[i];
+        if (op == OP_ATOM) {
+            for (int k = 0; k < 3; k++) t.lo[k] = below(nodes[i].lo[k]), t.hi[k] = above(nodes[i].hi[k]);
+            t.mid = (uint16_t)i;
+        } else if (op == OP_TRUE || op == OP_FALSE) {
+            t.mid = (uint16_t)i;
+        } else if (op == OP_NOT) {
+            t.mid = t.start;  // all of its code is its right operand's
+        } else {
+            t.mid = (uint16_t)start[i - 1];
+            t.left_cfalse = (uint8_t)nodes[t.mid - 1].cfalse, t.right_cfalse = (uint8_t)nodes[i - 1].cfalse;
+        }
+    }
 }
 
 // Where a call's pieces sit in the program blob (offsets), and the blob's
@@ -800,7 +818,7 @@ void layout_upload(const std::vector<Job> &jobs, uint64_t nwords_all, uint64_t n
     U.nodes.resize(n);
     for (size_t s = 0; s < n; s++) {
         const Program &P = jobs[s].low->P;
-        if (jobs[s].low->nodes.size() != P.code.size()) job_nodes(P, U.nodes[s]);
+        if (jobs[s].low->nodes.size() < P.code.size()) job_nodes(P, U.nodes[s]);
         const std::vector<PlanNode> &nodes = U.nodes[s].empty() ? jobs[s].low->nodes : U.nodes[s];
         Upload::Off &po = U.po[s];
         po.code = place(P.code.size() * sizeof(Insn));
@@ -875,7 +893,7 @@ void fill_upload(std::vector<Job> &jobs, uint64_t nwords_all, uint64_t nbricks_a
         sg.brick0 = j.brick0, sg.nbricks = j.nbricks;
         sg.pos0 = j.pos0;
         sg.iters = j.iters;
-        sg.stage = j.cap && plan_stage_bytes(P) <= PLAN_STAGE_LIMIT ? 1 : 0;
+        sg.listed = j.cap && P.code.size() <= PLAN_LIST_MAX ? 1 : 0;
     };
     if (n >= 16) HostPool::get().run(n, fill);
     else
@@ -1009,7 +1027,7 @@ struct Call {
     int stack = 1;          // boolean stack entries of the call's programs
     bool bm = false;        // the scan takes the words in brick-major order (one culled solid)
     uint64_t nscan = 0;     // scan positions: words, or brick-major positions
-    size_t plan_lds = 0;
+    uint32_t plan_blocks = 0;
 };
 
 // The call's sizes; places every job's words and bricks.
@@ -1066,12 +1084,10 @@ int plan_call(std::vector<Job> &jobs, const mc3d_options &o, Call &c) {
         c.rows = c.rows && j.low->rows && j.scale.eta < 0.01 && std::isfinite(j.scale.inv_h);
         c.stack = std::max(c.stack, j.low->P.max_stack);
     }
-    c.plan_lds = PLAN_STACK_BYTES;
     if (c.cull)
-        for (const Job &j : jobs) {
-            const size_t lds = plan_stage_bytes(j.low->P);
-            if (lds <= PLAN_STAGE_LIMIT) c.plan_lds = std::max(c.plan_lds, lds);
-        }
+        for (const Job &j : jobs)
+            if (j.low->P.code.size() <= PLAN_LIST_MAX)
+                c.plan_blocks = std::max(c.plan_blocks, (uint32_t)(j.low->P.code.size() + 63) / 64);
     return MC3D_OK;
 }
 
@@ -1133,13 +1149,16 @@ Pipe make_pipe(const Call &c, const Upload &U) {
     p.wpb = c.wpb;
     p.rows = c.rows;
     p.stack = c.stack;
-    p.plan_lds = c.plan_lds;
-    // Launch shapes measured on MI355X: a single solid's plan waves take
-    // compact tiles, 16 bricks for programs that stage in LDS and 64 for the
-    // large ones walked through scalar loads (csg64 39.6 -> 37.4 us, the
-    // 512-primitive tree 183 -> 160 us); emit gets a block per 512 words.
+    p.plan_blocks = c.plan_blocks;
+    // Launch shapes measured on MI355X.  A plan wave folds up to 64 bricks in
+    // one walk over what meets any of them.  A single solid's waves take
+    // compact tiles: 64 bricks where that still makes 4 waves a CU (70k
+    // bricks: 20.5 us, with 32 bricks 26.4; 1M bricks: 143 us, 154), else 32
+    // (56k: 34.2 us, with 64 bricks 35.4; 2.5k: 10.0 and 11.7).  Of several
+    // solids, 16 consecutive bricks: a longer run's box meets more (32 solids:
+    // 98.6 us, with 64 bricks 113).
     p.plan_tile = true;
-    p.plan_gsz = c.plan_lds > PLAN_STACK_BYTES ? 16 : 64;
+    p.plan_gsz = c.nsegs > 1 ? 16 : (c.nbricks >= 64u * 1024 ? 64 : 32);
     p.emit_div = 512;
     p.scan_one_pass = classify_blocks(c) <= SCAN_ONE_PASS;
     return p;
@@ -2701,15 +2720,39 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
                         if (!node_misses(t, lo[k], hi[k])) return false;
                     return true;
                 };
+                float ulo[3], uhi[3];  // the group's box
+                for (int a = 0; a < 3; a++) {
+                    double l = lo[0][a], h = hi[0][a];
+                    for (int k = 1; k < NB; k++) l = std::min(l, lo[k][a]), h = std::max(h, hi[k][a]);
+                    ulo[a] = nextafterf((float)l, -INFINITY), uhi[a] = nextafterf((float)h, INFINITY);
+                }
+                const PlanTest *tests = (const PlanTest *)(nodes.data() + ncode);
+                std::vector<uint32_t> met(ncode + 1, 0), steps(ncode);  // atoms before a node that meet the box
+                for (uint32_t i = 0; i < ncode; i++) {
+                    const PlanTest &t = tests[i];
+                    const bool self = t.op == OP_ATOM && !test_misses(t, ulo, uhi);
+                    met[i + 1] = met[i] + self;
+                    steps[i] = plan_step_of(t, self, met[t.mid] > met[t.start], met[i] > met[t.mid]);
+                }
                 for (int k = 0; k < NB; k++) {
                     const uint32_t cap = (group + k) % 4 == 0 ? (uint32_t)(next() % 4) : 64u;
                     uint32_t S1[PLAN_STACK], S2[PLAN_STACK];
                     Insn o1[64], o2[64];
                     uint32_t n1 = 0, n2 = 0;
                     bool over1 = false, over2 = false;
-                    plan_fold(P.code.data(), boxes.data(), P.f64.data(), ncode, S1, lo[k], hi[k], o1, cap, n1, over1);
-                    plan_fold_nodes(nodes.data(), ncode, S2, lo[k], hi[k], o2, cap, n2, over2, all_miss);
+                    plan_fold(P.code.data(), boxes.data(), P.f64.data(), ncode, (uint32_t *)S1, lo[k], hi[k], o1, cap, n1, over1);
+                    plan_fold_nodes(nodes.data(), ncode, (uint32_t *)S2, lo[k], hi[k], o2, cap, n2, over2, all_miss);
                     bool same = S1[0] == S2[0] && n1 == n2 && over1 == over2;
+                    for (uint32_t i = 0; same && i < std::min(n1, cap); i++)
+                        same = o1[i].x == o2[i].x && o1[i].y == o2[i].y;
+                    // the nodes that say for themselves how they are walked
+                    S2[0] = nodes[ncode - 1].cfalse ? TAG_TRUE : TAG_FALSE;
+                    n2 = 0, over2 = false;
+                    int sp = 0;
+                    for (uint32_t i = 0; i < ncode; i++)
+                        if (steps[i] != STEP_SKIP)
+                            plan_step(steps[i], nodes[i], (uint32_t *)S2, sp, lo[k], hi[k], o2, cap, n2, over2);
+                    same = same && S1[0] == S2[0] && n1 == n2 && over1 == over2;
                     for (uint32_t i = 0; same && i < std::min(n1, cap); i++)
                         same = o1[i].x == o2[i].x && o1[i].y == o2[i].y;
                     nchecked++;

@@ -82,6 +82,19 @@ struct PlanNode {
 };
 static_assert(sizeof(PlanNode) == 128, "a plan node is one 128-byte fetch");
 
+// What the plan needs of a node to tell whether a group of bricks has to walk
+// it (plan_step_of): an atom's box, rounded outwards; where the node's code
+// and its right operand's code start; its operator and its operands' values
+// when all their atoms are false.  They follow the node records of a program
+// of at most PLAN_LIST_MAX nodes.
+struct PlanTest {
+    float lo[3], hi[3];
+    uint16_t start, mid;
+    uint8_t op, left_cfalse, right_cfalse, pad;
+};
+static_assert(sizeof(PlanTest) == 32, "a plan test is two 16-byte loads");
+constexpr uint32_t PLAN_LIST_MAX = 16384;
+
 // Conservative world-space AABB of where an atom can be true (used only to
 // cull atoms that are certainly false in a brick; never changes a result).
 struct AtomBox {

@@ -87,7 +87,7 @@ struct Seg {
     uint64_t brick0, nbricks;  // global bricks; brick0 % 128 == 0
     uint64_t pos0;             // first scan position (brick-major calls), else word0; pos0 % 64 == 0
     int32_t iters;
-    int32_t stage;  // the plan may stage this segment's program in LDS
+    int32_t listed;  // the program's plan tests follow its nodes
 };
 
 // Per-solid results, copied back with the control block.
@@ -100,10 +100,18 @@ struct SegOut {
 constexpr int SEG_WORD_SHIFT = 6;   // segment table entry per 64 words
 constexpr int SEG_BRICK_SHIFT = 7;  // and per 128 bricks
 
-// The brick plan: threads per block and the per-thread fold stack.
+// The brick plan: threads per block, the most entries of a fold's stack, node
+// records a wave holds in LDS at a time and its list of nodes to walk (a ring:
+// up to PLAN_CHUNK - 1 waiting and 64 new ones).
 constexpr int PLAN_BLOCK = 128;
 constexpr int PLAN_STACK = 33;
-constexpr size_t PLAN_STACK_BYTES = PLAN_BLOCK * PLAN_STACK * sizeof(uint32_t);
+constexpr int PLAN_CHUNK = 32;
+constexpr int PLAN_RING = 128;
+// A wave's LDS: node records, ring, per 64 nodes of the longest program a mask
+// and a count, the lanes' stacks.
+inline size_t plan_wave_bytes(uint32_t blocks64, uint32_t stack) {
+    return (PLAN_CHUNK * 128 + PLAN_RING * 4 + (size_t)blocks64 * 12 + (size_t)stack * 256 + 15) / 16 * 16;
+}
 
 // classify and the scan of its counts
 constexpr int SCAN_BLOCK = 256;

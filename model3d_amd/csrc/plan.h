@@ -7,13 +7,15 @@
 // expression whose code starts at output position n}; atoms whose
 // conservative box misses the brick are false, boxes, bounds checks and
 // spheres that contain it are true, and the operators simplify constants
-// away.  plan_fold walks every instruction; plan_fold_nodes walks the same
-// program as node records (PlanNode, one fetch per step) and jumps over
-// subtrees whose atoms' union box misses the brick (on the device: every
-// brick of the wave), pushing the constant that subtree has when all its
-// atoms are false -- which is exactly what plan_fold computes for it, having
-// emitted nothing for it -- so both produce the same folded code, the same
-// root and the same overflow flag.
+// away.  plan_fold walks every instruction.  A group of bricks (on the device:
+// a wave's) leaves most of them out: where no atom of a subtree meets the
+// group's box, the subtree has the constant it has when all its atoms are
+// false -- exactly what plan_fold computes for it, having emitted nothing for
+// it.  plan_step_of says for each node, from the atoms that do meet the box,
+// whether it is walked and how, independently of the other nodes;
+// plan_fold_nodes, for programs too long for that, finds the subtrees on its
+// way.  All three produce the same folded code, the same root and the same
+// overflow flag.
 #pragma once
 
 #include <math.h>
@@ -62,8 +64,8 @@ MC3D_HD inline int classify_atom(F64P f64, BoxP boxes, uint32_t pc, Insn in, con
 constexpr uint32_t TAG_EXPR = 0u, TAG_FALSE = 1u << 30, TAG_TRUE = 2u << 30, TAG_MASK = 3u << 30;
 
 // One instruction of the fold (S: the stack, sp its depth).
-template <class BoxP, class F64P>
-MC3D_HD inline void fold_step(BoxP boxes, F64P f64, uint32_t pc, Insn in, uint32_t *S, int &sp, const double *lo,
+template <class BoxP, class F64P, class Stack>
+MC3D_HD inline void fold_step(BoxP boxes, F64P f64, uint32_t pc, Insn in, Stack S, int &sp, const double *lo,
                               const double *hi, Insn *o, uint32_t cap, uint32_t &n, bool &over) {
     const uint32_t op = insn_op(in.x);
     if (op == OP_ATOM) {
@@ -128,8 +130,8 @@ MC3D_HD inline void fold_step(BoxP boxes, F64P f64, uint32_t pc, Insn in, uint32
 // Folds the whole program against one brick's box (lo, hi), instruction by
 // instruction; the folded code goes to o[0, cap) (`over` if it needs more),
 // the root's tag to S[0].
-template <class CodeP, class BoxP, class F64P>
-MC3D_HD inline void plan_fold(CodeP code, BoxP boxes, F64P f64, uint32_t ncode, uint32_t *S, const double *lo,
+template <class CodeP, class BoxP, class F64P, class Stack>
+MC3D_HD inline void plan_fold(CodeP code, BoxP boxes, F64P f64, uint32_t ncode, Stack S, const double *lo,
                               const double *hi, Insn *o, uint32_t cap, uint32_t &n, bool &over) {
     int sp = 0;
     for (uint32_t pc = 0; pc < ncode; ++pc)
@@ -171,6 +173,76 @@ MC3D_HD inline int classify_node(const PlanNode &nd, const double *lo, const dou
     return 2;
 }
 
+// One instruction of the fold from its node record.
+template <class Stack>
+MC3D_HD inline void fold_node(const PlanNode &cur, Stack S, int &sp, const double *lo, const double *hi, Insn *o,
+                              uint32_t cap, uint32_t &n, bool &over) {
+    const Insn in{cur.x, cur.y};
+    if (insn_op(cur.x) == OP_ATOM) {
+        const int c = classify_node(cur, lo, hi);
+        if (c == 2) {
+            if (n < cap) o[n] = in;
+            else over = true;
+            S[sp++] = TAG_EXPR | n;
+            n++;
+        } else {
+            S[sp++] = c ? TAG_TRUE : TAG_FALSE;
+        }
+    } else {
+        // not an atom: the operators' rules (no box involved)
+        fold_step((const AtomBox *)nullptr, (const double *)nullptr, 0, in, S, sp, lo, hi, o, cap, n, over);
+    }
+}
+
+// How a group of bricks walks a node.  An operator with one operand whose
+// atoms all miss the group (a constant, never pushed) is the other operand,
+// or its negation, or a constant.
+constexpr uint32_t STEP_SKIP = 0, STEP_FOLD = 1, STEP_FALSE = 2, STEP_TRUE = 3, STEP_NOT = 4;
+
+// self: an atom that meets the group's box; left, right: the operands'
+// subtrees hold such an atom.
+MC3D_HD inline uint32_t plan_step_of(const PlanTest &t, bool self, bool left, bool right) {
+    const uint32_t op = t.op;
+    if (op == OP_ATOM) return self ? STEP_FOLD : STEP_SKIP;
+    if (op == OP_TRUE || op == OP_FALSE) return STEP_SKIP;
+    if (op == OP_NOT) return right ? STEP_FOLD : STEP_SKIP;
+    if (left == right) return left ? STEP_FOLD : STEP_SKIP;
+    const bool c = left ? t.right_cfalse : t.left_cfalse;
+    if (op == OP_OR) return c ? STEP_TRUE : STEP_SKIP;
+    if (op == OP_AND) return c ? STEP_SKIP : STEP_FALSE;
+    // a & !b (OP_ANDNOT), !a & b: the constant is the negated operand, or the other
+    if ((op == OP_ANDNOT) == left) return c ? STEP_FALSE : STEP_SKIP;
+    return c ? STEP_NOT : STEP_FALSE;
+}
+
+// The node walked: fold_step's rules with the constant operand in place.
+template <class Stack>
+MC3D_HD inline void plan_step(uint32_t step, const PlanNode &cur, Stack S, int &sp, const double *lo, const double *hi,
+                              Insn *o, uint32_t cap, uint32_t &n, bool &over) {
+    if (step == STEP_FOLD) {
+        fold_node(cur, S, sp, lo, hi, o, cap, n, over);
+        return;
+    }
+    const uint32_t v = S[sp - 1];
+    const bool expr = (v & TAG_MASK) == TAG_EXPR;
+    if (step == STEP_NOT) {
+        if (v == TAG_TRUE) S[sp - 1] = TAG_FALSE;
+        else if (v == TAG_FALSE) S[sp - 1] = TAG_TRUE;
+        else {
+            if (n < cap) o[n] = Insn{OP_NOT, 0};
+            else over = true;
+            n++;
+        }
+        return;
+    }
+    if (expr) n = v & ~TAG_MASK;
+    S[sp - 1] = step == STEP_TRUE ? TAG_TRUE : TAG_FALSE;
+}
+
+MC3D_HD inline bool test_misses(const PlanTest &t, const float *lo, const float *hi) {
+    return hi[0] < t.lo[0] || lo[0] > t.hi[0] || hi[1] < t.lo[1] || lo[1] > t.hi[1] || hi[2] < t.lo[2] || lo[2] > t.hi[2];
+}
+
 // A node fetched whole (one 128-byte read: LDS broadcast, or scalar loads
 // through a constant-address-space pointer), its instruction and link made
 // wave-uniform.
@@ -192,8 +264,8 @@ MC3D_HD inline PlanNode fetch_node(NodeP nodes, uint32_t i) {
 // the walk stays the same for all lanes).  Everything else is fold_step's
 // rule on the node's instruction, box and params, so the folded code, the
 // root and the overflow flag are plan_fold's.
-template <class NodeP, class AllMiss>
-MC3D_HD inline void plan_fold_nodes(NodeP nodes, uint32_t ncode, uint32_t *S, const double *lo, const double *hi,
+template <class NodeP, class Stack, class AllMiss>
+MC3D_HD inline void plan_fold_nodes(NodeP nodes, uint32_t ncode, Stack S, const double *lo, const double *hi,
                                     Insn *o, uint32_t cap, uint32_t &n, bool &over, AllMiss &&all_miss) {
     int sp = 0;
     uint32_t pc = 0;
@@ -215,21 +287,7 @@ MC3D_HD inline void plan_fold_nodes(NodeP nodes, uint32_t ncode, uint32_t *S, co
             }
             if (skip) continue;
         }
-        const Insn in{cur.x, cur.y};
-        if (op == OP_ATOM) {
-            const int c = classify_node(cur, lo, hi);
-            if (c == 2) {
-                if (n < cap) o[n] = in;
-                else over = true;
-                S[sp++] = TAG_EXPR | n;
-                n++;
-            } else {
-                S[sp++] = c ? TAG_TRUE : TAG_FALSE;
-            }
-        } else {
-            // not an atom: the operators' rules (no box involved)
-            fold_step((const AtomBox *)nullptr, (const double *)nullptr, pc, in, S, sp, lo, hi, o, cap, n, over);
-        }
+        fold_node(cur, S, sp, lo, hi, o, cap, n, over);
         ++pc;
     }
 }
