@@ -51,6 +51,7 @@ void bisect(const Pipe &p, const Bufs &b, double *verts, double *interior, uint6
 hipError_t launch_bisect(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
                          hipStream_t st) {
     if (p.rows) return launch_bisect_rows(p, b, verts, interior, vcap, st);
+    if (p.ray_rows) return launch_bisect_rays(p, b, verts, interior, vcap, st);
     if (p.mode == 0)
         p.stats ? bisect<0, true>(p, b, verts, interior, vcap, st) : bisect<0, false>(p, b, verts, interior, vcap, st);
     else

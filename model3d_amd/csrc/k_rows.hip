@@ -20,11 +20,6 @@
 namespace mc3d {
 namespace {
 
-__device__ __forceinline__ RowScale row_scale(const Grid &g) {
-    const auto p = scalar_ptr(g.zs + g.nz);
-    return RowScale{p[0], p[1], p[2], p[3]};
-}
-
 // The corners of one word (from x0, in row (y, z)) that a program holds for.
 template <bool UNI, class CodeP, class F64P>
 __device__ __forceinline__ uint64_t word_bits(CodeP code, uint32_t n, F64P f64, const Grid &g, int x0, int y, int z,

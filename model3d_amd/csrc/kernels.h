@@ -61,6 +61,11 @@ __device__ __forceinline__ Seg pick_seg(const Seg *__restrict__ segs, const Seg 
     return s;
 }
 
+__device__ __forceinline__ RowScale row_scale(const Grid &g) {
+    const auto p = scalar_ptr(g.zs + g.nz);
+    return RowScale{p[0], p[1], p[2], p[3]};
+}
+
 __device__ __forceinline__ size_t word_index(const Grid &g, int wx, int y, int z) {
     return ((size_t)z * g.ny + y) * g.W + wx;
 }

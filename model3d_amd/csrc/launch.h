@@ -49,6 +49,7 @@ struct Pipe {
     bool plan_tile = false;  // plan waves take compact tiles of bricks (one solid)
     bool scan_one_pass = false;  // classify scans its counts itself (at most SCAN_ONE_PASS blocks)
     bool rows = false;  // every atom has a row form: corners and bisection decide lines, not points
+    int ray_rows = 0;   // the solid is a collider decided by rows, so many a wave (0: no)
     int stack = 1;      // boolean stack entries of the call's programs
     uint32_t emit_div = 1024;  // emit blocks: occupancy words / emit_div, in [512, 4096]
 };
@@ -66,8 +67,10 @@ hipError_t launch_corners_ms<1, false>(const Pipe &p, const Bufs &b, hipStream_t
 template <>
 hipError_t launch_corners_ms<1, true>(const Pipe &p, const Bufs &b, hipStream_t st);
 hipError_t launch_rows(const Pipe &p, const Bufs &b, hipStream_t st);
+hipError_t launch_ray_rows(const Pipe &p, const Bufs &b, hipStream_t st);
 inline hipError_t launch_corners(const Pipe &p, const Bufs &b, hipStream_t st) {
     if (p.rows) return launch_rows(p, b, st);
+    if (p.ray_rows) return launch_ray_rows(p, b, st);
     if (p.mode == 0) return p.stats ? launch_corners_ms<0, true>(p, b, st) : launch_corners_ms<0, false>(p, b, st);
     return p.stats ? launch_corners_ms<1, true>(p, b, st) : launch_corners_ms<1, false>(p, b, st);
 }
@@ -77,8 +80,18 @@ hipError_t launch_classify(const Pipe &p, const Bufs &b, hipStream_t st);
 // the scan of classify's counts, the list of emitting words and (calls of
 // several solids) each solid's output ranges
 hipError_t launch_scan(const Pipe &p, const Bufs &b, hipStream_t st);
+// A collider's triangles by planes (k_rays.hip): n ray-grid records into forms
+// and extents, at[b] = the entries of bin b, *bad if one is too large for it;
+// start and *total from at (left as the fill's cursors); the lists.
+hipError_t launch_ray_forms(const double *rec, uint32_t n, const RayPlanes &R, double *forms, double *extent, uint32_t *at,
+                            uint32_t *bad, hipStream_t st);
+hipError_t launch_ray_scan(uint32_t *at, uint32_t bins, uint32_t *start, unsigned long long *total, hipStream_t st);
+hipError_t launch_ray_fill(const double *extent, uint32_t n, const RayPlanes &R, uint32_t *at, uint32_t *list,
+                           hipStream_t st);
 hipError_t launch_emit(const Pipe &p, const Bufs &b, uint32_t *tris, uint64_t vcap, uint64_t tcap, hipStream_t st);
 hipError_t launch_bisect_rows(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
+                              hipStream_t st);
+hipError_t launch_bisect_rays(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
                               hipStream_t st);
 hipError_t launch_bisect(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap,
                          hipStream_t st);

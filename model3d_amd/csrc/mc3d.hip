@@ -411,7 +411,7 @@ struct MeshBuffers {
 struct ColliderCache {
     std::shared_ptr<const ColliderData> keep;
     double R = 0;  // radius of its sphere queries (0: none)
-    DevBuf rec, start, tris, srec, sstart, stris;
+    DevBuf rec, start, tris, srec, sstart, stris, forms, pstart, plist;
     DevCollider dev{};
 };
 
@@ -614,6 +614,52 @@ int prepare_job(Job &j, const mc3d_options &o, bool check = true) {
     return layout_job(j, o, check);
 }
 
+// The collider's triangles by planes, for rows of corners (k_rays.hip); none
+// where triangles are too large or lists would be longer than 64 entries a
+// triangle.
+int collider_planes(mc3d_ctx *ctx, const ColliderData &cd, ColliderCache &c) {
+    DevCollider &d = c.dev;
+    const size_t n = cd.ray_grid().rec.size() / RAY_REC;
+    if (n == 0 || n >= (1u << 28)) return MC3D_OK;
+    RayPlanes P{};
+    const double dy = 0.10494477243214506, dz = 0.43558938446126527, len = sqrt(dy * dy + dz * dz);
+    P.ny = -dz / len, P.nz = dy / len;  // x axis times the ray
+    double lo = 0, hi = 0, mag = 0;
+    for (int a = 0; a < 3; a++) mag = std::max({mag, fabs(cd.mn[a]), fabs(cd.mx[a])});
+    for (int a = 1; a < 3; a++) {
+        const double k = a == 1 ? P.ny : P.nz;
+        lo += std::min(k * cd.mn[a], k * cd.mx[a]), hi += std::max(k * cd.mn[a], k * cd.mx[a]);
+    }
+    if (!(mag < 1e100) || !(hi > lo)) return MC3D_OK;
+    // A bin about as wide as a triangle of an even mesh is long.
+    P.bins = (int)std::min((double)RAY_BINS, std::max(8.0, 1.5 * sqrt((double)n)));
+    P.s0 = lo, P.width = (hi - lo) / P.bins, P.inv = 1 / P.width;
+    if (!std::isfinite(P.inv)) return MC3D_OK;
+    DevBuf extent, at, head;
+    int rc;
+    if ((rc = extent.ensure(n * 16)) || (rc = at.ensure((size_t)P.bins * 4 + 16)) || (rc = head.ensure(32)) ||
+        (rc = c.forms.ensure(n * RAY_FORM * sizeof(double))) || (rc = c.pstart.ensure((size_t)P.bins * 4 + 16)))
+        return rc;
+    hipStream_t st = ctx->stream;
+    HIP_TRY(launch_ray_forms(d.rec, (uint32_t)n, P, c.forms.as<double>(), extent.as<double>(), at.as<uint32_t>(),
+                             head.as<uint32_t>(), st));
+    HIP_TRY(launch_ray_scan(at.as<uint32_t>(), (uint32_t)P.bins, c.pstart.as<uint32_t>(),
+                            (unsigned long long *)(head.as<char>() + 16), st));
+    uint64_t got[4];
+    HIP_TRY(hipStreamSynchronize(st));
+    HIP_TRY(hipMemcpy(got, head.p, 32, hipMemcpyDeviceToHost));
+    if ((uint32_t)got[0] || got[2] > 64 * n || got[2] >= (1ull << 32)) {
+        return MC3D_OK;
+    }
+    if ((rc = c.plist.ensure(got[2] * 4 + 16))) return rc;
+    HIP_TRY(launch_ray_fill(extent.as<double>(), (uint32_t)n, P, at.as<uint32_t>(), c.plist.as<uint32_t>(), st));
+    HIP_TRY(hipStreamSynchronize(st));
+    d.forms = c.forms.as<double>();
+    d.pstart = c.pstart.as<uint32_t>(), d.plist = c.plist.as<uint32_t>();
+    d.pentries = got[2], d.mag = mag, d.planes = P;
+    return MC3D_OK;
+}
+
 // The device copy of a collider's ray grid and, for sphere queries of
 // radius R, its sphere grid (uploaded once per context).
 int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> &cd, double R, DevCollider &out,
@@ -649,6 +695,8 @@ int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> 
     d.u0 = G.u0, d.v0 = G.v0, d.inv_cell = G.inv_cell, d.nu = G.nu, d.nv = G.nv;
     d.srec = nullptr, d.scell_start = d.scell_tris = nullptr;
     d.so[0] = d.so[1] = d.so[2] = 0, d.sinv = 1, d.sn[0] = d.sn[1] = d.sn[2] = 0, d.pad = 0;
+    d.forms = nullptr, d.pstart = d.plist = nullptr, d.pentries = 0, d.mag = 0, d.planes = RayPlanes{};
+    if (R == 0 && (rc = collider_planes(ctx, *cd, *c))) return rc;
     if (R > 0) {
         const SphereGrid &S = cd->sphere_grid(R);
         if ((rc = c->srec.ensure(S.rec.size() * sizeof(double) + 8)) ||
@@ -782,6 +830,9 @@ struct Upload {
     const double *conj = nullptr;  // job 0's MarchingCubesConj inverse chain (records of 10 doubles)
     uint32_t conj_nops = 0;
     uint32_t epoch = 0;  // this call's scan epoch (written into the control block)
+    bool collider_only = false;  // job 0's program is one collider atom, without a frame, an inset or a radius
+    RowScale scale{};            // job 0's
+    uint32_t row_corners = 0;
 };
 
 // The blob's layout: the control block, the per-solid results, the
@@ -915,6 +966,14 @@ void fill_upload(std::vector<Job> &jobs, uint64_t nwords_all, uint64_t nbricks_a
 // The colliders of every job on this context's device.
 int upload_colliders(mc3d_ctx *ctx, const std::vector<Job> &jobs, Upload &U) {
     const size_t n = jobs.size();
+    {
+        const Program &P = jobs[0].low->P;
+        const Insn in = P.code[0];
+        U.collider_only = P.code.size() == 1 && insn_op(in.x) == OP_ATOM && insn_kind(in.x) == A_COLLIDER &&
+                          insn_frame(in.x) == 0 && P.f64[in.y + 7] == 0 && P.f64[in.y + 8] == 0;
+        U.scale = jobs[0].scale;
+        U.row_corners = (uint32_t)jobs[0].g.nx;
+    }
     size_t ncol = 0;
     for (const Job &j : jobs) ncol += j.low->P.colliders.size();
     U.cols.assign(n, {});
@@ -1126,6 +1185,25 @@ int ctx_buffers(mc3d_ctx *ctx, const Call &c, Bufs &b, uint32_t &epoch) {
     return MC3D_OK;
 }
 
+// Rows that a wave takes where a call's solid is one collider without an inset
+// or a frame; 0: its corners are looked up point by point.
+int collider_rows(const Upload &U) {
+    if (U.cols.size() != 1 || U.cols[0].size() != 1 || !U.cols[0][0].forms || !U.collider_only) return 0;
+    const RayPlanes &P = U.cols[0][0].planes;
+    const RowScale &rs = U.scale;
+    if (!(rs.eta < 0.01) || !std::isfinite(rs.inv_h)) return 0;
+    // A wave reads its bin's whole list for a row, and an edge's halvings read
+    // the lists of every cell that it crosses: rows where the grid is not much
+    // coarser than the mesh.  Measured (a mesh made at spacing 0.02 / 0.05, whole
+    // calls by points and by rows): edges of about 42 cells 124 and 213 us, 17
+    // cells 133 and 149 us, 12 cells 334 and 207 us, 8 cells 262 and 124 us.
+    const DevCollider &C = U.cols[0][0];
+    if (!(rs.h * C.inv_cell < 14) || C.pentries > 256ull * P.bins * U.row_corners) return 0;
+    for (int rows = RAY_ROWS; rows > 1; rows /= 2)
+        if ((rows - 1) * P.nz * rs.h < 0.999 * P.width) return rows;
+    return 1;
+}
+
 Pipe make_pipe(const Call &c, const Upload &U) {
     Pipe p;
     memset((void *)&p, 0, sizeof p);  // padding included: graph keys compare the bytes
@@ -1148,6 +1226,7 @@ Pipe make_pipe(const Call &c, const Upload &U) {
     p.rows_per_walk = c.rows_per_walk;
     p.wpb = c.wpb;
     p.rows = c.rows;
+    p.ray_rows = c.nsegs == 1 && !c.stats && !c.host ? collider_rows(U) : 0;
     p.stack = c.stack;
     p.plan_blocks = c.plan_blocks;
     // Launch shapes measured on MI355X.  A plan wave folds up to 64 bricks in

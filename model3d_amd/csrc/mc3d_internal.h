@@ -144,7 +144,21 @@ struct ColliderData {
     const SphereGrid &sphere_grid(double R) const;  // built on first use per radius
 };
 
-// Device view of a RayGrid and (insets, hollow shells) a SphereGrid.
+// For rows of corners (k_rays.hip): the planes through a row (a line in x) and
+// the ray direction, at s = ny y + nz z; the kept triangles binned by their
+// extents in s, each from `width` (a bin's) below its own on, in bins of
+// floor((s - s0) inv).  A triangle's linear forms are RAY_FORM doubles; a wave
+// takes up to RAY_ROWS rows.
+constexpr int RAY_FORM = 16;
+constexpr int RAY_ROWS = 4;
+constexpr int RAY_BINS = 4096;  // at most
+struct RayPlanes {
+    double ny, nz, s0, inv, width;
+    int bins, pad;
+};
+
+// Device view of a RayGrid, (without sphere queries) its triangles by planes,
+// and (insets, hollow shells) a SphereGrid.
 struct DevCollider {
     const double *rec;
     const uint32_t *cell_start;
@@ -157,6 +171,11 @@ struct DevCollider {
     const uint32_t *scell_tris;
     double so[3], sinv;
     int sn[3], pad;
+    const double *forms;  // null: no planes
+    const uint32_t *pstart, *plist;
+    uint64_t pentries;  // of all lists
+    double mag;         // largest |coordinate|
+    RayPlanes planes;
 };
 
 struct HostAtom {
