@@ -971,25 +971,26 @@ __device__ __forceinline__ uint64_t vkey(int axis, int x, int y, int z) {
     return (uint64_t)axis | ((uint64_t)x << 2) | ((uint64_t)y << 22) | ((uint64_t)z << 42);
 }
 
-// Occupancy word, crossing masks and vertex base of one (row, word).  The
+// Occupancy word, crossing masks and vertex bases of one (row, word).  The
 // vertices of a word are numbered from its scanned base: its x crossings,
 // then y, then z, each in bit order.
 struct WordInfo {
-    uint64_t bits, cx, cy, cz;
-    uint32_t base, tbase;  // scanned first vertex and first triangle of the word
+    uint64_t c[3];     // its crossings per axis
+    uint32_t base[3];  // the first vertex of each
+    uint32_t d[3];     // its bits and the next word's first 32
 };
 
-// Listed words a wave takes per iteration of emit.
+// Listed words a wave takes at a time, and cubes whose triangles it does.
 constexpr int EMIT_G = 8;
-static_assert(3 * EMIT_G <= 64 && EMIT_G <= 32, "emit's per-group prefixes fit one wave");
+static_assert(3 * EMIT_G <= 64 && EMIT_G % 8 == 0, "a lane per word and axis, eight words a staging pass");
+constexpr int EMIT_CUBES = 64;
 
 // A word of a wave's group, as emit's later steps need it (LDS).
 struct GroupWord {
     uint32_t y, z, x0;  // row, and the x of the word's first corner
     uint32_t si;        // segment
     uint32_t vsolid;    // the solid's first vertex (its triangles index from there)
-    uint32_t zin;       // a plane above the word's: it has cubes
-    uint64_t keep;      // block filter: the word's cubes of accepted blocks
+    uint32_t tbase;     // the word's scanned first triangle
 };
 
 // Position of the r-th set bit of m (r < popcount(m)).
@@ -1005,25 +1006,34 @@ __device__ __forceinline__ int select_bit(uint64_t m, int r) {
     return pos;
 }
 
-// Largest i < n with pre[i] <= j (pre ascending from pre[0] == 0; n <= 64).
-__device__ __forceinline__ int owner(const uint32_t *pre, int n, uint32_t j) {
+// Largest i < n with pre[i] <= j (pre ascending from pre[0] == 0; n <= 2 MAX).
+template <int MAX, class T>
+__device__ __forceinline__ int owner(const T *pre, int n, uint32_t j) {
     int L = 0;
-    for (int step = 32; step; step >>= 1)
+    for (int step = MAX; step; step >>= 1)
         if (L + step < n && pre[L + step] <= j) L += step;
     return L;
 }
 
-// Emit: a wave takes EMIT_G consecutive listed words at a time.  Their
-// vertices and triangles are consecutive in the outputs (the scan numbers
-// them in list order), so the group's work is flattened: the 2 x 2 rows by
-// 2 words around each word are staged in LDS (a lane per word and
-// neighbour), then the group's vertices are spread over the lanes (vertex j
-// of the group: its word, axis and crossing found from per-word prefix
-// counts), then its mixed cubes (a lane per cube, its case from the staged
-// bits), then the corners of its triangles (corner j belongs to triangle
-// j / 3 of the cube whose prefix covers it).  No lane works on a cube
+// Emit: a wave takes EMIT_G consecutive listed words at a time.  Their vertices
+// and triangles are consecutive in the outputs (the scan numbers them in list
+// order), so the group's work is flattened: the 2 x 2 rows by 2 words around
+// each word are staged in LDS (a lane per word and neighbour; the word's mixed
+// cubes folded from its eight lanes), then the group's vertices are spread
+// over the lanes (vertex j of the group: its word, axis and crossing found
+// from the words' bases), then its mixed cubes (a lane per cube, its case from
+// the staged bits), then the triangles of up to EMIT_CUBES of them (a lane
+// finds its triangle's cube by the cubes' prefix).  No lane works on a cube
 // without triangles.  Writes at or beyond the capacities are dropped and
 // flagged (the host grows the buffers and runs this stage again).
+// Bound by vector issue (560 instructions a group of 8 words, 41 of 64 lanes
+// at work: 26 vertices, 28 cubes and 52 triangles of the 512-atom solid at
+// spacing 0.002).  A corner's index is two LDS reads and a popcount, a cube's
+// case two bits of each row by one shift.  16 words a group fill the lanes
+// better (10.2 against 13.5 k instructions a wave) but halve the waves that the
+// LDS holds: 446 us, and 36.6 for the 64-atom solid at 0.005.  Measured, with
+// the masks selected and the case's bits taken one by one before: 475 -> 408 us,
+// 41 -> 35, one slab at 0.003 58 -> 50, 32 solids 80 -> 70.
 template <bool MULTI>
 __global__ __launch_bounds__(256) void k_emit(const Seg *__restrict__ segs, uint32_t nsegs, const Seg seg0,
                                               const uint32_t *__restrict__ word_seg,
@@ -1034,14 +1044,15 @@ __global__ __launch_bounds__(256) void k_emit(const Seg *__restrict__ segs, uint
                                               uint32_t *__restrict__ tris, const uint64_t *__restrict__ keep_all,
                                               uint64_t vcap, uint64_t tcap, bool bm) {
     __shared__ __align__(16) uint8_t tab[256 * 16];
-    __shared__ WordInfo wi_all[4][EMIT_G][8];
-    __shared__ GroupWord gw_all[4][EMIT_G];
-    __shared__ uint64_t mixed_all[4][EMIT_G];
-    __shared__ uint32_t vpre_all[4][3 * EMIT_G];
-    __shared__ uint32_t mpre_all[4][EMIT_G];
-    __shared__ uint32_t s_pre[4][64];
-    __shared__ uint16_t s_cube[4][64];
-    __shared__ uint8_t s_cs[4][64];
+    constexpr int G = EMIT_G;
+    __shared__ WordInfo wi_all[4][G][8];
+    __shared__ GroupWord gw_all[4][G];
+    __shared__ uint64_t mixed_all[4][G];
+    __shared__ uint32_t vpre_all[4][3 * G];
+    __shared__ uint32_t mpre_all[4][G];
+    __shared__ uint16_t s_pre[4][EMIT_CUBES];
+    __shared__ uint16_t s_cube[4][EMIT_CUBES];
+    __shared__ uint8_t s_cs[4][EMIT_CUBES];
     // the listed words' count, loaded beside the table
     const uint32_t nact = (uint32_t)ctl->totals[2];
     // (table: the case table with each edge decoded to axis | dx << 2 |
@@ -1056,15 +1067,17 @@ __global__ __launch_bounds__(256) void k_emit(const Seg *__restrict__ segs, uint
     uint32_t *vpre = vpre_all[wave], *mpre = mpre_all[wave];
     const uint64_t below = lane ? (~0ull >> (64 - lane)) : 0ull;
     bool over = false;
-    const uint32_t kstep = gridDim.x * 4 * EMIT_G;
-    for (uint32_t k0 = (blockIdx.x * 4 + wave) * EMIT_G; k0 < nact; k0 += kstep) {
-        const int ng = (int)min((uint32_t)EMIT_G, nact - k0);  // words in the group
+    const uint32_t kstep = gridDim.x * 4 * G;
+    for (uint32_t k0 = (blockIdx.x * 4 + wave) * G; k0 < nact; k0 += kstep) {
+        const int ng = (int)min((uint32_t)G, nact - k0);  // words in the group
         wave_sync();  // the previous group's LDS reads are done
         // 1. Item 8 g + e stages neighbour e of word g: entry bits 0 next
         //    word, 1 row y+1, 2 row z+1.
-        for (int q = lane; q < 8 * EMIT_G; q += 64) {
+        for (int q0 = 0; q0 < 8 * G; q0 += 64) {
+            const int q = q0 + lane;
             const int g = q >> 3, e = q & 7;
-            WordInfo r{0, 0, 0, 0, 0, 0};
+            WordInfo r{};
+            uint64_t any = 0, all = 0, kw = 0;  // the row's part of the word's mixed cubes
             if (g < ng) {
                 const uint32_t gw = active[k0 + g];
                 const uint32_t si = MULTI ? word_seg[gw >> SEG_WORD_SHIFT] : 0u;
@@ -1099,49 +1112,38 @@ __global__ __launch_bounds__(256) void k_emit(const Seg *__restrict__ segs, uint
                 const uint64_t bz = bits[idx + (hz ? plane : 0u)];
                 const uint2 o = offs[bm ? bm_index(g_, B_, cx, cy, cz) : idx];
                 if (in) {
-                    r.bits = b;
                     // (the top plane, also of a z slab: no z edges)
-                    Masks m{b ^ ((b >> 1) | ((hx ? bn : 0) << 63)), b ^ (hy ? by : 0), hz ? b ^ bz : 0};
+                    const uint64_t next = hx ? bn : 0, up = (b >> 1) | (next << 63);
+                    Masks m{b ^ up, b ^ (hy ? by : 0), hz ? b ^ bz : 0};
                     if (!MULTI && keep_all) keep_masks(g_, keep_all + word0, ex, ey, ez, m);
-                    r.cx = m.cx, r.cy = m.cy, r.cz = m.cz;
-                    r.base = o.x;
-                    r.tbase = o.y;
+                    r.d[0] = (uint32_t)b, r.d[1] = (uint32_t)(b >> 32), r.d[2] = (uint32_t)next;
+                    r.c[0] = m.cx, r.c[1] = m.cy, r.c[2] = m.cz;
+                    r.base[0] = o.x, r.base[1] = o.x + (uint32_t)__popcll(m.cx);
+                    r.base[2] = r.base[1] + (uint32_t)__popcll(m.cy);
+                    any = b | up, all = b & up;
                 }
                 if (e == 0) {
                     const uint32_t vsolid = MULTI ? offs[0].x : 0u;
-                    const uint64_t kw = (!MULTI && keep_all) ? keep_all[word0 + idx] : ~0ull;
-                    gwd[g] = GroupWord{(uint32_t)y, (uint32_t)z, (uint32_t)wx * 64u, si, vsolid,
-                                       z + 1 < g_.nz ? 1u : 0u, kw};
+                    // the word's cubes: none without a plane above; under a
+                    // block filter those of accepted blocks
+                    if (z + 1 < g_.nz) kw = (!MULTI && keep_all) ? keep_all[word0 + idx] : ~0ull;
+                    gwd[g] = GroupWord{(uint32_t)y, (uint32_t)z, (uint32_t)wx * 64u, si, vsolid, o.y};
                 }
             }
             wi[g][e] = r;
+            for (int d = 2; d <= 4; d <<= 1) any |= __shfl_xor(any, d), all &= __shfl_xor(all, d);
+            if (e == 0) mixed[g] = any & ~all & kw;
         }
         wave_sync();
-        const uint32_t vbase = wi[0][0].base, tbase = wi[0][0].tbase;  // the group's first vertex / triangle
-        // 2. Vertex keys.  Lane 3 g + a counts word g's crossings on axis a;
-        //    their exclusive prefix numbers the group's vertices.
-        uint32_t nvg;
-        {
-            uint32_t c = 0;
-            if (lane < 3 * EMIT_G && lane / 3 < ng) {
-                const WordInfo &me = wi[lane / 3][0];
-                const int a = lane % 3;
-                c = (uint32_t)__popcll(a == 0 ? me.cx : (a == 1 ? me.cy : me.cz));
-            }
-            uint32_t inc = c;
-            for (int d = 1; d < 3 * EMIT_G; d <<= 1) {
-                const uint32_t t = __shfl_up(inc, d);
-                if (lane >= d) inc += t;
-            }
-            if (lane < 3 * EMIT_G) vpre[lane] = inc - c;
-            nvg = __shfl(inc, 3 * EMIT_G - 1);
-        }
+        // the group's first vertex and triangle
+        const uint32_t vbase = wi[0][0].base[0], tbase = gwd[0].tbase;
+        // 2. Vertex keys.  Lane 3 g + a: word g's first vertex on axis a.
+        if (lane < 3 * G) vpre[lane] = lane < 3 * ng ? wi[lane / 3][0].base[lane % 3] - vbase : ~0u;
+        const uint32_t nvg = wi[ng - 1][0].base[2] + (uint32_t)__popcll(wi[ng - 1][0].c[2]) - vbase;
         wave_sync();
         for (uint32_t j = lane; j < nvg; j += 64) {
-            const int q = owner(vpre, 3 * EMIT_G, j), g = q / 3, a = q - 3 * g;
-            const WordInfo &me = wi[g][0];
-            const uint64_t m = a == 0 ? me.cx : (a == 1 ? me.cy : me.cz);
-            const int bit = select_bit(m, (int)(j - vpre[q]));
+            const int q = owner<32>(vpre, 3 * G, j), g = q / 3, a = q - 3 * g;
+            const int bit = select_bit(wi[g][0].c[a], (int)(j - vpre[q]));
             const GroupWord gw = gwd[g];
             const uint64_t v = (uint64_t)vbase + j;
             if (v < vcap) {
@@ -1151,51 +1153,43 @@ __global__ __launch_bounds__(256) void k_emit(const Seg *__restrict__ segs, uint
                 over = true;
             }
         }
-        // 3. Each word's mixed cubes (lane g); their prefix numbers the
-        //    group's mixed cubes.
+        // 3. The mixed cubes' prefix over the words numbers the group's.
         uint32_t nmg;
         {
-            uint32_t c = 0;
-            if (lane < ng) {
-                Nbhd h;
-                for (int k = 0; k < 8; k++) h.n[k] = wi[lane][k].bits;
-                h.zin = gwd[lane].zin != 0;
-                const uint64_t m = mixed_cubes(nbhd_corners(h)) & gwd[lane].keep;
-                mixed[lane] = m;
-                c = (uint32_t)__popcll(m);
-            }
+            const uint32_t c = lane < G ? (uint32_t)__popcll(mixed[lane]) : 0u;
             uint32_t inc = c;
-            for (int d = 1; d < EMIT_G; d <<= 1) {
+            for (int d = 1; d < G; d <<= 1) {
                 const uint32_t t = __shfl_up(inc, d);
                 if (lane >= d) inc += t;
             }
-            if (lane < EMIT_G) mpre[lane] = inc - c;
-            nmg = __shfl(inc, EMIT_G - 1);
+            if (lane < G) mpre[lane] = inc - c;
+            nmg = __shfl(inc, G - 1);
         }
         wave_sync();
-        // 4. Triangles, up to 64 mixed cubes at a time.
+        // 4. Triangles, up to EMIT_CUBES mixed cubes at a time.
         uint32_t tdone = 0;
-        for (uint32_t c0 = 0; c0 < nmg; c0 += 64) {
-            const uint32_t j = c0 + lane;
-            int cs = 0, g = 0, i = 0;
-            if (j < nmg) {
-                g = owner(mpre, ng, j);
-                i = select_bit(mixed[g], (int)(j - mpre[g]));
-                for (int dz = 0; dz < 2; dz++)
-                    for (int dy = 0; dy < 2; dy++) {
-                        const int e = 2 * dy + 4 * dz;
-                        const uint64_t b = wi[g][(dy << 1) | (dz << 2)].bits, bn = wi[g][1 | (dy << 1) | (dz << 2)].bits;
-                        cs |= (int)((b >> i) & 1) << e;
-                        cs |= (int)((((b >> 1) | (bn << 63)) >> i) & 1) << (e + 1);
+        for (uint32_t c0 = 0; c0 < nmg; c0 += EMIT_CUBES) {
+            const uint32_t cn = min(nmg - c0, (uint32_t)EMIT_CUBES);
+            uint32_t tw = 0;  // triangles of these cubes
+            for (uint32_t s0 = 0; s0 < cn; s0 += 64) {
+                const uint32_t j = c0 + s0 + lane;
+                int cs = 0, g = 0, i = 0;
+                if (j < nmg) {
+                    g = owner<G / 2>(mpre, ng, j);
+                    i = select_bit(mixed[g], (int)(j - mpre[g]));
+                    for (int r = 0; r < 4; r++) {  // row r: corners i and i + 1
+                        const uint32_t *d = wi[g][2 * r].d + (i >> 5);
+                        cs |= (int)(__builtin_amdgcn_alignbit(d[1], d[0], (uint32_t)i & 31u) & 3u) << (2 * r);
                     }
+                }
+                const int nt = tab[16 * cs];
+                const uint32_t pre = tw + __popcll(__ballot(nt & 1) & below) + 2 * __popcll(__ballot(nt & 2) & below) +
+                                     4 * __popcll(__ballot(nt & 4) & below);
+                s_pre[wave][s0 + lane] = (uint16_t)pre;
+                s_cs[wave][s0 + lane] = (uint8_t)cs;
+                s_cube[wave][s0 + lane] = (uint16_t)((g << 6) | i);
+                tw = __shfl(pre + nt, 63);
             }
-            const int nt = tab[16 * cs];
-            const uint32_t pre = __popcll(__ballot(nt & 1) & below) + 2 * __popcll(__ballot(nt & 2) & below) +
-                                 4 * __popcll(__ballot(nt & 4) & below);
-            const uint32_t tw = __shfl(pre + nt, 63);  // triangles of these cubes
-            s_pre[wave][lane] = pre;
-            s_cs[wave][lane] = (uint8_t)cs;
-            s_cube[wave][lane] = (uint16_t)((g << 6) | i);
             wave_sync();
             const uint64_t t0 = (uint64_t)tbase + tdone;
             if (t0 + tw > tcap) {
@@ -1204,23 +1198,17 @@ __global__ __launch_bounds__(256) void k_emit(const Seg *__restrict__ segs, uint
                 // triangle ti belongs to the cube whose prefix covers it (a
                 // lane per triangle: one search for its three corners)
                 for (uint32_t ti = lane; ti < tw; ti += 64) {
-                    const int L = owner(s_pre[wave], 64, ti);
+                    const int L = owner<EMIT_CUBES / 2>(s_pre[wave], (int)cn, ti);
                     const int c = s_cs[wave][L], gi = s_cube[wave][L], gg = gi >> 6, ii = gi & 63;
-                    const int k0 = 3 * (int)(ti - s_pre[wave][L]);
-                    const uint32_t vsolid = gwd[gg].vsolid;
+                    const uint8_t *te = tab + 16 * c + 1 + 3 * (int)(ti - s_pre[wave][L]);
+                    const uint32_t vsolid = MULTI ? gwd[gg].vsolid : 0u;
                     uint32_t corner[3];
                     for (int ec = 0; ec < 3; ec++) {
-                        const int e = tab[16 * c + 1 + k0 + ec];
-                        const int axis = e & 3, ddx = (e >> 2) & 1, ddy = (e >> 3) & 1, ddz = (e >> 4) & 1;
-                        const int ex = ii + ddx;  // x within the word (64: the next word's first)
-                        const WordInfo &o = wi[gg][(ex >> 6) | (ddy << 1) | (ddz << 2)];
-                        const int bb = ex & 63;
-                        const uint64_t bl = bb ? (~0ull >> (64 - bb)) : 0ull;
-                        // vertices of the word before this edge: its x crossings, then y, then z
-                        const uint64_t m = axis == 0 ? o.cx : (axis == 1 ? o.cy : o.cz);
-                        const uint32_t idx = o.base + (axis > 0 ? (uint32_t)__popcll(o.cx) : 0u) +
-                                             (axis > 1 ? (uint32_t)__popcll(o.cy) : 0u) + (uint32_t)__popcll(m & bl);
-                        corner[ec] = idx - vsolid;
+                        const int e = te[ec], axis = e & 3;
+                        const int ex = ii + ((e >> 2) & 1);  // x within the word (64: the next word's first)
+                        const WordInfo &o = wi[gg][((e >> 2) & 6) | (ex >> 6)];
+                        // vertices of the word before this edge
+                        corner[ec] = o.base[axis] + (uint32_t)__popcll((o.c[axis] << (63 - (ex & 63))) << 1) - vsolid;
                     }
                     uint32_t *dst = tris + 3 * (t0 + ti);
                     dst[0] = corner[0], dst[1] = corner[1], dst[2] = corner[2];
