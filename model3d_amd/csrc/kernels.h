@@ -750,33 +750,6 @@ __device__ __forceinline__ void keep_masks(const Grid &g, const uint64_t *__rest
     m.cz &= kz | (kz << 1) | ((p00 | p10) >> 63);
 }
 
-// c[k] bit i is corner k (k = dx + 2 dy + 4 dz, mc.go:260-301) of cube 64wx+i.
-struct CubeCorners {
-    uint64_t c[8];
-};
-// The top plane of the grid (of a z slab) has no cubes: no corners.
-__device__ __forceinline__ CubeCorners nbhd_corners(const Nbhd &h) {
-    CubeCorners cc;
-    for (int r = 0; r < 4; r++) {  // r = dy + 2 dz
-        const uint64_t b = h.zin ? h.n[2 * r] : 0, bn = h.zin ? h.n[2 * r + 1] : 0;
-        cc.c[2 * r] = b;
-        cc.c[2 * r + 1] = (b >> 1) | (bn << 63);
-    }
-    return cc;
-}
-
-__device__ __forceinline__ uint64_t mixed_cubes(const CubeCorners &cc) {
-    uint64_t any = 0, all = ~0ull;
-    for (int k = 0; k < 8; k++) any |= cc.c[k], all &= cc.c[k];
-    return any & ~all;
-}
-
-__device__ __forceinline__ int cube_case(const CubeCorners &cc, int i) {
-    int c = 0;
-    for (int k = 0; k < 8; k++) c |= (int)((cc.c[k] >> i) & 1) << k;
-    return c;
-}
-
 // Brick-major order of a one-solid culled call's words (all words of brick
 // 0 row by row, then brick 1, ...): the scan numbers vertices in this order,
 // so the vertices of a brick come out together and the bisection's waves
@@ -839,9 +812,17 @@ __device__ __forceinline__ uint4 classify_position(const Seg *__restrict__ segs,
             h = load_nbhd(g, bits, wx, y, z);
         }
     }
+    // Cube 64wx + i has corners i and i + 1 of the four rows (corner k = dx +
+    // 2 dy + 4 dz, mc.go:260-301); row r = dy + 2 dz is n[2 r] and n[2 r + 1].
+    // Most words lie in one brick constant like its neighbours: no crossings.
+    uint64_t any = 0, all = ~0ull;
+    for (int r = 0; r < 4; r++) {
+        const uint64_t b = h.n[2 * r], up = (b >> 1) | (h.n[2 * r + 1] << 63);
+        any |= b | up, all &= b & up;
+    }
+    if (any == 0 || ~all == 0) return make_uint4(0, 0, 0, 0);
     Masks m = nbhd_masks(h);
-    const CubeCorners cc = nbhd_corners(h);
-    uint64_t mixed = mixed_cubes(cc);
+    uint64_t mixed = h.zin ? any & ~all : 0;  // (the top plane of the grid, or of a z slab, has no cubes)
     if (keep_all) {  // a block filter: only the cubes of accepted blocks
         const uint64_t *keep = keep_all + sg.word0;
         keep_masks(g, keep, wx, y, z, m);
@@ -849,10 +830,18 @@ __device__ __forceinline__ uint4 classify_position(const Seg *__restrict__ segs,
     }
     const uint32_t nv = __popcll(m.cx) + __popcll(m.cy) + __popcll(m.cz);
     uint32_t nt = 0;
+    if (mixed >> 63) {  // the last cube's second corners are the next words'
+        uint32_t cs = 0;
+        for (int r = 0; r < 4; r++) cs |= ((uint32_t)(h.n[2 * r] >> 63) | ((uint32_t)h.n[2 * r + 1] & 1u) << 1) << (2 * r);
+        nt += ntri[cs];
+        mixed &= ~0ull >> 1;
+    }
     while (mixed) {
         const int i = __ffsll((unsigned long long)mixed) - 1;
         mixed &= mixed - 1;
-        nt += ntri[cube_case(cc, i)];
+        uint32_t cs = 0;
+        for (int r = 0; r < 4; r++) cs |= ((uint32_t)(h.n[2 * r] >> i) & 3u) << (2 * r);
+        nt += ntri[cs];
     }
     return make_uint4(nv, nt, (nv | nt) != 0 ? 1u : 0u, 0u);
 }
@@ -860,7 +849,12 @@ __device__ __forceinline__ uint4 classify_position(const Seg *__restrict__ segs,
 // counts[pos] = crossed edges | triangles << 8 | (1 if the word emits
 // anything) << 17, a position per thread, and per block (CLASSIFY_BLOCK
 // positions) the block's sums {edges, triangles, emitting words, 0} for the
-// scan: part_sums[blockIdx.x] (npos: the positions).
+// scan: part_sums[blockIdx.x] (npos: the positions).  Bound by the latency of
+// a wave's loads and, where bricks are crossed, by the loop over a word's mixed
+// cubes: words of one constant leave before their masks are made, and a cube's
+// case is two bits of each row (one at a time before: 512 primitives at 1.0 G
+// corners 224 -> 198 us, 32 solids 49 -> 38, one sphere at 102^3 with the scan
+// 13.5 -> 10.8).
 template <bool MULTI, bool SHFL = false>
 __global__ __launch_bounds__(CLASSIFY_BLOCK) void k_classify(const Seg *__restrict__ segs, uint32_t nsegs, const Seg seg0,
                                                          const uint32_t *__restrict__ word_seg,
