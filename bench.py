@@ -58,12 +58,14 @@ PLAIN_RUN = dict(precision="fp64", cull=False, brick=0, rows_per_walk=1, waves_p
 # rocprofv3 summaries.
 STAGE_KERNEL = {
     "ms_plan": "k_plan",
-    "ms_corners": "k_corners_act",
+    "ms_corners": "k_rows_act",
     "ms_classify": "k_classify",
     "ms_scan": "k_scan_*",
     "ms_emit": "k_emit",
-    "ms_bisect": "k_bisect",
+    "ms_bisect": "k_bisect_rows",
 }
+# where a workload's stage runs another kernel: without culling, and for a collider
+OTHER_KERNEL = {"k_rows_all": "ms_corners", "k_ray_rows": "ms_corners", "k_bisect_rays": "ms_bisect"}
 SUMMED = ("corners", "vertices", "triangles", "bisection_evals", "bricks_total", "program_length")
 
 
@@ -466,14 +468,16 @@ def stage_times(work, run, steps=4):
     return stages, dict(sst[0])
 
 
-def kernel_rooflines(stages, counts, run):
+def kernel_rooflines(stages, counts, run, name):
     kernels = {}
     for stage in STAGE_KERNEL:
         if stages[stage] > 0:
             kernels[STAGE_KERNEL[stage]] = roofline_of(stage, stages[stage], counts)
-    if not run["cull"]:
-        kernels.pop("k_corners_act", None)
-        kernels["k_corners"] = dict(roofline_of("ms_corners", stages["ms_corners"], counts), kernel="k_corners")
+    others = ["k_ray_rows", "k_bisect_rays"] if name == "collider" else ([] if run["cull"] else ["k_rows_all"])
+    for k in others:
+        stage = OTHER_KERNEL[k]
+        if kernels.pop(STAGE_KERNEL[stage], None):
+            kernels[k] = dict(roofline_of(stage, stages[stage], counts), kernel=k)
     return kernels
 
 
@@ -489,7 +493,7 @@ def config_entry(name, steps=5, warmup=2):
     other = "fp32_guard" if run["precision"] == "fp64" else "fp64"
     wall2, _ = run_gpu(work, dict(run, precision=other), steps, 1)
     stages, counts = stage_times(work, run, steps=3)
-    kernels = kernel_rooflines(stages, counts, run)
+    kernels = kernel_rooflines(stages, counts, run, name)
     dom = max(kernels, key=lambda k: kernels[k]["avg_ms"])
     s0 = st[0]
     e = {
@@ -652,7 +656,7 @@ def main():
     }
 
     # Roofline of every kernel; the dominant one is the headline.
-    kernels = kernel_rooflines(stages, counts, run)
+    kernels = kernel_rooflines(stages, counts, run, args.workload)
     dom = max(kernels, key=lambda k: kernels[k]["avg_ms"])
     traffic, source = load_traffic(args.workload, run, dom.rstrip("*").rstrip("_"))
     head = dict(kernels[dom])

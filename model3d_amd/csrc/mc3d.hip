@@ -57,7 +57,12 @@ using namespace mc3d;
 // ---------------------------------------------------------------------------
 constexpr size_t SCRATCH_BYTES = 64u << 20;
 constexpr size_t SCRATCH_AGG_BYTES = 4096;
-static __device__ __align__(256) char scratch[SCRATCH_BYTES];
+// Beside them the parts of the blob that do not count against the limit
+// (Upload::beside): a program's plan tests and the grid's row scale.
+constexpr size_t SCRATCH_BESIDE = 1u << 20;
+constexpr size_t SCRATCH_ALL = SCRATCH_BYTES + SCRATCH_BESIDE;
+static_assert(PLAN_LIST_MAX * sizeof(PlanTest) + 1024 <= SCRATCH_BESIDE, "the largest plan tests fit");
+static __device__ __align__(256) char scratch[SCRATCH_ALL];
 
 namespace {
 
@@ -83,7 +88,7 @@ int scratch_address(int dev, void **out) {
             return MC3D_E_HIP;
         }
         // the one-pass scan sums start zeroed (epoch generation 0)
-        if ((e = hipMemset((char *)p + SCRATCH_BYTES - SCRATCH_AGG_BYTES, 0, SCRATCH_AGG_BYTES)) != hipSuccess ||
+        if ((e = hipMemset((char *)p + SCRATCH_ALL - SCRATCH_AGG_BYTES, 0, SCRATCH_AGG_BYTES)) != hipSuccess ||
             (e = hipDeviceSynchronize()) != hipSuccess) {
             set_error(std::string("hipMemset(scratch): ") + hipGetErrorString(e));
             return MC3D_E_HIP;
@@ -811,6 +816,7 @@ void plan_nodes(const Program &P, const std::vector<AtomBox> &boxes, std::vector
 // device address once placed.
 struct Upload {
     // layout (bytes from the blob's start)
+    size_t beside = 0;  // bytes of plan tests and row scales in the total
     size_t total = 0, o_sout = 0, o_segs = 0, o_wseg = 0, o_bseg = 0, o_pseg = 0, o_conj = 0;
     uint64_t npos_all = 0;  // brick-major scan positions of a call of several (0: none)
     struct Off {
@@ -878,8 +884,11 @@ void layout_upload(const std::vector<Job> &jobs, uint64_t nwords_all, uint64_t n
         po.f32 = place((P.f32.size() + MAX_ATOM_PARAMS) * sizeof(float));
         po.fr = place(P.frames.size() * sizeof(Frame));
         po.nodes = place(nodes.size() * sizeof(PlanNode));
+        U.beside += off - po.nodes - align_up(P.code.size() * sizeof(PlanNode), 256);
         po.col = place(P.colliders.size() * sizeof(DevCollider));
-        po.ax = place((jobs[s].ax[0].size() + jobs[s].ax[1].size() + jobs[s].ax[2].size()) * sizeof(double) + sizeof(RowScale));
+        const size_t axes = (jobs[s].ax[0].size() + jobs[s].ax[1].size() + jobs[s].ax[2].size()) * sizeof(double);
+        po.ax = place(axes + sizeof(RowScale));
+        U.beside += off - po.ax - align_up(axes, 256);
     }
     U.total = off;
 }
@@ -1845,7 +1854,7 @@ int search_noalloc(mc3d_ctx *ctx, const mc3d_solid *s, double delta, int iters, 
     Bufs b;
     size_t need = 0;
     char *base = (char *)ctx->scratch;
-    const uint64_t kcap = carve_scratch(base, SCRATCH_BYTES - SCRATCH_AGG_BYTES, c, U.total, vcap, b, need);
+    const uint64_t kcap = carve_scratch(base, SCRATCH_BYTES - SCRATCH_AGG_BYTES + U.beside, c, U.total, vcap, b, need);
     if (!kcap && vcap) {
         set_error("mc3d_marching_cubes_search_noalloc: the grid needs " + std::to_string(need) +
                   " bytes of scratch, more than the " + std::to_string(SCRATCH_BYTES) + " the library holds");
@@ -1853,7 +1862,7 @@ int search_noalloc(mc3d_ctx *ctx, const mc3d_solid *s, double delta, int iters, 
     }
     b.table = ctx->table.as<uint8_t>();
     b.etable = ctx->etable.as<uint8_t>();
-    b.agg = (ScanAgg *)(base + SCRATCH_BYTES - SCRATCH_AGG_BYTES);
+    b.agg = (ScanAgg *)(base + SCRATCH_ALL - SCRATCH_AGG_BYTES);
     uint64_t gen;
     next_epoch(U.epoch, gen);
     if (g_scratch_agg_gen[ctx->device] != gen) {  // the epochs started over: zero the sums again
