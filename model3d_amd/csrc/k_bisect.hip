@@ -37,7 +37,8 @@ namespace {
 
 template <int MODE, bool STATS>
 void bisect(const Pipe &p, const Bufs &b, double *verts, double *interior, uint64_t vcap, hipStream_t st) {
-    const unsigned grid = grid_for(vcap, 256, 1u << 14);
+    // (the vertices are counted on the device: lanes for either form)
+    const unsigned grid = std::max(grid_for(vcap, 256, 1u << 14), grid_for(std::min(vcap, SPREAD_MAX) * SPREAD, 256));
     if (p.nsegs > 1)
         k_bisect<MODE, STATS, true><<<grid, 256, 0, st>>>(p.segs, p.nsegs, p.seg0, b.vseg, b.bits, b.vkeys, verts,
                                                           interior, p.ctl, vcap);

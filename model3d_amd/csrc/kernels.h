@@ -1306,6 +1306,84 @@ __device__ __forceinline__ void bisect_vertex(const Seg &sg, const uint64_t *__r
     }
 }
 
+// mcSearchPoint for a call of few vertices: SPREAD lanes a vertex evaluate the
+// points that three halvings can reach at once.  A lane a vertex (k_bisect)
+// leaves most of the chip idle while each wave waits for `iters` dependent
+// walks; here there are a third as many, but more of them in all, which costs
+// more once the chip is full.  Measured (a rotated tree of 16 primitives, float32
+// guard, whole calls, a lane a vertex and eight): about 1 k vertices 145 and 113
+// us, 9 k 128 and 106, 34 k 138 and 131, 46 k 168 and 158, 65 k 173 and 179.
+constexpr int SPREAD = 8;
+constexpr uint64_t SPREAD_MAX = 48 * 1024;
+template <int MODE>
+__device__ __forceinline__ void bisect_spread(const Seg &sg, const uint64_t *__restrict__ bits_all,
+                                              const uint64_t *__restrict__ vkeys, double *__restrict__ verts,
+                                              double *__restrict__ interior, uint64_t nv) {
+    const DevProg &P = sg.P;
+    const Grid &g = sg.g;
+    const Bricks &B = sg.B;
+    const uint64_t *bits = bits_all + sg.word0;
+    const int s = (int)(threadIdx.x % SPREAD), first = (int)(threadIdx.x & 63) - s;
+    for (uint64_t v = ((uint64_t)blockIdx.x * 256 + threadIdx.x) / SPREAD; v < nv; v += (uint64_t)gridDim.x * (256 / SPREAD)) {
+        const uint64_t key = vkeys[v];
+        const int axis = (int)(key & 3);
+        const int x = (int)((key >> 2) & 0xfffff), y = (int)((key >> 22) & 0xfffff), z = (int)((key >> 42) & 0xfffff);
+        const double px = g.xs[x], py = g.ys[y], pz = g.zs[z];
+        const double lo = axis == 0 ? px : (axis == 1 ? py : pz);
+        const double hi = *(axis == 0 ? g.xs + x + 1 : (axis == 1 ? g.ys + y + 1 : g.zs + z + 1));
+        const bool up = corner_bit(g, bits, x + (axis == 0), y + (axis == 1), z + (axis == 2));
+        double fp = up ? lo : hi, tp = up ? hi : lo, res;  // the ends outside and inside
+        if (sg.iters == 0) {
+            res = (lo + hi) * 0.5;
+        } else {
+            // the edge's brick program (bisect_vertex)
+            const Insn *code = P.code;
+            uint32_t ncode = P.ncode;
+            int konst = -1;
+            if (B.info) {
+                const uint2 bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
+                if (bi.y == 0) konst = 0;
+                else if (bi.y == BRICK_TRUE) konst = 1;
+                else code = brick_code(P, B, bi), ncode = bi.y;
+            }
+            const uint64_t cp = (uint64_t)code;
+            const uint64_t cp0 = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)cp) |
+                                 ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(cp >> 32)) << 32);
+            const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)ncode);
+            const bool uni = __ballot(cp != cp0 || ncode != n0 || konst >= 0) == 0;
+            GStats gs;
+            for (int left = sg.iters; left > 0;) {
+                const int levels = min(left, 3), top = 1 << (levels - 1);
+                left -= levels;
+                // point s of the bracket, 2^levels steps from fp to tp
+                double m = fp, a = fp, b = tp;
+                for (int bit = top, at = 0; bit; bit >>= 1) {
+                    const double h = (a + b) / 2;
+                    if (at + bit == s) m = h;
+                    if (s > at + bit) a = h, at += bit;
+                    else b = h;
+                }
+                const double qx = axis == 0 ? m : px, qy = axis == 1 ? m : py, qz = axis == 2 ? m : pz;
+                const bool in = konst >= 0 ? konst != 0
+                                : uni      ? eval_code<MODE, false, true>((const Insn *)cp0, n0, P, qx, qy, qz, gs)
+                                           : eval_code<MODE, false, false>(code, ncode, P, qx, qy, qz, gs);
+                const uint32_t mask = (uint32_t)(__ballot(in) >> first);
+                for (int bit = top, at = 0; bit; bit >>= 1) {
+                    const double mid = (fp + tp) / 2;
+                    if ((mask >> (at + bit)) & 1u) tp = mid;
+                    else fp = mid, at += bit;
+                }
+            }
+            res = (fp + tp) / 2;
+        }
+        if (s < 3) {
+            const double at = s == 0 ? px : (s == 1 ? py : pz);
+            verts[3 * v + s] = s == axis ? res : at;
+            if (interior) interior[3 * v + s] = s == axis ? tp : at;
+        }
+    }
+}
+
 template <int MODE, bool STATS, bool MULTI>
 __global__ __launch_bounds__(256) void k_bisect(const Seg *__restrict__ segs, uint32_t nsegs, const Seg seg0,
                                                 const uint32_t *__restrict__ vseg,
@@ -1319,6 +1397,12 @@ __global__ __launch_bounds__(256) void k_bisect(const Seg *__restrict__ segs, ui
     const uint64_t key0 = v0 < vcap ? vkeys[v0] : 0;
     const uint32_t seg0v = MULTI && v0 < vcap ? vseg[v0] : 0u;
     const uint64_t nv = min((uint64_t)ctl->totals[0], vcap);
+    if constexpr (!STATS && !MULTI) {
+        if (nv <= SPREAD_MAX) {
+            bisect_spread<MODE>(seg0, bits_all, vkeys, verts, interior, nv);
+            return;
+        }
+    }
     for (uint64_t v = v0; v < nv; v += (uint64_t)gridDim.x * blockDim.x) {
         const uint64_t key = v == v0 ? key0 : vkeys[v];
         // Lanes may belong to different solids: take them one solid at a time.
