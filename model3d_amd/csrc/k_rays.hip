@@ -19,7 +19,8 @@
 // instructions for 64 triangles of 4 rows).  Measured (kernel trace, MI355X, a
 // mesh made at spacing 0.02): 256^3 corners 993 -> 215 us, their vertices'
 // bisection (8 halvings) 448 -> 192 us; the whole call at 40^3 corners 462 ->
-// 180 us.
+// 180 us; the corners of a mesh with faces in the grid's planes, 1,410 -> 262 us
+// (838 with a lane looking up all the undecided corners of its 32).
 #include "launch.h"
 #include "rows.h"
 
@@ -144,10 +145,10 @@ struct RayBound {
     double lo, lo_z, hi, hi_z, w;
 };
 __device__ __forceinline__ bool ray_flat(double A, double e, double nx) { return !(fabs(A) * nx > 1e3 * e); }
-__device__ __forceinline__ RayBound ray_bound(double A, double B, double slope, double e) {
+__device__ __forceinline__ RayBound ray_bound(double A, double B, double slope, double e, bool flat) {
     const double q = recip(A), at = -B * q, z = -slope * q;
-    const bool up = A > 0;
-    return RayBound{up ? at : -1e9, up ? z : 0, up ? 1e9 : at, up ? 0 : z, e * fabs(q)};
+    const bool up = A > 0 && !flat, down = !up && !flat;
+    return RayBound{up ? at : -1e9, up ? z : 0, down ? at : 1e9, down ? z : 0, flat ? 0 : e * fabs(q)};
 }
 // Corners that may be in ([p0, p1]) and that are ([s0, s1]).
 struct RayRange {
@@ -222,10 +223,11 @@ __global__ __launch_bounds__(64) void k_ray_rows(const Seg sg, uint64_t *__restr
                 const double c1 = q[0] * px + q[3] * py + q[9], c2 = q[1] * px + q[4] * py + q[10];
                 const double c3 = q[2] * px + q[5] * py + q[11];
                 const double A12 = -(A1 + A2), c12 = 1 - c1 - c2, q12 = -(q[6] + q[7]), e12 = e1 + e2 + 1e-15;
-                const bool flat = have && (ray_flat(A1, e1, nx) || ray_flat(A2, e2, nx) || ray_flat(A12, e12, nx) || ray_flat(A3, e3, nx));
-                const bool slow = __ballot(flat) != 0;
-                const RayBound b1 = ray_bound(A1, c1, q[6], e1), b2 = ray_bound(A2, c2, q[7], e2);
-                const RayBound b12 = ray_bound(A12, c12, q12, e12), b3 = ray_bound(A3, c3, q[8], e3);
+                // (edges along x: common in meshes of boxes and of grids)
+                const bool f1 = ray_flat(A1, e1, nx), f2 = ray_flat(A2, e2, nx), f12 = ray_flat(A12, e12, nx), f3 = ray_flat(A3, e3, nx);
+                const bool flat = __ballot(f1 || f2 || f12 || f3) != 0;
+                const RayBound b1 = ray_bound(A1, c1, q[6], e1, f1), b2 = ray_bound(A2, c2, q[7], e2, f2);
+                const RayBound b12 = ray_bound(A12, c12, q12, e12, f12), b3 = ray_bound(A3, c3, q[8], e3, f3);
                 const double w = fmax(fmax(b1.w, b2.w), fmax(b12.w, b3.w)) + rs.eta;
                 for (int r = 0; r < RAY_ROWS; r++) {
                     if (r >= nr) break;
@@ -235,23 +237,16 @@ __global__ __launch_bounds__(64) void k_ray_rows(const Seg sg, uint64_t *__restr
                     const double hi = fmin(fmin(__builtin_fma(b1.hi_z, z, b1.hi), __builtin_fma(b2.hi_z, z, b2.hi)),
                                            fmin(__builtin_fma(b12.hi_z, z, b12.hi), __builtin_fma(b3.hi_z, z, b3.hi)));
                     RayRange g4 = ray_range(lo, hi, w, nx);
-                    if (slow && flat) {  // bound by bound
-                        double l = -1e9, h = 1e9, wm = rs.eta;
+                    if (flat) {
                         bool may = true, sure = true;
-                        auto bound = [&](double A, double B, double e, const RayBound &b) {
-                            if (ray_flat(A, e, nx)) {
-                                const double m = e + fabs(A) * nx;
-                                may = may && !(B < -m), sure = sure && B >= m;
-                            } else {
-                                l = fmax(l, __builtin_fma(b.lo_z, z, b.lo)), h = fmin(h, __builtin_fma(b.hi_z, z, b.hi));
-                                wm = fmax(wm, b.w + rs.eta);
-                            }
+                        auto check = [&](bool f, double A, double B, double e) {
+                            const double m = e + fabs(A) * nx;
+                            may = may && !(f && B < -m), sure = sure && !(f && !(B >= m));
                         };
-                        bound(A1, c1 + q[6] * z, e1, b1);
-                        bound(A2, c2 + q[7] * z, e2, b2);
-                        bound(A12, c12 + q12 * z, e12, b12);
-                        bound(A3, c3 + q[8] * z, e3, b3);
-                        g4 = ray_range(l, h, wm, nx);
+                        check(f1, A1, c1 + q[6] * z, e1);
+                        check(f2, A2, c2 + q[7] * z, e2);
+                        check(f12, A12, c12 + q12 * z, e12);
+                        check(f3, A3, c3 + q[8] * z, e3);
                         if (!may) g4.p1 = -1;
                         if (!sure) g4.s1 = -1;
                     }
@@ -281,21 +276,24 @@ __global__ __launch_bounds__(64) void k_ray_rows(const Seg sg, uint64_t *__restr
                 for (int d = 1; d < 32; d <<= 1) v ^= v << d;
                 const uint64_t odd = __ballot(v >> 31);
                 if (__popcll(odd & ((1ull << lane) - 1)) & 1) v = ~v;
-                // the corners within the collider's bounds
+                // the corners within the collider's bounds, and the undecided
+                // ones of them looked up, a lane a corner (a row in the plane
+                // of a mesh face has them all the way along)
+                uint32_t undecided = 0, found = 0;
                 for (int w = 0; w < (nx + 63) / 64; w++) {
                     const int x = x0 + 64 * w + lane;
                     const double X = g.xs[min(x, g.nx - 1)];
-                    const uint64_t m = __ballot(x < g.nx && in_lo(X, a[1]) && in_hi(X, a[4]));
-                    if (lane >> 1 == w) inside = lane & 1 ? (uint32_t)(m >> 32) : (uint32_t)m;
+                    const bool in = x < g.nx && in_lo(X, a[1]) && in_hi(X, a[4]);
+                    const bool ask = in && ((open[r][2 * w + (lane >> 5)] >> (lane & 31)) & 1u);
+                    const uint64_t m = __ballot(in), q = __ballot(ask);
+                    uint64_t hit = 0;
+                    if (q) hit = __ballot(ask && collider_contains(C, (const double *)(sg.P.f64 + sg.P.code[0].y), X, py, z));
+                    if (lane >> 1 == w) {
+                        const int half = 32 * (lane & 1);
+                        inside = (uint32_t)(m >> half), undecided = (uint32_t)(q >> half), found = (uint32_t)(hit >> half);
+                    }
                 }
-                uint32_t undecided = lane < RAY_SPAN / 32 ? open[r][lane] & inside : 0u;
-                while (undecided) {
-                    const int k = __ffs(undecided) - 1;
-                    undecided &= undecided - 1;
-                    const bool in = collider_contains(C, (const double *)(sg.P.f64 + sg.P.code[0].y), g.xs[x0 + 32 * lane + k],
-                                                      py, z);
-                    v = (v & ~(1u << k)) | ((uint32_t)in << k);
-                }
+                v = (v & ~undecided) | found;
                 v &= inside;
             }
             // (a word's two halves: an odd last half is written by the lane after it)
