@@ -1933,8 +1933,11 @@ int mc3d_ctx_create(int device, mc3d_ctx **out) {
             mc3d_ctx_destroy(c.release());
             return MC3D_E_HIP;
         }
-        for (auto &ev : c->ev) {
-            if (hipEventCreate(&ev) != hipSuccess) {
+        for (int i = 0; i < EV_N; i++) {
+            // The events between stages only time them: nothing waits for one,
+            // so they need not make memory visible to the system.
+            const bool timing = i == EV_PLAN0 || i == EV_PLAN1 || i == EV_CORNERS || i == EV_CLASSIFY || i == EV_SCAN || i == EV_EMIT0;
+            if (hipEventCreateWithFlags(&c->ev[i], timing ? hipEventDisableSystemFence : hipEventDefault) != hipSuccess) {
                 set_error("hipEventCreate failed");
                 mc3d_ctx_destroy(c.release());
                 return MC3D_E_HIP;
