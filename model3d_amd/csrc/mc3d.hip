@@ -238,7 +238,10 @@ struct Pool {
 // Host threads kept for the library's parallel host loops (lowering a
 // batch's solids, filling its upload): run(n, fn) calls fn(i) for every
 // i < n on up to 16 threads, the caller's included, and returns when all
-// are done.  Runs from several threads take turns.
+// are done -- not when every thread has woken: a thread that wakes late finds
+// its task's indices taken (it holds the task itself) and sleeps again (a
+// batch of 32 solids, whole calls: 769 -> 733 us).  Runs from several threads
+// take turns.
 class HostPool {
   public:
     static HostPool &get() {
@@ -252,15 +255,18 @@ class HostPool {
             return;
         }
         std::lock_guard<std::mutex> one(run_mu_);
+        const auto task = std::make_shared<Task>();
+        task->fn = &fn, task->n = n;
         {
             std::lock_guard<std::mutex> lk(mu_);
-            fn_ = &fn, n_ = n, next_ = 0, busy_ = workers_.size(), gen_++;
+            task_ = task, gen_++;
         }
         cv_.notify_all();
-        drain();
+        drain(*task);
         std::unique_lock<std::mutex> lk(mu_);
-        done_cv_.wait(lk, [&] { return busy_ == 0; });
-        fn_ = nullptr;
+        done_cv_.wait(lk, [&] { return task->done == n; });
+        task_ = nullptr;
+        if (task->error) std::rethrow_exception(task->error);
     }
 
   private:
@@ -276,28 +282,44 @@ class HostPool {
         cv_.notify_all();
         for (std::thread &t : workers_) t.join();
     }
-    void drain() {
-        for (size_t i; (i = next_.fetch_add(1)) < n_;) (*fn_)(i);
+    // One run's work; fn is the caller's, and outlives every index claimed.
+    struct Task {
+        const std::function<void(size_t)> *fn = nullptr;
+        size_t n = 0;
+        std::atomic<size_t> next{0}, done{0};
+        std::exception_ptr error;  // the first thrown (under mu_)
+    };
+    void drain(Task &t) {
+        for (size_t i; (i = t.next.fetch_add(1)) < t.n;) {
+            try {
+                (*t.fn)(i);
+            } catch (...) {
+                std::lock_guard<std::mutex> lk(mu_);
+                if (!t.error) t.error = std::current_exception();
+            }
+            if (t.done.fetch_add(1) + 1 == t.n) {
+                std::lock_guard<std::mutex> lk(mu_);  // (the caller is waiting, or has yet to look)
+                done_cv_.notify_all();
+            }
+        }
     }
     void loop() {
         uint64_t seen = 0;
         for (;;) {
+            std::shared_ptr<Task> task;
             {
                 std::unique_lock<std::mutex> lk(mu_);
                 cv_.wait(lk, [&] { return stop_ || gen_ != seen; });
                 if (stop_) return;
                 seen = gen_;
+                task = task_;  // (null: that run is over)
             }
-            drain();
-            std::lock_guard<std::mutex> lk(mu_);
-            if (--busy_ == 0) done_cv_.notify_all();
+            if (task) drain(*task);
         }
     }
     std::mutex run_mu_, mu_;
     std::condition_variable cv_, done_cv_;
-    const std::function<void(size_t)> *fn_ = nullptr;
-    size_t n_ = 0, busy_ = 0;
-    std::atomic<size_t> next_{0};
+    std::shared_ptr<Task> task_;
     uint64_t gen_ = 0;
     bool stop_ = false;
     std::vector<std::thread> workers_;
