@@ -342,9 +342,10 @@ int mc3d_case_table(uint8_t out[256 * 16]);
 int mc3d_diag_stream(mc3d_ctx *ctx, size_t bytes, int32_t write, double *ms);
 
 /* Diagnostics (host only, no GPU): folds random programs against random
- * brick boxes with the brick plan's two folds -- every instruction in turn,
- * and with subtrees whose atoms all miss the brick skipped -- and counts the
- * cases whose folded code, root or overflow differ (must be 0).  No
+ * brick boxes with the brick plan's folds -- every instruction in turn, and
+ * with subtrees whose atoms all miss the brick skipped -- and counts the
+ * cases whose folded code, root or overflow differ, or whose brick record
+ * has a bisection walk anything but that code (must be 0).  No
  * counterpart in the reference; it checks the library's own culling. */
 int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked, uint64_t *mismatches);
 

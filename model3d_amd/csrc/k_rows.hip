@@ -161,21 +161,28 @@ __device__ __forceinline__ void bisect_rows(const Seg &sg, const uint64_t *__res
     // the high corner decides which end is inside
     const bool up = corner_bit(g, bits, x + (k == 0), y + (k == 1), z + (k == 2));
     if (sg.iters > 0) {
-        // the edge's brick program (a crossed edge lies in a brick that is
-        // evaluated: the boxes of constant bricks hold their +1 corners)
-        uint2 bi = make_uint2(BRICK_FULL, P.ncode);
-        if (B.info) bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
-        const uint2 b0 = make_uint2((uint32_t)__builtin_amdgcn_readfirstlane((int)bi.x),
-                                    (uint32_t)__builtin_amdgcn_readfirstlane((int)bi.y));
-        const bool uni = __ballot(bi.x != b0.x || bi.y != b0.y) == 0;  // one program for the wave: scalar loads
-        const Insn *code = brick_code(P, B, bi), *code0 = brick_code(P, B, b0);
+        // the edge's brick program (an edge crossed in a brick that the plan
+        // found constant is decided by that constant, as in bisect_vertex)
+        BrickProgram bp{P.code, P.ncode, -1};
+        if (B.info) {
+            const uint2 bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
+            bp = brick_program(P, B, bi.x, bi.y);
+        }
+        const uint64_t cp = (uint64_t)bp.code;
+        const uint64_t cp0 = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)cp) |
+                             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(cp >> 32)) << 32);
+        const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)bp.n);
+        // one program for the wave: scalar loads
+        const bool uni = __ballot(cp != cp0 || bp.n != n0 || bp.konst >= 0) == 0;
+        const Insn *code = bp.code, *code0 = (const Insn *)cp0;
         const LineAxis<false> ax(k);
         int left = sg.iters;
         while (left > 2) {
             const int levels = min(left, 6);
-            const uint64_t m = uni ? bracket_bits<true>(scalar_ptr(code0), b0.y, scalar_ptr(P.f64), g, ax, lo, hi, px, py,
+            const uint64_t m = bp.konst >= 0 ? (bp.konst ? ~0ull : 0)
+                               : uni ? bracket_bits<true>(scalar_ptr(code0), n0, scalar_ptr(P.f64), g, ax, lo, hi, px, py,
                                                         pz, levels, stack)
-                                   : bracket_bits<false>(code, bi.y, P.f64, g, ax, lo, hi, px, py, pz, levels, stack);
+                                   : bracket_bits<false>(code, bp.n, P.f64, g, ax, lo, hi, px, py, pz, levels, stack);
             for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
                 const double mid = (lo + hi) / 2;
                 const bool in = (m >> (at + bit)) & 1;
@@ -188,8 +195,9 @@ __device__ __forceinline__ void bisect_rows(const Seg &sg, const uint64_t *__res
             const double mid = (lo + hi) / 2;
             const double qx = k == 0 ? mid : px, qy = k == 1 ? mid : py, qz = k == 2 ? mid : pz;
             GStats gs;
-            const bool in = uni ? eval_code<0, false, true>(code0, b0.y, P, qx, qy, qz, gs)
-                                : eval_code<0, false, false>(code, bi.y, P, qx, qy, qz, gs);
+            const bool in = bp.konst >= 0 ? bp.konst != 0
+                            : uni         ? eval_code<0, false, true>(code0, n0, P, qx, qy, qz, gs)
+                                          : eval_code<0, false, false>(code, bp.n, P, qx, qy, qz, gs);
             if (in == up) hi = mid;
             else lo = mid;
         }

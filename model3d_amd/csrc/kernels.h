@@ -294,11 +294,8 @@ __global__ __launch_bounds__(PLAN_BLOCK) void k_plan(const Seg *__restrict__ seg
         }
         if (valid) {
             const uint32_t root = S[0];
-            uint2 bi;
-            if (root == TAG_FALSE) bi = make_uint2(0, 0);
-            else if (root == TAG_TRUE) bi = make_uint2(0, BRICK_TRUE);
-            else if (over) bi = make_uint2(BRICK_FULL, P.ncode), active = true;
-            else bi = make_uint2((uint32_t)(gb * cap), n), active = true;
+            const uint2 bi = brick_record(root, over, (uint32_t)(gb * cap), n, P.ncode);
+            active = root != TAG_FALSE && root != TAG_TRUE;
             info[gb] = bi;
             if (!active) {  // the constant brick's words
                 const bool t = root == TAG_TRUE;
@@ -1258,9 +1255,8 @@ __device__ __forceinline__ void bisect_vertex(const Seg &sg, const uint64_t *__r
             int konst = -1;
             if (B.info) {
                 const uint2 bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
-                if (bi.y == 0) konst = 0;
-                else if (bi.y == BRICK_TRUE) konst = 1;
-                else code = brick_code(P, B, bi), ncode = bi.y;
+                const BrickProgram bp = brick_program(P, B, bi.x, bi.y);
+                code = bp.code, ncode = bp.n, konst = bp.konst;
             }
             // One program for every lane of the wave (no culling, or lanes
             // of one brick: vertices are numbered brick by brick): walked
@@ -1342,9 +1338,8 @@ __device__ __forceinline__ void bisect_spread(const Seg &sg, const uint64_t *__r
             int konst = -1;
             if (B.info) {
                 const uint2 bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
-                if (bi.y == 0) konst = 0;
-                else if (bi.y == BRICK_TRUE) konst = 1;
-                else code = brick_code(P, B, bi), ncode = bi.y;
+                const BrickProgram bp = brick_program(P, B, bi.x, bi.y);
+                code = bp.code, ncode = bp.n, konst = bp.konst;
             }
             const uint64_t cp = (uint64_t)code;
             const uint64_t cp0 = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)cp) |

@@ -2868,6 +2868,16 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
                     same = same && S1[0] == S2[0] && n1 == n2 && over1 == over2;
                     for (uint32_t i = 0; same && i < std::min(n1, cap); i++)
                         same = o1[i].x == o2[i].x && o1[i].y == o2[i].y;
+                    // what its record has a bisection walk: nothing where it is constant
+                    const uint2 rec = brick_record(S1[0], over1, 0, n1, ncode);
+                    DevProg dp{};
+                    dp.code = P.code.data(), dp.ncode = ncode;
+                    Bricks B{};
+                    B.code = o1;
+                    const BrickProgram bp = brick_program(dp, B, rec.x, rec.y);
+                    const int konst = S1[0] == TAG_TRUE ? 1 : S1[0] == TAG_FALSE ? 0 : -1;
+                    const uint32_t len = konst >= 0 ? 0 : over1 ? ncode : n1;
+                    same = same && bp.konst == konst && bp.n == len && (len == 0 || bp.code == (over1 ? dp.code : o1));
                     nchecked++;
                     nbad += same ? 0 : 1;
                 }

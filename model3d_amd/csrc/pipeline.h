@@ -75,6 +75,19 @@ struct Bricks {
     int BY, BZ, nby, nbz;
 };
 
+// What a brick's record says to evaluate: konst 0 or 1 where the solid is that
+// all over the brick (no instruction is walked: n is 0), else -1 and the code.
+struct BrickProgram {
+    const Insn *code;
+    uint32_t n;
+    int konst;
+};
+MC3D_HD inline BrickProgram brick_program(const DevProg &P, const Bricks &B, uint32_t at, uint32_t n) {
+    if (n == 0) return BrickProgram{P.code, 0, 0};
+    if (n == BRICK_TRUE) return BrickProgram{P.code, 0, 1};
+    return BrickProgram{at == BRICK_FULL ? P.code : B.code + at, n, -1};
+}
+
 // One solid of a call.  B.info / B.code are the call's arrays, indexed by the
 // global brick number; word and brick numbers are local to the segment
 // unless named global.  Kernels also take the first segment by value (a

@@ -23,6 +23,7 @@
 
 #include "eval.h"
 #include "mc3d_internal.h"
+#include "pipeline.h"
 
 namespace mc3d {
 
@@ -62,6 +63,14 @@ MC3D_HD inline int classify_atom(F64P f64, BoxP boxes, uint32_t pc, Insn in, con
 }
 
 constexpr uint32_t TAG_EXPR = 0u, TAG_FALSE = 1u << 30, TAG_TRUE = 2u << 30, TAG_MASK = 3u << 30;
+
+// The record (Bricks::info) of a brick whose fold left `root`, n instructions
+// at `at`, or more than its slot holds.
+MC3D_HD inline uint2 brick_record(uint32_t root, bool over, uint32_t at, uint32_t n, uint32_t ncode) {
+    if (root == TAG_FALSE) return make_uint2(0, 0);
+    if (root == TAG_TRUE) return make_uint2(0, BRICK_TRUE);
+    return over ? make_uint2(BRICK_FULL, ncode) : make_uint2(at, n);
+}
 
 // One instruction of the fold (S: the stack, sp its depth).
 template <class BoxP, class F64P, class Stack>

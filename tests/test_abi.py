@@ -120,3 +120,17 @@ def test_row_bounds_match_contains():
     assert checked.value > 300000 * 32
     assert bad.value == 0
     assert opened.value < checked.value // 2  # (most points are decided)
+
+
+def test_constant_bricks_have_no_code():
+    """A brick that the plan folds to a constant gives a bisection that
+    constant and no instruction to walk; any other its folded code, or the
+    whole program where that overflowed (the records of 20,000 random
+    programs x 16 bricks, tiny slots among them; host code, no GPU)."""
+    import ctypes
+
+    L = _lib.lib()
+    checked, bad = ctypes.c_uint64(), ctypes.c_uint64()
+    assert L.mc3d_selftest_plan_fold(31, 20000, ctypes.byref(checked), ctypes.byref(bad)) == 0
+    assert checked.value == 20000 * 16
+    assert bad.value == 0
