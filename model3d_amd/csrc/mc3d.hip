@@ -2903,8 +2903,11 @@ int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_
         auto uni = [&](double lo, double hi) { return lo + (hi - lo) * (double)(next() >> 11) * 0x1.0p-53; };
         auto mag10 = [&](double lo, double hi) { return pow(10.0, uni(lo, hi)); };
         for (uint32_t l = 0; l < lines; l++) {
-            // spacing, and coordinates up to 10^6 spacings from the origin
-            const double h = next() % 4 ? mag10(-4, 0) : pow(2.0, -(double)(next() % 8)), far = h * mag10(0, 6);
+            // spacing -- also of solids as small and as large as the row forms
+            // take -- and coordinates up to 10^6 (there 10^9) spacings from the origin
+            const bool scaled = next() & 1;
+            const double unit = scaled ? mag10(-90, 85) : 1;
+            const double h = unit * (next() % 4 ? mag10(-4, 0) : pow(2.0, -(double)(next() % 8))), far = h * mag10(0, scaled ? 8.5 : 6);
             double c[3], d[3], p[3];
             for (int a = 0; a < 3; a++) c[a] = uni(-far, far), d[a] = uni(-1, 1);
             const int k = (int)(next() % 3);
@@ -2935,6 +2938,14 @@ int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_
             const int o = (k + 1 + (int)(next() & 1)) % 3;
             if (next() % 4 == 0) p[(k + 1) % 3] = c[(k + 1) % 3], p[(k + 2) % 3] = c[(k + 2) % 3];
             if (next() % 3 == 0) p[o] = c[o] + r * (1 + (next() & 1 ? 0 : uni(-1, 1) * mag10(-16, -6)));
+            if (next() % 4 == 0) {  // beside or on the axis: a tangent of the round side
+                double n[3] = {0, 0, 0};
+                n[(k + 1) % 3] = -d[(k + 2) % 3], n[(k + 2) % 3] = d[(k + 1) % 3];
+                const double nn = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]), t = uni(0, 1);
+                const double at = (1 + (next() & 1 ? 0 : uni(-1, 1) * mag10(-16, -6))) * r;
+                if (nn > 0)
+                    for (int q = 0; q < 3; q++) p[q] = c[q] + t * (e[q] - c[q]) + n[q] / nn * at;
+            }
             if (next() % 4 == 0) p[k] = (next() & 1 ? lo[k] : hi[k]) - (double)(next() % 60) * h;
             else p[k] -= uni(0, 64) * h;
             const bool edge = next() & 1;

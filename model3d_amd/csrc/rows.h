@@ -48,19 +48,17 @@ MC3D_HD inline double recip(double x) {
 }
 
 // ro >= sqrt(w') >= ri for every w' in [w - D, w + D] (w >= -D), with e0
-// more on each side; ri < 0: w' may be below zero.
+// more on each side; ri < 0: w' may be below zero.  (All in float64: D goes
+// down to 1e-219 over the coordinates that span_range admits.)
 MC3D_HD inline void span_root(double w, double D, double e0, double &ro, double &ri) {
-    if (w <= 4 * D) {  // the line grazes the surface
-        ro = (double)sqrtf((float)(5 * D)) * 1.001 + e0;
-        ri = -1;
-        return;
-    }
-    const double y = rsq_estimate(w);
-    double r = w * y;
-    r = r + 0.5 * y * __builtin_fma(-r, r, w);
-    const double e = 1.1 * D * y + 1e-10 * r + e0;
+    const bool graze = w <= 4 * D;  // the line grazes the surface
+    const double v = graze ? 5 * D : w;
+    const double y = rsq_estimate(v);
+    double r = v * y;
+    r = r + 0.5 * y * __builtin_fma(-r, r, v);
+    const double e = graze ? 1e-3 * r + e0 : 1.1 * D * y + 1e-10 * r + e0;
     ro = r + e;
-    ri = r - e;
+    ri = graze ? -1 : r - e;
 }
 
 // Coordinates that are neither so large nor so small that a square or a

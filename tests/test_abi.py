@@ -134,3 +134,18 @@ def test_constant_bricks_have_no_code():
     assert L.mc3d_selftest_plan_fold(31, 20000, ctypes.byref(checked), ctypes.byref(bad)) == 0
     assert checked.value == 20000 * 16
     assert bad.value == 0
+
+
+def test_row_bounds_match_contains_at_every_scale():
+    """The same over solids from 1e-90 to 1e85 in size (half of the draws),
+    with tangent lines of tilted cylinders among them: a bound that loses its
+    digits, underflows or overflows at some scale calls wrong points certain."""
+    import ctypes
+
+    L = _lib.lib()
+    checked, opened, bad = ctypes.c_uint64(), ctypes.c_uint64(), ctypes.c_uint64()
+    for seed in (5, 6):
+        assert L.mc3d_selftest_rows(seed, 500000, ctypes.byref(checked), ctypes.byref(opened), ctypes.byref(bad)) == 0
+        assert checked.value > 500000 * 32
+        assert bad.value == 0
+        assert opened.value < checked.value // 2
