@@ -358,6 +358,16 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
  * bounds the corner and bisection kernels decide whole rows by. */
 int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_t *open, uint64_t *mismatches);
 
+/* Diagnostics (host only, no GPU): the entries of GroupTriangles' three
+ * orders of n triangles as three threads of a grid of that many walk them
+ * (the first, the middle and the last); *visited of them, *misplaced not at
+ * the axis and position of their number (must be 0). */
+int mc3d_selftest_group_entries(uint32_t n, uint64_t grid, uint64_t *visited, uint64_t *misplaced);
+/* mc3d_group_triangles with the three axes' keys sorted one by one, as for
+ * more than 2^31 / 3 triangles (the same order). */
+int mc3d_selftest_group_sorts(mc3d_ctx *ctx, const double *verts, size_t nv, const uint32_t *tris, size_t nt,
+                              uint32_t *perm);
+
 const char *mc3d_last_error(void);
 const char *mc3d_version(void);
 

@@ -198,6 +198,12 @@ SIGNATURES = {
     "mc3d_selftest_rows": (
         ctypes.c_int, [ctypes.c_uint64, ctypes.c_uint32] + [ctypes.POINTER(ctypes.c_uint64)] * 3
     ),
+    "mc3d_selftest_group_entries": (
+        ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint64, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]
+    ),
+    "mc3d_selftest_group_sorts": (
+        ctypes.c_int, [_P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
+    ),
     "mc3d_last_error": (ctypes.c_char_p, []),
     "mc3d_version": (ctypes.c_char_p, []),
 }

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void k_grp_boxes(const double *__restrict__ ve
                                                    uint32_t *__restrict__ vals, uint32_t step) {
     for (uint32_t t = blockIdx.x * blockDim.x + threadIdx.x; t < n; t += gridDim.x * blockDim.x) {
         const double *p[3];
-        for (int k = 0; k < 3; k++) p[k] = verts + 3 * (size_t)(tris ? tris[3 * (size_t)t + k] : 3 * t + k);
+        for (int k = 0; k < 3; k++) p[k] = verts + 3 * (tris ? (size_t)tris[3 * (size_t)t + k] : 3 * (size_t)t + k);
         GroupBox b;
         for (int a = 0; a < 3; a++) {
             b.mn[a] = rc::go_min(rc::go_min(p[0][a], p[1][a]), p[2][a]);
@@ -235,13 +235,11 @@ __global__ __launch_bounds__(256) void k_grp_axis_slots(GroupLevel G, const unsi
 // flag[t] = 1 for the triangles in the first half of their node along the
 // node's axis (splitBounders, bvh.go:159-217).
 __global__ __launch_bounds__(256) void k_grp_flags(GroupLevel G) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 3 * G.n; i += gridDim.x * blockDim.x) {
-        const int a = (int)(i / G.n);
-        const uint32_t p = i - a * G.n;
+    each_order_entry(G.n, blockIdx.x * (uint64_t)blockDim.x + threadIdx.x, (uint64_t)gridDim.x * blockDim.x, [&](int a, uint32_t p) {
         uint32_t lo, hi;
         const uint32_t k = node_of(p, G.n, G.L, lo, hi);
         if (G.axis[k] == a) G.flag[G.perm[a][p]] = p < lo + (hi - lo) / 2;
-    }
+    });
 }
 
 // Triangles flagged in the nodes of level L that lie before position lo, the
@@ -552,7 +550,7 @@ __global__ __launch_bounds__(GRP_THREADS) void k_grp_local(GroupLevel G, uint32_
 
 __global__ __launch_bounds__(256) void k_grp_apply(const uint32_t *__restrict__ tris, const uint32_t *__restrict__ perm,
                                                    uint32_t n, uint32_t *__restrict__ out) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < 3 * n; i += gridDim.x * blockDim.x)
+    for (uint64_t i = blockIdx.x * (uint64_t)blockDim.x + threadIdx.x; i < 3ull * n; i += (uint64_t)gridDim.x * blockDim.x)
         out[i] = tris[3 * (size_t)perm[i / 3] + i % 3];
 }
 

@@ -173,6 +173,15 @@ struct GroupLevel {
     uint8_t *axis = nullptr;
     uint8_t *flag = nullptr;
 };
+// Entries first, first + step, ... of the three orders of n triangles (3 n of
+// them, more than 32 bits from n = 2^32 / 3 on): f(axis, position).
+template <class F>
+MC3D_HD inline void each_order_entry(uint32_t n, uint64_t first, uint64_t step, F &&f) {
+    for (uint64_t i = first; i < 3ull * n; i += step) {
+        const int a = i >= 2ull * n ? 2 : (i >= n ? 1 : 0);
+        f(a, (uint32_t)(i - (uint64_t)a * n));
+    }
+}
 // boxes and midpoint keys of triangles (verts + tris, or 9 doubles each when
 // tris is null): keys[a * n + t] with vals[a * n + t] = a * step + t
 hipError_t launch_grp_boxes(const double *verts, const uint32_t *tris, uint32_t n, GroupBox *box, uint64_t *keys,

@@ -2504,8 +2504,11 @@ namespace {
 // GroupTriangles of n triangles on this context's device (vertices and
 // triangle indices, or 9 doubles per triangle when tris is null): *perm
 // receives a device array of n triangle indices in the grouped order
-// (valid until the next grouping on this context).
-int group_order(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, uint64_t n, const uint32_t **perm) {
+// (valid until the next grouping on this context).  one_sort: from this many
+// entries on the axes are sorted one by one (a sort takes at most 2^31 - 1).
+constexpr uint64_t GROUP_ONE_SORT = 1ull << 31;
+int group_order(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, uint64_t n, const uint32_t **perm,
+                uint64_t one_sort = GROUP_ONE_SORT) {
     *perm = nullptr;
     if (n >= (1ull << 31)) {
         set_error("GroupTriangles: more than 2^31 triangles");
@@ -2525,9 +2528,8 @@ int group_order(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, uint64
     const uint32_t n32 = (uint32_t)n;
     // One sort of the three axes' keys, then each axis's own out of it: a sort
     // of a few hundred thousand keys is bound by its launches (203k triangles:
-    // 253 us, split included, for 574 us in three).  Past the sort's 2^31 entries
-    // there are three.
-    const bool one = 3 * n < (1ull << 31);
+    // 253 us, split included, for 574 us in three).
+    const bool one = 3 * n < one_sort;
     const uint32_t entries = one ? 3 * n32 : n32;
     size_t sort_bytes = 0;
     HIP_TRY(grp_sort(nullptr, sort_bytes, nullptr, nullptr, nullptr, nullptr, entries, st));
@@ -2567,6 +2569,25 @@ int group_order(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, uint64
     }
     *perm = P[0];
     return MC3D_OK;
+}
+
+// GroupTriangles over host arrays (checked by the caller).
+int group_host_arrays(mc3d_ctx *ctx, const double *verts, size_t nv, const uint32_t *tris, size_t nt, uint32_t *perm,
+                      uint64_t one_sort) {
+    return guarded([&]() -> int {
+        HIP_TRY(hipSetDevice(ctx->device));
+        int rc;
+        if ((rc = ctx->stl_in.ensure(nv * 24 + nt * 12 + 16))) return rc;
+        double *dv = ctx->stl_in.as<double>();
+        uint32_t *dt = (uint32_t *)(ctx->stl_in.as<char>() + align_up(nv * 24, 16));
+        if (nv) HIP_TRY(hipMemcpyAsync(dv, verts, nv * 24, hipMemcpyHostToDevice, ctx->stream));
+        if (nt) HIP_TRY(hipMemcpyAsync(dt, tris, nt * 12, hipMemcpyHostToDevice, ctx->stream));
+        const uint32_t *dp = nullptr;
+        if ((rc = group_order(ctx, dv, dt, nt, &dp, one_sort))) return rc;
+        if (nt) HIP_TRY(hipMemcpyAsync(perm, dp, nt * 4, hipMemcpyDeviceToHost, ctx->stream));
+        HIP_TRY(hipStreamSynchronize(ctx->stream));
+        return MC3D_OK;
+    });
 }
 
 int encode_stl_device(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, uint64_t nt, uint8_t *out,
@@ -2627,20 +2648,7 @@ int mc3d_group_triangles(mc3d_ctx *ctx, const double *verts, size_t nv, const ui
                       std::to_string(tris[i]) + " of " + std::to_string(nv));
             return MC3D_E_INVALID_ARG;
         }
-    return guarded([&]() -> int {
-        HIP_TRY(hipSetDevice(ctx->device));
-        int rc;
-        if ((rc = ctx->stl_in.ensure(nv * 24 + nt * 12 + 16))) return rc;
-        double *dv = ctx->stl_in.as<double>();
-        uint32_t *dt = (uint32_t *)(ctx->stl_in.as<char>() + align_up(nv * 24, 16));
-        if (nv) HIP_TRY(hipMemcpyAsync(dv, verts, nv * 24, hipMemcpyHostToDevice, ctx->stream));
-        if (nt) HIP_TRY(hipMemcpyAsync(dt, tris, nt * 12, hipMemcpyHostToDevice, ctx->stream));
-        const uint32_t *dp = nullptr;
-        if ((rc = group_order(ctx, dv, dt, nt, &dp))) return rc;
-        if (nt) HIP_TRY(hipMemcpyAsync(perm, dp, nt * 4, hipMemcpyDeviceToHost, ctx->stream));
-        HIP_TRY(hipStreamSynchronize(ctx->stream));
-        return MC3D_OK;
-    });
+    return group_host_arrays(ctx, verts, nv, tris, nt, perm, GROUP_ONE_SORT);
 }
 
 int mc3d_mesh_group_triangles(mc3d_ctx *ctx, mc3d_mesh *m) {
@@ -2887,6 +2895,36 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
         if (mismatches) *mismatches = nbad;
         return MC3D_OK;
     });
+}
+
+int mc3d_selftest_group_entries(uint32_t n, uint64_t grid, uint64_t *visited, uint64_t *misplaced) {
+    if (!visited || !misplaced || !grid) {
+        set_error("mc3d_selftest_group_entries: null argument");
+        return MC3D_E_INVALID_ARG;
+    }
+    *visited = *misplaced = 0;
+    for (uint64_t first : {(uint64_t)0, grid / 2, grid - 1}) {
+        uint64_t at = first;
+        each_order_entry(n, first, grid, [&](int a, uint32_t p) {
+            *misplaced += p >= n || a > 2 || (uint64_t)a * n + p != at;
+            ++*visited, at += grid;
+        });
+    }
+    return MC3D_OK;
+}
+
+int mc3d_selftest_group_sorts(mc3d_ctx *ctx, const double *verts, size_t nv, const uint32_t *tris, size_t nt,
+                              uint32_t *perm) {
+    if (!ctx || !verts || !tris || !perm) {
+        set_error("mc3d_selftest_group_sorts: null argument");
+        return MC3D_E_INVALID_ARG;
+    }
+    for (size_t i = 0; i < 3 * nt; i++)
+        if (tris[i] >= nv) {
+            set_error("mc3d_selftest_group_sorts: vertex index out of range");
+            return MC3D_E_INVALID_ARG;
+        }
+    return group_host_arrays(ctx, verts, nv, tris, nt, perm, 0);
 }
 
 int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_t *open, uint64_t *mismatches) {

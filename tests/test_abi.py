@@ -149,3 +149,18 @@ def test_row_bounds_match_contains_at_every_scale():
         assert checked.value > 500000 * 32
         assert bad.value == 0
         assert opened.value < checked.value // 2
+
+
+def test_group_entries_past_32_bits():
+    """GroupTriangles takes up to 2^31 - 1 triangles; the 3 n entries of its
+    orders need more than 32 bits from 2^32 / 3 on.  The kernels' walk, on the
+    host: every thread's share, each entry at its axis and position."""
+    import ctypes
+
+    L = _lib.lib()
+    grid = 8192 * 256
+    visited, misplaced = ctypes.c_uint64(), ctypes.c_uint64()
+    for n in (1, 2, 1000, 2**32 // 6, 2**32 // 3, 2**32 // 3 + 1, 2**31 - 1):
+        assert L.mc3d_selftest_group_entries(n, grid, ctypes.byref(visited), ctypes.byref(misplaced)) == 0
+        assert visited.value == sum(len(range(first, 3 * n, grid)) for first in (0, grid // 2, grid - 1)), n
+        assert misplaced.value == 0, n
