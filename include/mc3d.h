@@ -350,9 +350,10 @@ int mc3d_diag_stream(mc3d_ctx *ctx, size_t bytes, int32_t write, double *ms);
 int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked, uint64_t *mismatches);
 
 /* Diagnostics (host only, no GPU): random spheres, boxes, capsules and
- * cylinders (aligned, grazed, degenerate, far away, huge) on random lines of
- * corners and of edge midpoints -- every point that the row form of an atom
- * calls certainly inside or certainly outside is compared with the atom's
+ * cylinders (aligned, grazed, degenerate, far away, tiny, huge) on random
+ * lines of corners and of the midpoints of an edge's brackets -- every point
+ * that the row form of an atom calls certainly inside or certainly outside,
+ * with the tolerances that the kernels give it, is compared with the atom's
  * float64 Contains; differing points are counted (must be 0), and the points
  * it leaves open.  No counterpart in the reference; it checks the interval
  * bounds the corner and bisection kernels decide whole rows by. */

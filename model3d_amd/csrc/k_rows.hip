@@ -117,20 +117,11 @@ __device__ __forceinline__ uint64_t bracket_bits(CodeP code, uint32_t n, F64P f6
                                                  double z, int levels, uint64_t *stack) {
     const int k = ax.k;
     const double scale = (double)(1 << levels) * recip(hi - lo);
-    // (the points' rounding, in steps between them)
-    const double mag = row_scale(g).mag, eta = 1e-6 + 1e-15 * mag * scale;
+    const double mag = row_scale(g).mag, eta = bracket_eta(mag, scale);
     const int last = (1 << levels) - 1;
     return row_program<UNI, uint64_t>(code, n, f64, ax, k == 0 ? lo : x, k == 1 ? lo : y, k == 2 ? lo : z, hi - lo, mag,
-                                      scale, eta, last, ~1ull, stack, 256, [&](int i) {
-                                          double a = lo, b = hi, m = lo;
-                                          for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
-                                              m = (a + b) / 2;
-                                              if (at + bit == i) break;
-                                              if (i > at + bit) a = m, at += bit;
-                                              else b = m;
-                                          }
-                                          return m;
-                                      });
+                                      scale, eta, last, ~1ull, stack, 256,
+                                      [&](int i) { return bracket_point(lo, hi, levels, i); });
 }
 
 // mcSearchPoint (mc.go:223-258) of one vertex: up to six halvings are

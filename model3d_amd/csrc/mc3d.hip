@@ -588,8 +588,7 @@ int layout_job(Job &j, const mc3d_options &o, bool check) {
     RowScale &rs = j.scale;
     rs = RowScale{j.delta, 1 / j.delta, 0, 0};
     for (int a = 0; a < 3; a++) rs.mag = std::max({rs.mag, fabs(j.ax[a].front()), fabs(j.ax[a].back())});
-    // 64 additions of delta, each rounded to half an ulp of the coordinate
-    rs.eta = 1e-6 + 1e-11 * rs.mag * rs.inv_h;
+    rs.eta = row_eta(rs.mag, rs.inv_h);
     if (check && j.nwords >= (1ull << 32)) {
         set_error("grid too large: more than 2^32 occupancy words");
         return MC3D_E_UNSUPPORTED;
@@ -2990,20 +2989,18 @@ int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_
             double pts[64];
             int last = 63;
             double scale = 1 / h, smax = 64 * h, mag = 0;
-            if (edge) {  // the 32 dyadic points of one edge, as halvings reach them
-                const double t1 = p[k] + h;
-                last = 31, scale = 32 / (t1 - p[k]), smax = t1 - p[k];
-                pts[0] = p[k];
-                for (int i = 1; i < 32; i++) {
-                    double f = p[k], t = t1, m = 0;
-                    for (int bit = 16, at = 0; bit; bit >>= 1) {
-                        m = (f + t) / 2;
-                        if (at + bit == i) break;
-                        if (i > at + bit) f = m, at += bit;
-                        else t = m;
-                    }
-                    pts[i] = m;
+            if (edge) {  // a bracket of 3 to 6 levels, up to 45 halvings down an edge
+                const int levels = 3 + (int)(next() % 4);
+                double f = p[k], t = p[k] + h;
+                for (int n = next() & 1 ? (int)(next() % 46) : 0; n > 0; n--) {
+                    const double m = (f + t) / 2;
+                    if (next() & 1) f = m;
+                    else t = m;
                 }
+                p[k] = f;
+                last = (1 << levels) - 1, scale = (1 << levels) / (t - f), smax = t - f;
+                pts[0] = f;
+                for (int i = 1; i <= last; i++) pts[i] = bracket_point(f, t, levels, i);
             } else {
                 double x = p[k];
                 for (int i = 0; i < 64; i++, x += h) pts[i] = x;
@@ -3013,7 +3010,7 @@ int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_
             uint64_t sure, maybe;
             const Span sp = k == 0 && (next() & 1) ? atom_span(kind, a, LineAxis<true>(0), p[0], p[1], p[2], smax, mag)
                                                    : atom_span(kind, a, LineAxis<false>(k), p[0], p[1], p[2], smax, mag);
-            row_mask(sp, scale, 1e-6 + 1e-11 * mag / h, last, sure, maybe);
+            row_mask(sp, scale, edge ? bracket_eta(mag, scale) : row_eta(mag, scale), last, sure, maybe);
             for (int i = 0; i <= last; i++) {
                 p[k] = pts[i];
                 const bool in = atom64(kind, a, p[0], p[1], p[2]), yes = sure >> i & 1, may = maybe >> i & 1;

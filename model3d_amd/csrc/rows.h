@@ -199,6 +199,23 @@ MC3D_HD inline void row_mask(const Span &s, double scale, double eta, int last, 
     sure = c <= 63 ? bit_range(c, d) & maybe : 0;
 }
 
+// How far the points of a row (64 additions of h, each rounded) and of a bracket
+// (halvings, scale steps a unit) stray from even spacing, in steps.
+MC3D_HD inline double row_eta(double mag, double inv_h) { return 1e-6 + 1e-11 * mag * inv_h; }
+MC3D_HD inline double bracket_eta(double mag, double scale) { return 1e-6 + 1e-15 * mag * scale; }
+
+// The point i / 2^levels of the bracket [a, b], as halvings reach it.
+MC3D_HD inline double bracket_point(double a, double b, int levels, int i) {
+    double m = a;
+    for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
+        m = (a + b) / 2;
+        if (at + bit == i) break;
+        if (i > at + bit) a = m, at += bit;
+        else b = m;
+    }
+    return m;
+}
+
 // The atom's mask over the points: sure ones, and those of the rest at
 // which atom64 is true (point(i): the i-th point's coordinate along axis k).
 // Only the points of `want` matter.

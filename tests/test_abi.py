@@ -164,3 +164,15 @@ def test_group_entries_past_32_bits():
         assert L.mc3d_selftest_group_entries(n, grid, ctypes.byref(visited), ctypes.byref(misplaced)) == 0
         assert visited.value == sum(len(range(first, 3 * n, grid)) for first in (0, grid // 2, grid - 1)), n
         assert misplaced.value == 0, n
+
+
+def test_row_bounds_with_the_kernels_tolerances():
+    """Brackets of 3 to 6 levels, whole edges and up to 45 halvings down one,
+    by the tolerance that the bisection itself takes for its points."""
+    import ctypes
+
+    L = _lib.lib()
+    checked, opened, bad = ctypes.c_uint64(), ctypes.c_uint64(), ctypes.c_uint64()
+    assert L.mc3d_selftest_rows(91, 1000000, ctypes.byref(checked), ctypes.byref(opened), ctypes.byref(bad)) == 0
+    assert checked.value > 1000000 * 32
+    assert bad.value == 0
