@@ -439,6 +439,7 @@ struct ColliderCache {
     std::shared_ptr<const ColliderData> keep;
     double R = 0;  // radius of its sphere queries (0: none)
     DevBuf rec, start, tris, srec, sstart, stris, forms, pstart, plist;
+    bool planes = false;  // collider_planes has been asked
     DevCollider dev{};
 };
 
@@ -640,6 +641,16 @@ int prepare_job(Job &j, const mc3d_options &o, bool check = true) {
     return layout_job(j, o, check);
 }
 
+// Rows of corners instead of point lookups for a collider of this cell size: a
+// wave reads its bin's whole list for a row, and an edge's halvings read the
+// lists of every cell that it crosses, so rows where the grid is not much
+// coarser than the mesh.  Measured (a mesh made at spacing 0.02 / 0.05, whole
+// calls by points and by rows): edges of about 42 cells 124 and 213 us, 17
+// cells 133 and 149 us, 12 cells 334 and 207 us, 8 cells 262 and 124 us.
+bool ray_rows_pay(const RowScale &rs, double inv_cell) {
+    return rs.h > 0 && rs.eta < 0.01 && std::isfinite(rs.inv_h) && rs.h * inv_cell < 14;
+}
+
 // The collider's triangles by planes, for rows of corners (k_rays.hip); none
 // where triangles are too large or lists would be longer than 64 entries a
 // triangle.
@@ -687,11 +698,20 @@ int collider_planes(mc3d_ctx *ctx, const ColliderData &cd, ColliderCache &c) {
 }
 
 // The device copy of a collider's ray grid and, for sphere queries of
-// radius R, its sphere grid (uploaded once per context).
-int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> &cd, double R, DevCollider &out,
-                       size_t keep_at_least) {
+// radius R, its sphere grid (uploaded once per context).  rows: the spacing of a
+// search of this collider alone (else null), whose rows may want its planes:
+// they are added once, by the first search that does.
+int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> &cd, double R, const RowScale *rows,
+                       DevCollider &out, size_t keep_at_least) {
+    int rc;
+    auto planes = [&](ColliderCache &c) -> int {
+        if (c.planes || !rows || !ray_rows_pay(*rows, c.dev.inv_cell)) return MC3D_OK;
+        c.planes = true;
+        return collider_planes(ctx, *cd, c);
+    };
     for (size_t i = 0; i < ctx->colliders.size(); i++) {
         if (ctx->colliders[i]->keep->id == cd->id && ctx->colliders[i]->R == R) {
+            if ((rc = planes(*ctx->colliders[i]))) return rc;
             out = ctx->colliders[i]->dev;
             std::unique_ptr<ColliderCache> hit = std::move(ctx->colliders[i]);  // now the most recent
             ctx->colliders.erase(ctx->colliders.begin() + i);
@@ -703,7 +723,6 @@ int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> 
     std::unique_ptr<ColliderCache> c(new ColliderCache);
     c->keep = cd;
     c->R = R;
-    int rc;
     if ((rc = c->rec.ensure(G.rec.size() * sizeof(double) + 8)) ||
         (rc = c->start.ensure(G.cell_start.size() * sizeof(uint32_t) + 8)) ||
         (rc = c->tris.ensure(G.cell_tris.size() * sizeof(uint32_t) + 8)))
@@ -722,7 +741,7 @@ int collider_on_device(mc3d_ctx *ctx, const std::shared_ptr<const ColliderData> 
     d.srec = nullptr, d.scell_start = d.scell_tris = nullptr;
     d.so[0] = d.so[1] = d.so[2] = 0, d.sinv = 1, d.sn[0] = d.sn[1] = d.sn[2] = 0, d.pad = 0;
     d.forms = nullptr, d.pstart = d.plist = nullptr, d.pentries = 0, d.mag = 0, d.planes = RayPlanes{};
-    if (R == 0 && (rc = collider_planes(ctx, *cd, *c))) return rc;
+    if ((rc = planes(*c))) return rc;
     if (R > 0) {
         const SphereGrid &S = cd->sphere_grid(R);
         if ((rc = c->srec.ensure(S.rec.size() * sizeof(double) + 8)) ||
@@ -999,7 +1018,7 @@ int upload_colliders(mc3d_ctx *ctx, const std::vector<Job> &jobs, Upload &U) {
     {
         const Program &P = jobs[0].low->P;
         const Insn in = P.code[0];
-        U.collider_only = P.code.size() == 1 && insn_op(in.x) == OP_ATOM && insn_kind(in.x) == A_COLLIDER &&
+        U.collider_only = n == 1 && P.code.size() == 1 && insn_op(in.x) == OP_ATOM && insn_kind(in.x) == A_COLLIDER &&
                           insn_frame(in.x) == 0 && P.f64[in.y + 7] == 0 && P.f64[in.y + 8] == 0;
         U.scale = jobs[0].scale;
         U.row_corners = (uint32_t)jobs[0].g.nx;
@@ -1011,7 +1030,8 @@ int upload_colliders(mc3d_ctx *ctx, const std::vector<Job> &jobs, Upload &U) {
         const Program &P = jobs[s].low->P;
         U.cols[s].resize(P.colliders.size());
         for (size_t i = 0; i < U.cols[s].size(); i++) {
-            int rc = collider_on_device(ctx, P.colliders[i], P.collider_R[i], U.cols[s][i], ncol);
+            int rc = collider_on_device(ctx, P.colliders[i], P.collider_R[i], U.collider_only ? &U.scale : nullptr,
+                                        U.cols[s][i], ncol);
             if (rc) return rc;
         }
     }
@@ -1221,14 +1241,8 @@ int collider_rows(const Upload &U) {
     if (U.cols.size() != 1 || U.cols[0].size() != 1 || !U.cols[0][0].forms || !U.collider_only) return 0;
     const RayPlanes &P = U.cols[0][0].planes;
     const RowScale &rs = U.scale;
-    if (!(rs.eta < 0.01) || !std::isfinite(rs.inv_h)) return 0;
-    // A wave reads its bin's whole list for a row, and an edge's halvings read
-    // the lists of every cell that it crosses: rows where the grid is not much
-    // coarser than the mesh.  Measured (a mesh made at spacing 0.02 / 0.05, whole
-    // calls by points and by rows): edges of about 42 cells 124 and 213 us, 17
-    // cells 133 and 149 us, 12 cells 334 and 207 us, 8 cells 262 and 124 us.
     const DevCollider &C = U.cols[0][0];
-    if (!(rs.h * C.inv_cell < 14) || C.pentries > 256ull * P.bins * U.row_corners) return 0;
+    if (!ray_rows_pay(rs, C.inv_cell) || C.pentries > 256ull * P.bins * U.row_corners) return 0;
     for (int rows = RAY_ROWS; rows > 1; rows /= 2)
         if ((rows - 1) * P.nz * rs.h < 0.999 * P.width) return rows;
     return 1;

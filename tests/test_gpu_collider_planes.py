@@ -1,0 +1,45 @@
+"""A mesh collider's triangles by planes: made for a search that decides its
+rows by them, and not before."""
+import numpy as np
+import pytest
+import torch
+
+import model3d_amd as m3
+from oracle.binding import oracle_search
+from tests.helpers import same_triangles
+
+pytestmark = pytest.mark.gpu
+
+
+def _free():
+    torch.cuda.synchronize()
+    return torch.cuda.mem_get_info()[0]
+
+
+def test_planes_only_for_rows():
+    """50 k triangles (6 MB of linear forms): a tree that holds the collider
+    and a grid of long edges look up points; the planes come with the
+    collider's own search, and its mesh is the oracle's all along."""
+    mesh = m3.MarchingCubesSearch(m3.Sphere((0.03, -0.02, 0.01), 1.0), 0.0274, 4)
+    n = len(mesh.faces)
+    col = m3.NewColliderSolid(m3.MeshToCollider(mesh))
+    tree = m3.JoinedSolid([col, m3.Sphere((0.9, 0.0, 0.0), 0.3)])
+    print(f"collider of {n} triangles", flush=True)
+    assert n > 48_000
+    d = 0.08
+    want_tree, _ = oracle_search(tree, d, 3, threads=8)
+    want, _ = oracle_search(col, d, 3, threads=8)
+    # the row kernels on another collider (their code, a graph's memory), then
+    # all that this one is asked before its own search
+    box = m3.NewColliderSolid(m3.MeshToCollider(m3.NewMeshRect((0, 0, 0), (1, 1, 1))))
+    m3.MarchingCubesSearch(box, d, 3)
+    for _ in range(2):
+        assert same_triangles(m3.MarchingCubesSearch(tree, d, 3).triangles(), want_tree)
+        m3.MarchingCubesSearch(col, 0.3, 0)
+    before = _free()
+    assert same_triangles(m3.MarchingCubesSearch(col, d, 3).triangles(), want)
+    planes = before - _free()
+    print(f"planes {planes} bytes", flush=True)
+    assert planes >= 128 * n
+    assert same_triangles(m3.MarchingCubesSearch(tree, d, 3).triangles(), want_tree)
+    assert same_triangles(m3.MarchingCubesSearch(col, d, 3).triangles(), want)
