@@ -369,6 +369,10 @@ int mc3d_selftest_group_entries(uint32_t n, uint64_t grid, uint64_t *visited, ui
 int mc3d_selftest_group_sorts(mc3d_ctx *ctx, const double *verts, size_t nv, const uint32_t *tris, size_t nt,
                               uint32_t *perm);
 
+/* Diagnostics: device allocations of more than `bytes` made by this thread's
+ * calls fail as they do on a full device (0: none do). */
+void mc3d_selftest_alloc_cap(size_t bytes);
+
 const char *mc3d_last_error(void);
 const char *mc3d_version(void);
 

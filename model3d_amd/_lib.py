@@ -204,6 +204,7 @@ SIGNATURES = {
     "mc3d_selftest_group_sorts": (
         ctypes.c_int, [_P, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p, ctypes.c_size_t, ctypes.c_void_p]
     ),
+    "mc3d_selftest_alloc_cap": (None, [ctypes.c_size_t]),
     "mc3d_last_error": (ctypes.c_char_p, []),
     "mc3d_version": (ctypes.c_char_p, []),
 }

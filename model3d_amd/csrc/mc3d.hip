@@ -138,6 +138,9 @@ int guarded(F &&f) {
     }
 }
 
+// The largest device allocation this thread may make (mc3d_selftest_alloc_cap).
+thread_local size_t t_alloc_cap = SIZE_MAX;
+
 // Grow-only device buffer.
 struct DevBuf {
     void *p = nullptr;
@@ -145,23 +148,25 @@ struct DevBuf {
     DevBuf() = default;
     DevBuf(const DevBuf &) = delete;
     DevBuf &operator=(const DevBuf &) = delete;
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
-    }
+    ~DevBuf() { release(); }
     int ensure(size_t bytes) {
         if (bytes <= cap) return MC3D_OK;
-        if (p) (void)hipFree(p);
-        p = nullptr;
-        cap = 0;
+        release();
         const size_t want = bytes + bytes / 4 + 4096;
-        hipError_t e = hipMalloc(&p, want);
+        hipError_t e = want > t_alloc_cap ? hipErrorOutOfMemory : hipMalloc(&p, want);
         if (e != hipSuccess) {
             p = nullptr;
+            (void)hipGetLastError();  // (not the next launch's)
             set_error(std::string("hipMalloc: ") + hipGetErrorString(e));
             return MC3D_E_OOM;
         }
         cap = want;
         return MC3D_OK;
+    }
+    void release() {
+        if (p) (void)hipFree(p);
+        p = nullptr;
+        cap = 0;
     }
     template <class T>
     T *as() const {
@@ -652,9 +657,9 @@ bool ray_rows_pay(const RowScale &rs, double inv_cell) {
 }
 
 // The collider's triangles by planes, for rows of corners (k_rays.hip); none
-// where triangles are too large or lists would be longer than 64 entries a
-// triangle.
-int collider_planes(mc3d_ctx *ctx, const ColliderData &cd, ColliderCache &c) {
+// (c.dev.forms stays null) where triangles are too large or lists would be
+// longer than 64 entries a triangle.
+int build_planes(mc3d_ctx *ctx, const ColliderData &cd, ColliderCache &c) {
     DevCollider &d = c.dev;
     const size_t n = cd.ray_grid().rec.size() / RAY_REC;
     if (n == 0 || n >= (1u << 28)) return MC3D_OK;
@@ -695,6 +700,14 @@ int collider_planes(mc3d_ctx *ctx, const ColliderData &cd, ColliderCache &c) {
     d.pstart = c.pstart.as<uint32_t>(), d.plist = c.plist.as<uint32_t>();
     d.pentries = got[2], d.mag = mag, d.planes = P;
     return MC3D_OK;
+}
+
+// The planes where they fit: without the memory for them, as without the
+// planes themselves, a collider's corners are looked up point by point.
+int collider_planes(mc3d_ctx *ctx, const ColliderData &cd, ColliderCache &c) {
+    const int rc = build_planes(ctx, cd, c);
+    if (!c.dev.forms) c.forms.release(), c.pstart.release(), c.plist.release();
+    return rc == MC3D_E_OOM ? MC3D_OK : rc;
 }
 
 // The device copy of a collider's ray grid and, for sphere queries of
@@ -2909,6 +2922,8 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
         return MC3D_OK;
     });
 }
+
+void mc3d_selftest_alloc_cap(size_t bytes) { t_alloc_cap = bytes ? bytes : SIZE_MAX; }
 
 int mc3d_selftest_group_entries(uint32_t n, uint64_t grid, uint64_t *visited, uint64_t *misplaced) {
     if (!visited || !misplaced || !grid) {

@@ -5,6 +5,7 @@ import pytest
 import torch
 
 import model3d_amd as m3
+from model3d_amd import _lib
 from oracle.binding import oracle_search
 from tests.helpers import same_triangles
 
@@ -43,3 +44,27 @@ def test_planes_only_for_rows():
     assert planes >= 128 * n
     assert same_triangles(m3.MarchingCubesSearch(tree, d, 3).triangles(), want_tree)
     assert same_triangles(m3.MarchingCubesSearch(col, d, 3).triangles(), want)
+
+
+@pytest.mark.parametrize("per_triangle", [112, 1000])
+def test_planes_without_memory(per_triangle):
+    """Where the planes do not fit (the forms, 128 bytes a triangle; their
+    records, 104, do) the search looks its corners up: the same mesh, and no
+    error of that allocation left for the calls after it."""
+    mesh = m3.MarchingCubesSearch(m3.Sphere((0.01, 0.02, -0.04), 1.0), 0.0134, 4)
+    n = len(mesh.faces)
+    with_planes = m3.NewColliderSolid(m3.MeshToCollider(mesh))
+    without = m3.NewColliderSolid(m3.MeshToCollider(mesh))
+    print(f"collider of {n} triangles, {per_triangle} bytes a triangle", flush=True)
+    d = 0.04
+    want = m3.MarchingCubesSearch(with_planes, d, 6)
+    L = _lib.lib()
+    L.mc3d_selftest_alloc_cap(per_triangle * n * 5 // 4 + 4096)
+    try:
+        got = m3.MarchingCubesSearch(without, d, 6)
+    finally:
+        L.mc3d_selftest_alloc_cap(0)
+    assert np.array_equal(got.vertices, want.vertices) and np.array_equal(got.faces, want.faces)
+    for c in (without, with_planes):
+        got = m3.MarchingCubesSearch(c, d, 6)
+        assert np.array_equal(got.vertices, want.vertices) and np.array_equal(got.faces, want.faces)
