@@ -359,6 +359,13 @@ int mc3d_selftest_plan_fold(uint64_t seed, uint32_t programs, uint64_t *checked,
  * bounds the corner and bisection kernels decide whole rows by. */
 int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_t *open, uint64_t *mismatches);
 
+/* Diagnostics (host only, no GPU): what the row form of one atom (a sphere, box,
+ * capsule or cylinder solid) says of points on a line along an axis: bit i of
+ * *sure, certainly inside, and of *maybe, not certainly outside, for the 64
+ * corners p + i h (levels 0) or the points that `levels` halvings of the edge
+ * from p to p + h reach; *inside has the atom's Contains. */
+int mc3d_selftest_line(const mc3d_solid *s, const double p[3], int32_t axis, double h, int32_t levels, uint64_t *sure,
+                       uint64_t *maybe, uint64_t *inside);
 /* Diagnostics (host only, no GPU): the entries of GroupTriangles' three
  * orders of n triangles as three threads of a grid of that many walk them
  * (the first, the middle and the last); *visited of them, *misplaced not at

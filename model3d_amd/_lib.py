@@ -198,6 +198,10 @@ SIGNATURES = {
     "mc3d_selftest_rows": (
         ctypes.c_int, [ctypes.c_uint64, ctypes.c_uint32] + [ctypes.POINTER(ctypes.c_uint64)] * 3
     ),
+    "mc3d_selftest_line": (
+        ctypes.c_int,
+        [_P, _dp, ctypes.c_int32, ctypes.c_double, ctypes.c_int32] + [ctypes.POINTER(ctypes.c_uint64)] * 3,
+    ),
     "mc3d_selftest_group_entries": (
         ctypes.c_int, [ctypes.c_uint32, ctypes.c_uint64, ctypes.POINTER(ctypes.c_uint64), ctypes.POINTER(ctypes.c_uint64)]
     ),

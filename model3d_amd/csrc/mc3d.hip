@@ -2639,6 +2639,36 @@ int encode_stl_device(mc3d_ctx *ctx, const double *verts, const uint32_t *tris, 
     parallel_copy(out + 84, ctx->outstage.p, body);
     return MC3D_OK;
 }
+// What the row form of an atom (kind, params a) says of points on the line
+// through p along axis k -- a row's 64 corners h apart (levels 0), or the dyadic
+// points of the bracket from p[k] to t -- and its Contains at each.
+struct HostRow {
+    uint64_t sure, maybe, inside;
+    int last;
+};
+HostRow host_row(uint32_t kind, const double *a, int k, const double *p, double t, double h, int levels, bool x_axis) {
+    HostRow r{0, 0, 0, levels ? (1 << levels) - 1 : 63};
+    double q[3] = {p[0], p[1], p[2]}, pts[64];
+    double scale = 1 / h, smax = 64 * h, mag = 0;
+    if (levels) {
+        scale = (1 << levels) / (t - p[k]), smax = t - p[k];
+        for (int i = 0; i <= r.last; i++) pts[i] = i ? bracket_point(p[k], t, levels, i) : p[k];
+    } else {
+        double x = p[k];
+        for (int i = 0; i < 64; i++, x += h) pts[i] = x;
+    }
+    for (int a2 = 0; a2 < 3; a2++) mag = std::max(mag, fabs(p[a2]));
+    mag = std::max(mag, fabs(pts[r.last]));
+    const Span sp = k == 0 && x_axis ? atom_span(kind, a, LineAxis<true>(0), p[0], p[1], p[2], smax, mag)
+                                     : atom_span(kind, a, LineAxis<false>(k), p[0], p[1], p[2], smax, mag);
+    row_mask(sp, scale, levels ? bracket_eta(mag, scale) : row_eta(mag, scale), r.last, r.sure, r.maybe);
+    for (int i = 0; i <= r.last; i++) {
+        q[k] = pts[i];
+        r.inside |= (uint64_t)atom64(kind, a, q[0], q[1], q[2]) << i;
+    }
+    return r;
+}
+
 }  // namespace
 
 extern "C" {
@@ -2955,6 +2985,25 @@ int mc3d_selftest_group_sorts(mc3d_ctx *ctx, const double *verts, size_t nv, con
     return group_host_arrays(ctx, verts, nv, tris, nt, perm, 0);
 }
 
+int mc3d_selftest_line(const mc3d_solid *s, const double p[3], int32_t axis, double h, int32_t levels, uint64_t *sure,
+                       uint64_t *maybe, uint64_t *inside) {
+    if (!s || !p || !sure || !maybe || !inside || axis < 0 || axis > 2 || !(h > 0) || levels < 0 || levels > 6) {
+        set_error("mc3d_selftest_line: invalid argument");
+        return MC3D_E_INVALID_ARG;
+    }
+    return guarded([&]() -> int {
+        Program P;
+        std::string msg;
+        if (!lower_solid(*s->ptr, P, msg) || P.code.size() != 1 || insn_op(P.code[0].x) != OP_ATOM || insn_frame(P.code[0].x)) {
+            set_error("mc3d_selftest_line: not a single atom");
+            return MC3D_E_UNSUPPORTED;
+        }
+        const HostRow r = host_row(insn_kind(P.code[0].x), P.f64.data() + P.code[0].y, axis, p, p[axis] + h, h, levels, true);
+        *sure = r.sure, *maybe = r.maybe, *inside = r.inside;
+        return MC3D_OK;
+    });
+}
+
 int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_t *open, uint64_t *mismatches) {
     for (uint64_t *p : {checked, open, mismatches})
         if (p) *p = 0;
@@ -3014,39 +3063,22 @@ int mc3d_selftest_rows(uint64_t seed, uint32_t lines, uint64_t *checked, uint64_
             }
             if (next() % 4 == 0) p[k] = (next() & 1 ? lo[k] : hi[k]) - (double)(next() % 60) * h;
             else p[k] -= uni(0, 64) * h;
-            const bool edge = next() & 1;
-            double pts[64];
-            int last = 63;
-            double scale = 1 / h, smax = 64 * h, mag = 0;
-            if (edge) {  // a bracket of 3 to 6 levels, up to 45 halvings down an edge
-                const int levels = 3 + (int)(next() % 4);
-                double f = p[k], t = p[k] + h;
+            int levels = 0;
+            double f = p[k], t = p[k] + h;
+            if (next() & 1) {  // a bracket of 3 to 6 levels, up to 45 halvings down an edge
+                levels = 3 + (int)(next() % 4);
                 for (int n = next() & 1 ? (int)(next() % 46) : 0; n > 0; n--) {
                     const double m = (f + t) / 2;
                     if (next() & 1) f = m;
                     else t = m;
                 }
                 p[k] = f;
-                last = (1 << levels) - 1, scale = (1 << levels) / (t - f), smax = t - f;
-                pts[0] = f;
-                for (int i = 1; i <= last; i++) pts[i] = bracket_point(f, t, levels, i);
-            } else {
-                double x = p[k];
-                for (int i = 0; i < 64; i++, x += h) pts[i] = x;
             }
-            for (int q = 0; q < 3; q++) mag = std::max(mag, fabs(p[q]));
-            mag = std::max(mag, fabs(pts[last]));
-            uint64_t sure, maybe;
-            const Span sp = k == 0 && (next() & 1) ? atom_span(kind, a, LineAxis<true>(0), p[0], p[1], p[2], smax, mag)
-                                                   : atom_span(kind, a, LineAxis<false>(k), p[0], p[1], p[2], smax, mag);
-            row_mask(sp, scale, edge ? bracket_eta(mag, scale) : row_eta(mag, scale), last, sure, maybe);
-            for (int i = 0; i <= last; i++) {
-                p[k] = pts[i];
-                const bool in = atom64(kind, a, p[0], p[1], p[2]), yes = sure >> i & 1, may = maybe >> i & 1;
-                nchecked++;
-                nopen += may && !yes;
-                nbad += (yes && !in) || (!may && in);
-            }
+            const HostRow row = host_row(kind, a, k, p, t, h, levels, next() & 1);
+            const uint64_t all = ~0ull >> (63 - row.last);
+            nchecked += row.last + 1;
+            nopen += __builtin_popcountll(row.maybe & ~row.sure & all);
+            nbad += __builtin_popcountll(((row.sure & ~row.inside) | (~row.maybe & row.inside)) & all);
         }
         if (checked) *checked = nchecked;
         if (open) *open = nopen;

@@ -106,7 +106,7 @@ MC3D_HD inline Span sphere_span(const LineAxis<KX> &ax, double dx, double dy, do
 template <bool KX>
 MC3D_HD inline Span cylinder_span(const LineAxis<KX> &ax, double vx, double vy, double vz, double dx, double dy, double dz,
                                   double L, double T, double smax, double M) {
-    const double c = __builtin_fma(vz, dz, __builtin_fma(vy, dy, vx * dx));
+    const double c = vx * dx + vy * dy + vz * dz;  // (atom64's own sum)
     const double nx = __builtin_fma(-dx, c, vx), ny = __builtin_fma(-dy, c, vy), nz = __builtin_fma(-dz, c, vz);
     const double nk = ax.along(nx, ny, nz), dk = ax.along(dx, dy, dz), A = ax.across2(dx, dy, dz);
     const double w = T - __builtin_fma(nz, nz, __builtin_fma(ny, ny, nx * nx)), D = 1e-13 * M * M;
@@ -125,7 +125,12 @@ MC3D_HD inline Span cylinder_span(const LineAxis<KX> &ax, double vx, double vy, 
         if (ri > 0) s.ai = (-nk - ri) * iA + e, s.bi = (-nk + ri) * iA - e;
     }
     const double f = 1e-13 * M;  // rounding of the position along the axis
-    if (fabs(dk) < 1e-7) {
+    if (dk == 0) {
+        // Across the axis every point has this same sum, bit for bit (its k
+        // term is a zero).  End faces mostly lie in planes of the grid, where
+        // a margin would leave whole rows and edges open.
+        if (c < 0 || c > L) return span_none();
+    } else if (fabs(dk) < 1e-7) {
         const double f2 = f + fabs(dk) * smax;
         if (c < -f2 || c > L + f2) return span_none();
         if (!(c > f2 && c < L - f2)) s.ai = INFINITY, s.bi = -INFINITY;
