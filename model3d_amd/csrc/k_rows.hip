@@ -20,15 +20,31 @@
 namespace mc3d {
 namespace {
 
-// The corners of one word (from x0, in row (y, z)) that a program holds for.
+// The corners of one word (from x0, in row (y, z)) that a program holds for,
+// each lane its own word (live: it has one).  A word with more than a few open
+// corners is taken by the whole wave, a lane a corner: one lane after another's
+// 64 evaluations is what a wave would wait for (a row along a cylinder's side).
 template <bool UNI, class CodeP, class F64P>
 __device__ __forceinline__ uint64_t word_bits(CodeP code, uint32_t n, F64P f64, const Grid &g, int x0, int y, int z,
-                                              uint64_t *stack) {
+                                              bool live, uint64_t *stack) {
     const RowScale rs = row_scale(g);
-    const int last = min(63, g.nx - 1 - x0);
+    const int lane = threadIdx.x & 63, last = min(63, g.nx - 1 - x0);
     const double *xs = g.xs + x0;
-    const uint64_t m = row_program<UNI, uint64_t>(code, n, f64, LineAxis<true>(0), xs[0], g.ys[y], g.zs[z], 64 * rs.h, rs.mag,
-                                                  rs.inv_h, rs.eta, last, ~0ull, stack, 64, [&](int i) { return xs[i]; });
+    const double py = g.ys[y], pz = g.zs[z];
+    const LineAxis<true> ax(0);
+    auto rest = [&](uint32_t kind, auto a, uint64_t open) {
+        if (__ballot(open != 0) == 0) return (uint64_t)0;
+        uint64_t in = 0;
+        for (uint64_t many = __ballot(__popcll(open) > FEW_OPEN); many; many &= many - 1) {
+            const int j = __ffsll((unsigned long long)many) - 1;
+            const double x = g.xs[min(__shfl(x0, j) + lane, g.nx - 1)];
+            const uint64_t m = __ballot(atom64(kind, a, x, __shfl(py, j), __shfl(pz, j)));
+            if (lane == j) in = m & open, open = 0;
+        }
+        return in | open_points(kind, a, ax, 0, py, pz, open, [&](int i) { return xs[i]; });
+    };
+    const uint64_t m = row_program<UNI, uint64_t>(code, n, f64, ax, xs[0], py, pz, 64 * rs.h, rs.mag, rs.inv_h, rs.eta, last,
+                                                  live ? ~0ull : 0ull, stack, 64, rest);
     return m & (~0ull >> (63 - last));
 }
 
@@ -73,10 +89,12 @@ __global__ __launch_bounds__(256) void k_rows_act(const Seg *__restrict__ segs, 
         const uint2 bi = make_uint2((uint32_t)biw, (uint32_t)(biw >> 32));
         const auto code = scalar_ptr(brick_code(sg.P, B, bi));
         const int nrows = B.BY * B.BZ;
-        for (int j = lane; j < nrows; j += 64) {
-            const int jz = j / B.BY, y = by * B.BY + (j - jz * B.BY), z = bz * B.BZ + jz;
-            if (y >= g.ny || z >= g.nz) continue;
-            const uint64_t m = word_bits<true>(code, bi.y, scalar_ptr(sg.P.f64), g, bx * 64, y, z, stack);
+        for (int j0 = 0; j0 < nrows; j0 += 64) {
+            const int j = j0 + lane, jz = j / B.BY, y = by * B.BY + (j - jz * B.BY), z = bz * B.BZ + jz;
+            const bool live = j < nrows && y < g.ny && z < g.nz;
+            const uint64_t m = word_bits<true>(code, bi.y, scalar_ptr(sg.P.f64), g, bx * 64, min(y, g.ny - 1), min(z, g.nz - 1),
+                                               live, stack);
+            if (!live) continue;
             bits_all[sg.word0 + word_index(g, bx, y, z)] = m;
             check_faces(g, m, bx * 64, y, z, ctl, &sout[si]);
         }
@@ -92,52 +110,94 @@ __global__ __launch_bounds__(256) void k_rows_all(const Seg *__restrict__ segs, 
     extern __shared__ __align__(16) uint64_t row_stack[];
     uint64_t *stack = row_stack + (size_t)wave_id() * depth * 64 + (threadIdx.x & 63);
     // (word ranges are aligned to 64: a wave's words are one segment's)
-    for (uint64_t gw = (uint64_t)blockIdx.x * 256 + threadIdx.x; gw < nwords; gw += (uint64_t)gridDim.x * 256) {
+    for (uint64_t w0 = (uint64_t)blockIdx.x * 256 + wave_id() * 64; w0 < nwords; w0 += (uint64_t)gridDim.x * 256) {
+        const uint64_t gw = w0 + (threadIdx.x & 63);
         const uint32_t si = wave_seg<MULTI>(word_seg, gw, SEG_WORD_SHIFT);
         const Seg sg = pick_seg<MULTI>(segs, seg0, si);
         const Grid &g = sg.g;
         const uint64_t w = gw - sg.word0;
-        uint64_t m = 0;
-        if (w < sg.nwords) {  // else alignment padding
-            int wx, y, z;
-            word_coords(g, w, wx, y, z);
-            m = word_bits<true>(scalar_ptr(sg.P.code), sg.P.ncode, scalar_ptr(sg.P.f64), g, wx * 64, y, z, stack);
-            check_faces(g, m, wx * 64, y, z, ctl, &sout[si]);
-        }
-        bits[gw] = m;
+        const bool live = w < sg.nwords;  // else alignment padding
+        int wx, y, z;
+        word_coords(g, live ? w : 0, wx, y, z);
+        const uint64_t m = word_bits<true>(scalar_ptr(sg.P.code), sg.P.ncode, scalar_ptr(sg.P.f64), g, wx * 64, y, z, live, stack);
+        if (live) check_faces(g, m, wx * 64, y, z, ctl, &sout[si]);
+        if (gw < nwords) bits[gw] = live ? m : 0;
     }
 }
 
 // The program as a mask over the dyadic points of the bracket [lo, hi] on
 // axis k of the line through p: bit i is the point that halving the bracket
-// reaches at i / 2^levels.
+// reaches at i / 2^levels.  dense: an atom leaves more than a few points open,
+// and the mask says nothing.
 template <bool UNI, class CodeP, class F64P>
 __device__ __forceinline__ uint64_t bracket_bits(CodeP code, uint32_t n, F64P f64, const Grid &g,
                                                  const LineAxis<false> &ax, double lo, double hi, double x, double y,
-                                                 double z, int levels, uint64_t *stack) {
+                                                 double z, int levels, uint64_t *stack, bool &dense) {
     const int k = ax.k;
     const double scale = (double)(1 << levels) * recip(hi - lo);
     const double mag = row_scale(g).mag, eta = bracket_eta(mag, scale);
+    const double qx = k == 0 ? lo : x, qy = k == 1 ? lo : y, qz = k == 2 ? lo : z;
+    auto rest = [&](uint32_t kind, auto a, uint64_t open) -> uint64_t {
+        if (open == 0) return 0;
+        if (__popcll(open) > FEW_OPEN) {
+            dense = true;
+            return 0;
+        }
+        return open_points(kind, a, ax, qx, qy, qz, open, [&](int i) { return bracket_point(lo, hi, levels, i); });
+    };
     const int last = (1 << levels) - 1;
-    return row_program<UNI, uint64_t>(code, n, f64, ax, k == 0 ? lo : x, k == 1 ? lo : y, k == 2 ? lo : z, hi - lo, mag,
-                                      scale, eta, last, ~1ull, stack, 256,
-                                      [&](int i) { return bracket_point(lo, hi, levels, i); });
+    return row_program<UNI, uint64_t>(code, n, f64, ax, qx, qy, qz, hi - lo, mag, scale, eta, last, ~1ull, stack, 256, rest);
 }
 
-// mcSearchPoint (mc.go:223-258) of one vertex: up to six halvings are
-// decided at a time by the program's mask over the points they can reach,
-// the last one or two by evaluating it (a second mask costs more than two
-// evaluations, the last of three or more would not: 8 halvings as 6 + 2
-// took 31.6 -> 28.4 us, 573 -> 531 us against two masks).
+// `left` halvings of the bracket [lo, hi] of a vertex (mcSearchPoint, mc.go:
+// 223-258): up to six are decided at a time by the program's mask over the
+// points they can reach, the last one or two by evaluating it (a second mask
+// costs more than two evaluations, the last of three or more would not: 8
+// halvings as 6 + 2 took 31.6 -> 28.4 us, 573 -> 531 us against two masks).
+// Where an atom leaves more than a few of a bracket's points open -- its bounds
+// are no finer than the points after some 28 halvings, or far from the origin;
+// an edge may touch a cylinder's side -- the wave evaluates all further
+// halvings: deciding open points one by one is up to 63 evaluations for six
+// halvings (one sphere at 102^3 corners, 64 halvings, whole calls: 357 us so, 75
+// with the evaluations alone, 51 us for 8 halvings).
 //
-// Evaluating every halving is a chain of `iters` dependent program walks,
-// bound by the latency of its loads where few waves run (a small part) and by
-// the walks' scalar and vector issue where many do; one walk decides six
-// halvings here.  Bound by vector issue now (57% of the cycles at 4 waves per
-// SIMD; 115 registers).  Measured (kernel trace, MI355X, 8 halvings): 1,100
-// vertices 23 -> 12 us, 411k vertices of 64 primitives 43 -> 28 us (with the
-// float32 guard 64 -> 31 us), a batch of 32 solids 173 -> 103 us, 10.1M
-// vertices of 512 primitives 819 -> 531 us.
+// Evaluating every halving is a chain of dependent program walks, bound by the
+// latency of its loads where few waves run (a small part) and by the walks'
+// scalar and vector issue where many do; one walk decides six halvings here.
+// Bound by vector issue now, at 3 waves per SIMD (144 registers; 168 for several
+// solids).  UNI: one program for the wave.
+template <bool UNI>
+__device__ __forceinline__ void halve(const Insn *code, uint32_t n, const DevProg &P, const Grid &g, int k, double px, double py,
+                                      double pz, bool up, int left, double &lo, double &hi, uint64_t *stack) {
+    const LineAxis<false> ax(k);
+    bool dense = false;  // (then the wave halves on point by point)
+    while (left > 2 && __ballot(dense) == 0) {
+        const int levels = min(left, 6);
+        uint64_t m;
+        if constexpr (UNI) m = bracket_bits<true>(scalar_ptr(code), n, scalar_ptr(P.f64), g, ax, lo, hi, px, py, pz, levels, stack, dense);
+        else m = bracket_bits<false>(code, n, P.f64, g, ax, lo, hi, px, py, pz, levels, stack, dense);
+        if (dense) continue;
+        for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
+            const double mid = (lo + hi) / 2;
+            const bool in = (m >> (at + bit)) & 1;
+            if (in == up) hi = mid;  // the inside end moves
+            else lo = mid, at += bit;
+        }
+        left -= levels;
+    }
+    for (; left > 0; left--) {
+        const double mid = (lo + hi) / 2;
+        GStats gs;
+        const bool in = eval_code<0, false, UNI>(code, n, P, k == 0 ? mid : px, k == 1 ? mid : py, k == 2 ? mid : pz, gs);
+        if (in == up) hi = mid;
+        else lo = mid;
+    }
+}
+
+// One vertex.  Measured (kernel trace, MI355X, 8 halvings, against a walk for each
+// halving): 1,100 vertices 23 -> 12 us, 411k vertices of 64 primitives 43 -> 31 us
+// (with the float32 guard 64 -> 35 us), a batch of 32 solids 173 -> 109 us, 10.1M
+// vertices of 512 primitives 819 -> 670 us.
 __device__ __forceinline__ void bisect_rows(const Seg &sg, const uint64_t *__restrict__ bits_all, const uint64_t key,
                                             double *__restrict__ verts, double *__restrict__ interior, uint64_t v,
                                             uint64_t *stack) {
@@ -154,44 +214,16 @@ __device__ __forceinline__ void bisect_rows(const Seg &sg, const uint64_t *__res
     if (sg.iters > 0) {
         // the edge's brick program (an edge crossed in a brick that the plan
         // found constant is decided by that constant, as in bisect_vertex)
-        BrickProgram bp{P.code, P.ncode, -1};
-        if (B.info) {
-            const uint2 bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
-            bp = brick_program(P, B, bi.x, bi.y);
-        }
-        const uint64_t cp = (uint64_t)bp.code;
-        const uint64_t cp0 = (uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)cp) |
-                             ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(cp >> 32)) << 32);
-        const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)bp.n);
-        // one program for the wave: scalar loads
-        const bool uni = __ballot(cp != cp0 || bp.n != n0 || bp.konst >= 0) == 0;
-        const Insn *code = bp.code, *code0 = (const Insn *)cp0;
-        const LineAxis<false> ax(k);
+        uint2 bi = make_uint2(BRICK_FULL, P.ncode);
+        if (B.info) bi = B.info[sg.brick0 + ((size_t)(z / B.BZ) * B.nby + (y / B.BY)) * g.W + (x >> 6)];
+        const uint32_t at0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)bi.x);
+        const uint32_t n0 = (uint32_t)__builtin_amdgcn_readfirstlane((int)bi.y);
+        const bool uni = __ballot(bi.x != at0 || bi.y != n0) == 0;  // one program for the wave: scalar loads
         int left = sg.iters;
-        while (left > 2) {
-            const int levels = min(left, 6);
-            const uint64_t m = bp.konst >= 0 ? (bp.konst ? ~0ull : 0)
-                               : uni ? bracket_bits<true>(scalar_ptr(code0), n0, scalar_ptr(P.f64), g, ax, lo, hi, px, py,
-                                                        pz, levels, stack)
-                                   : bracket_bits<false>(code, bp.n, P.f64, g, ax, lo, hi, px, py, pz, levels, stack);
-            for (int bit = 1 << (levels - 1), at = 0; bit; bit >>= 1) {
-                const double mid = (lo + hi) / 2;
-                const bool in = (m >> (at + bit)) & 1;
-                if (in == up) hi = mid;  // the inside end moves
-                else lo = mid, at += bit;
-            }
-            left -= levels;
-        }
-        for (; left > 0; left--) {
-            const double mid = (lo + hi) / 2;
-            const double qx = k == 0 ? mid : px, qy = k == 1 ? mid : py, qz = k == 2 ? mid : pz;
-            GStats gs;
-            const bool in = bp.konst >= 0 ? bp.konst != 0
-                            : uni         ? eval_code<0, false, true>(code0, n0, P, qx, qy, qz, gs)
-                                          : eval_code<0, false, false>(code, bp.n, P, qx, qy, qz, gs);
-            if (in == up) hi = mid;
-            else lo = mid;
-        }
+        if (brick_constant(bi.y))  // (no halvings are left for a walk of its record's length)
+            for (; left > 0; left--) ((bi.y == BRICK_TRUE) == up ? hi : lo) = (lo + hi) / 2;
+        if (uni) halve<true>(brick_code(P, B, make_uint2(at0, n0)), n0, P, g, k, px, py, pz, up, left, lo, hi, stack);
+        else halve<false>(brick_code(P, B, bi), bi.y, P, g, k, px, py, pz, up, left, lo, hi, stack);
     }
     const double res = (lo + hi) / 2;
     verts[3 * v] = k == 0 ? res : px;

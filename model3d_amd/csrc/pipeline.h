@@ -75,6 +75,9 @@ struct Bricks {
     int BY, BZ, nby, nbz;
 };
 
+// The length in a record is no program's: the solid is a constant in the brick.
+MC3D_HD inline bool brick_constant(uint32_t n) { return n == 0 || n == BRICK_TRUE; }
+
 // What a brick's record says to evaluate: konst 0 or 1 where the solid is that
 // all over the brick (no instruction is walked: n is 0), else -1 and the code.
 struct BrickProgram {
@@ -83,8 +86,7 @@ struct BrickProgram {
     int konst;
 };
 MC3D_HD inline BrickProgram brick_program(const DevProg &P, const Bricks &B, uint32_t at, uint32_t n) {
-    if (n == 0) return BrickProgram{P.code, 0, 0};
-    if (n == BRICK_TRUE) return BrickProgram{P.code, 0, 1};
+    if (brick_constant(n)) return BrickProgram{P.code, 0, n == BRICK_TRUE ? 1 : 0};
     return BrickProgram{at == BRICK_FULL ? P.code : B.code + at, n, -1};
 }
 

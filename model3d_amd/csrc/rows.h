@@ -6,8 +6,8 @@
 // lie in it are one interval.  atom_span bounds that interval from outside
 // and from inside by more than the rounding of the reference's float64
 // expressions (atom64) and of the computation here: a point past the outer
-// bounds is false, a point within the inner bounds is true, and the few
-// points between the two are decided by atom64 itself.  A program over such
+// bounds is false, a point within the inner bounds is true, and the points
+// between the two, mostly few, are decided by atom64 itself.  A program over such
 // atoms is then a boolean expression over bit masks, one bit per point.
 // Every decision is the one atom64 makes at the point.
 #pragma once
@@ -51,14 +51,17 @@ MC3D_HD inline double recip(double x) {
 // more on each side; ri < 0: w' may be below zero.  (All in float64: D goes
 // down to 1e-219 over the coordinates that span_range admits.)
 MC3D_HD inline void span_root(double w, double D, double e0, double &ro, double &ri) {
-    const bool graze = w <= 4 * D;  // the line grazes the surface
-    const double v = graze ? 5 * D : w;
-    const double y = rsq_estimate(v);
-    double r = v * y;
-    r = r + 0.5 * y * __builtin_fma(-r, r, v);
-    const double e = graze ? 1e-3 * r + e0 : 1.1 * D * y + 1e-10 * r + e0;
+    if (w <= 4 * D) {  // the line grazes the surface
+        ro = 5 * D * rsq_estimate(5 * D) * 1.001 + e0;
+        ri = -1;
+        return;
+    }
+    const double y = rsq_estimate(w);
+    double r = w * y;
+    r = r + 0.5 * y * __builtin_fma(-r, r, w);
+    const double e = 1.1 * D * y + 1e-10 * r + e0;
     ro = r + e;
-    ri = graze ? -1 : r - e;
+    ri = r - e;
 }
 
 // Coordinates that are neither so large nor so small that a square or a
@@ -221,22 +224,35 @@ MC3D_HD inline double bracket_point(double a, double b, int levels, int i) {
     return m;
 }
 
-// The atom's mask over the points: sure ones, and those of the rest at
-// which atom64 is true (point(i): the i-th point's coordinate along axis k).
-// Only the points of `want` matter.
-template <bool KX, class F64P, class Point>
+// Open points that a lane evaluates one after another; a line with more of them
+// (one that touches the surface all along, or whose bounds are no finer than its
+// points) is decided otherwise.
+constexpr int FEW_OPEN = 4;
+
+// The atom's mask over the points: the sure ones, and those of the rest that
+// rest(kind, a, open) finds inside.  Only the points of `want` matter.
+template <bool KX, class F64P, class Rest>
 __device__ __forceinline__ uint64_t atom_mask(uint32_t kind, F64P a, const LineAxis<KX> &ax, double x, double y, double z, double smax,
                                               double mag, double scale, double eta, int last, uint64_t want,
-                                              Point &&point) {
+                                              Rest &&rest) {
     uint64_t sure, maybe;
     row_mask(atom_span(kind, a, ax, x, y, z, smax, mag), scale, eta, last, sure, maybe);
-    for (uint64_t open = maybe & ~sure & want; open; open &= open - 1) {
+    return sure | rest(kind, a, maybe & ~sure & want);
+}
+
+// The open points at which atom64 is true, one after another (point(i): the
+// i-th point's coordinate along the line's axis).
+template <bool KX, class F64P, class Point>
+__device__ __forceinline__ uint64_t open_points(uint32_t kind, F64P a, const LineAxis<KX> &ax, double x, double y, double z,
+                                                uint64_t open, Point &&point) {
+    uint64_t in = 0;
+    for (; open; open &= open - 1) {
         const int i = __ffsll((unsigned long long)open) - 1;
         const int k = KX ? 0 : ax.k;
         const double p = point(i);
-        if (atom64(kind, a, k == 0 ? p : x, k == 1 ? p : y, k == 2 ? p : z)) sure |= 1ull << i;
+        if (atom64(kind, a, k == 0 ? p : x, k == 1 ? p : y, k == 2 ? p : z)) in |= 1ull << i;
     }
-    return sure;
+    return in;
 }
 
 // One operator on masks: b is the top of the stack, a below it.
@@ -250,10 +266,10 @@ __device__ __forceinline__ M mask_op(uint32_t op, M a, M b) {
 
 // A program over such atoms as a mask over the points of a line; the stack
 // below its top lies in LDS (slot i of this lane: stack[i * stride]).
-template <bool UNI, class M, bool KX, class CodeP, class F64P, class Point>
+template <bool UNI, class M, bool KX, class CodeP, class F64P, class Rest>
 __device__ __forceinline__ M row_program(CodeP code, uint32_t n, F64P f64, const LineAxis<KX> &ax, double x, double y, double z,
                                          double smax, double mag, double scale, double eta, int last, M want,
-                                         M *stack, int stride, Point &&point) {
+                                         M *stack, int stride, Rest &&rest) {
     M top = 0;
     int sp = 0;
     for (uint32_t pc = 0; pc < n; ++pc) {
@@ -265,7 +281,7 @@ __device__ __forceinline__ M row_program(CodeP code, uint32_t n, F64P f64, const
             if (sp > 0) stack[(sp - 1) * stride] = top;
             sp++;
             top = op == OP_ATOM ? (M)atom_mask(insn_kind(in.x), f64 + in.y, ax, x, y, z, smax, mag, scale, eta, last,
-                                               (uint64_t)want, point)
+                                               (uint64_t)want, rest)
                                 : (op == OP_TRUE ? ~(M)0 : (M)0);
         } else if (op == OP_NOT) {
             top = ~top;
