@@ -19,20 +19,25 @@
 // a lane each: most are decided by summed-volume tables (no triangle listed
 // in the rect's cells: rejected; a segment origin in a cell inside it:
 // accepted, and with it every block above, whose rects contain the leaf's).
-// The few left open are asked with Triangle.RectCollision, a wave each, and
-// where the leaf is hit without an origin in it the blocks above it too.  The
-// reference's two-stage recursion (first down to max(volume / 4096, 64), then
-// each queued block down to 64) asks the same deterministic filter of the
-// same blocks, so its accepted leaves are these.
+// Those left open are asked with Triangle.RectCollision, a wave each, and where
+// the leaf is hit without an origin in it the blocks above it too: first of the
+// triangle that hits the leaf, a lane a block.  The reference's two-stage
+// recursion (first down to max(volume / 4096, 64), then each queued block down
+// to 64) asks the same deterministic filter of the same blocks, so its accepted
+// leaves are these.
 //
 // Level by level (a kernel per level, each waiting for the one above, four
 // blocks a wave so that open ones did not wait for each other) a grid of
-// 402^3 corners with 51k triangles took 1,660 us; here the leaves take 117
-// us (the mask's atomics) and the open ones 390 us, bound by the chain of
-// loads to each batch of 64 listed triangles (list, box, triangle).  Cells of
-// one coarse spacing instead of two list fewer triangles per rect (open 610
-// -> 460 us); the boxes kept from the binning reject most of a batch with six
-// comparisons (460 -> 372 us).
+// 402^3 corners with 51k triangles took 1,660 us; here the leaves take 54 us
+// (the mask's atomics) and the open ones 247 us, bound by the chain of
+// loads to each batch of 64 listed triangles (list, box, triangle) at 2 waves
+// per SIMD (240 registers, of the triangle test).  Cells of one coarse spacing
+// instead of two list fewer triangles per rect (open 610 -> 460 us); the boxes
+// kept from the binning reject most of a batch with six comparisons (460 -> 372
+// us); the blocks above asked of one triangle, not each in turn of the mesh, 376
+// -> 247 us.  A triangle as large as the grid leaves most leaves open: a list of a
+// quarter of them, the rest asked by the waves that found them, took 5,400 us for
+// twelve triangles on 202^3 corners (the levels 1,200 us; now 600).
 #include "launch.h"
 #include "rect_collide.h"
 
@@ -259,16 +264,27 @@ __device__ __forceinline__ bool boxes_overlap(const double *mn, const double *mx
            b.mn[2] <= mx[2] && mn[0] <= mx[0] && mn[1] <= mx[1] && mn[2] <= mx[2];
 }
 
+template <class T>
+__device__ __forceinline__ T lane_value(T v, int j) {
+    return __shfl(v, j, 64);
+}
+
+// One triangle's part of RectCollision for [mn, mx]: 0 no, 1 yes, 2 yes by a
+// segment origin inside, which is inside every larger rect too.
+__device__ __forceinline__ int tri_hits(const RectGridDev &R, uint32_t tri, const double *mn, const double *mx) {
+    const double *p = R.tris + 9 * (size_t)tri;
+    const rc::V v[3] = {rc::mk(p[0], p[1], p[2]), rc::mk(p[3], p[4], p[5]), rc::mk(p[6], p[7], p[8])};
+    return rc::vertex_inside(p, mn, mx) ? 2 : (rc::tri_rect(v, mn, mx) ? 1 : 0);
+}
+
 // RectCollision of the mesh for [mn, mx] where the vertex table gave no sure
-// hit, asked by a whole wave (the answer is wave-uniform: 0 no, 1 yes, 2 yes
-// by a segment origin inside, which is inside every larger rect too): every
-// candidate
-// triangle tested once -- the triangles binned in the cells the rect
+// hit, asked by a whole wave (the answer is wave-uniform, as tri_hits'; by: a
+// triangle that hits): every candidate triangle tested once -- the triangles binned in the cells the rect
 // overlaps, taken 64 at a time (each (y, z) row of those cells is one run
 // of the cell lists; a triangle listed in several of the rect's cells is
 // tested at the first of them), or, for a rect over more cells than half
 // the triangles, all triangles in a scattered order.
-__device__ int rect_hits(const RectGridDev &R, const double *mn, const double *mx) {
+__device__ int rect_hits(const RectGridDev &R, const double *mn, const double *mx, uint32_t &by) {
     const int lane = threadIdx.x & 63;
     int c0[3], c1[3];
     for (int a = 0; a < 3; a++) {
@@ -280,15 +296,15 @@ __device__ int rect_hits(const RectGridDev &R, const double *mn, const double *m
     if (2 * ncell > R.ntris) {
         for (uint32_t t0 = 0; t0 < R.ntris; t0 += 64) {
             int h = 0;
+            uint32_t t = 0;
             if (t0 + lane < R.ntris) {
-                const uint32_t t = scatter(t0 + lane, R.ntris, 4294967291ull);
-                const double *p = R.tris + 9 * (size_t)t;
-                if (boxes_overlap(mn, mx, R.box[t])) {
-                    const rc::V v[3] = {rc::mk(p[0], p[1], p[2]), rc::mk(p[3], p[4], p[5]), rc::mk(p[6], p[7], p[8])};
-                    h = rc::vertex_inside(p, mn, mx) ? 2 : (rc::tri_rect(v, mn, mx) ? 1 : 0);
-                }
+                t = scatter(t0 + lane, R.ntris, 4294967291ull);
+                if (boxes_overlap(mn, mx, R.box[t])) h = tri_hits(R, t, mn, mx);
             }
-            if (__ballot(h != 0)) return __ballot(h == 2) ? 2 : 1;
+            if (const uint64_t m = __ballot(h != 0)) {
+                by = lane_value(t, __ffsll((unsigned long long)m) - 1);
+                return __ballot(h == 2) ? 2 : 1;
+            }
         }
         return 0;
     }
@@ -322,10 +338,10 @@ __device__ int rect_hits(const RectGridDev &R, const double *mn, const double *m
             const uint32_t aj = __shfl(a, lo, 64), xj = __shfl(excl, lo, 64);
             const int yj = __shfl(ry, lo, 64), zj = __shfl(rz, lo, 64);
             int h = 0;
+            uint32_t tri = 0;
             if (e < total) {
                 const uint32_t idx = aj + (e - xj);
-                const uint32_t tri = R.cell_tris[idx];
-                const double *p = R.tris + 9 * (size_t)tri;
+                tri = R.cell_tris[idx];
                 const GroupBox tb = R.box[tri];
                 if (boxes_overlap(mn, mx, tb)) {
                     // the first of the rect's cells that list it: row (y, z)
@@ -334,23 +350,17 @@ __device__ int rect_hits(const RectGridDev &R, const double *mn, const double *m
                     for (int ax = 0; ax < 3; ax++) cell_range(tb.mn[ax], tb.mx[ax], R.o[ax], R.inv, R.n[ax], t0[ax], t1[ax]);
                     if (yj == max(t0[1], c0[1]) && zj == max(t0[2], c0[2])) {
                         const size_t cf = ((size_t)zj * R.n[1] + yj) * R.n[0] + max(t0[0], c0[0]);
-                        if (idx >= R.cell_start[cf] && idx < R.cell_start[cf + 1]) {
-                            const rc::V t[3] = {rc::mk(p[0], p[1], p[2]), rc::mk(p[3], p[4], p[5]),
-                                                rc::mk(p[6], p[7], p[8])};
-                            h = rc::vertex_inside(p, mn, mx) ? 2 : (rc::tri_rect(t, mn, mx) ? 1 : 0);
-                        }
+                        if (idx >= R.cell_start[cf] && idx < R.cell_start[cf + 1]) h = tri_hits(R, tri, mn, mx);
                     }
                 }
             }
-            if (__ballot(h != 0)) return __ballot(h == 2) ? 2 : 1;
+            if (const uint64_t m = __ballot(h != 0)) {
+                by = lane_value(tri, __ffsll((unsigned long long)m) - 1);
+                return __ballot(h == 2) ? 2 : 1;
+            }
         }
     }
     return 0;
-}
-
-template <class T>
-__device__ __forceinline__ T lane_value(T v, int j) {
-    return __shfl(v, j, 64);
 }
 
 // mcBlock.Pieces(64, ...) stops at this block (mc.go:760-775).
@@ -408,18 +418,30 @@ __device__ void open_leaf(const BlockFilter &F, const FBlock &root, int depth, u
     for (; leaf < depth && !is_leaf(b); leaf++) halve(b, (path >> (depth - 1 - leaf)) & 1);
     double mn[3], mx[3];
     block_rect(F, b, mn, mx);
-    int hit = rect_hits(F.R, mn, mx);
-    if (!hit) return;
-    if (hit == 1) {  // the blocks above (lane i: i halvings down), up to one that certainly is hit
-        FBlock u = root;
-        for (int d = 0; d < min(lane, leaf); d++) halve(u, (path >> (depth - 1 - d)) & 1);
-        block_rect(F, u, mn, mx);
-        const uint64_t sure = __ballot(lane < leaf && sure_hit(F.R, mn, mx));
-        for (int j = leaf - 1; j >= 0 && hit != 2 && !((sure >> j) & 1); j--) {
-            double jmn[3], jmx[3];
-            for (int a = 0; a < 3; a++) jmn[a] = lane_value(mn[a], j), jmx[a] = lane_value(mx[a], j);
-            if (!(hit = rect_hits(F.R, jmn, jmx))) return;
+    // The leaf, then (lane i: i halvings down) the blocks above it: almost always
+    // the triangle that hits the leaf hits them all, each asked of it by its own
+    // lane; one that it does not hit, and whose rect holds no other that certainly
+    // is hit, is asked of the mesh.
+    uint64_t ask = 0;
+    double amn[3], amx[3];
+    for (int at = leaf;;) {
+        uint32_t by = 0;
+        const int hit = rect_hits(F.R, mn, mx, by);
+        if (!hit) return;
+        if (hit == 2) break;
+        if (at == leaf) {
+            FBlock u = root;
+            for (int d = 0; d < min(lane, leaf); d++) halve(u, (path >> (depth - 1 - d)) & 1);
+            block_rect(F, u, amn, amx);
+            const int h = sure_hit(F.R, amn, amx) ? 2 : (boxes_overlap(amn, amx, F.R.box[by]) ? tri_hits(F.R, by, amn, amx) : 0);
+            ask = __ballot(lane < leaf && h == 0);
+            const uint64_t sure = __ballot(lane < leaf && h == 2);
+            if (sure) ask &= ~(~0ull >> __clzll((long long)sure));
         }
+        if (!ask) break;
+        at = 63 - __clzll((long long)ask);
+        ask &= ~(1ull << at);
+        for (int a = 0; a < 3; a++) mn[a] = lane_value(amn[a], at), mx[a] = lane_value(amx[a], at);
     }
     const int jy = b.mx[1] - b.mn[1], rows = jy * (b.mx[2] - b.mn[2]);
     for (int r = lane; r < rows; r += 64) set_cubes(keep_row(F, b.mn[1] + r % jy, b.mn[2] + r / jy), b.mn[0], b.mx[0]);
@@ -428,19 +450,20 @@ __device__ void open_leaf(const BlockFilter &F, const FBlock &root, int depth, u
 // Rows of a wave's common block whose cubes are gathered in LDS.
 constexpr int LEAF_ROWS = 640;
 
-// A lane per leaf; a wave's 64 leaves share the block 6 halvings up, which is
-// asked first, and whose cubes are gathered row by row before they go out.
-// The leaves left open go to the list, or where it is full are asked here.
-__global__ __launch_bounds__(256) void k_filter_leaves(BlockFilter F, FBlock root, int depth, uint64_t npath,
-                                                       uint64_t *__restrict__ open, uint32_t *__restrict__ nopen,
-                                                       uint32_t ocap) {
+// The leaves of paths [path0, path0 + npath) (path0 a multiple of 64), a lane
+// each; a wave's 64 leaves share the block 6 halvings up, which is asked first,
+// and whose cubes are gathered row by row before they go out.  The leaves left
+// open go to the list, which holds npath.
+__global__ __launch_bounds__(256) void k_filter_leaves(BlockFilter F, FBlock root, int depth, uint64_t path0,
+                                                       uint64_t npath, uint64_t *__restrict__ open,
+                                                       uint32_t *__restrict__ nopen) {
     __shared__ unsigned long long rows_all[4][LEAF_ROWS];
     const int lane = threadIdx.x & 63;
     const int wid = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));  // (scalar: so is the walk to the common block)
     unsigned long long *rows = rows_all[wid];
     const uint64_t wave = blockIdx.x * 4ull + wid, nw = gridDim.x * 4ull;
     const int above = depth > 6 ? depth - 6 : 0;
-    for (uint64_t base = wave * 64; base < npath; base += nw * 64) {
+    for (uint64_t base = path0 + wave * 64; base < path0 + npath; base += nw * 64) {
         FBlock b = root;
         int d = 0;
         for (; d < above && !is_leaf(b); d++) halve(b, (base >> (depth - 1 - d)) & 1);
@@ -450,7 +473,7 @@ __global__ __launch_bounds__(256) void k_filter_leaves(BlockFilter F, FBlock roo
         if ((single && (base & ((1ull << (depth - d)) - 1))) || sure_miss(F.R, mn, mx)) continue;
         const uint64_t path = base + lane;
         FBlock l = b;
-        bool valid = path < npath && (!single || lane == 0);
+        bool valid = path < path0 + npath && (!single || lane == 0);
         if (!single) {
             for (; d < depth && !is_leaf(l); d++) halve(l, (path >> (depth - 1 - d)) & 1);
             valid = valid && (path & ((1ull << (depth - d)) - 1)) == 0;
@@ -463,16 +486,9 @@ __global__ __launch_bounds__(256) void k_filter_leaves(BlockFilter F, FBlock roo
         const uint64_t am = __ballot(ask);
         if (am) {
             uint32_t at = 0;
-            if (lane == 0) {  // (a full list's count stops growing)
-                at = __hip_atomic_load(nopen, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                if (at < ocap) at = atomicAdd(nopen, (uint32_t)__popcll(am));
-            }
+            if (lane == 0) at = atomicAdd(nopen, (uint32_t)__popcll(am));
             at = lane_value(at, 0);
-            const uint32_t mine = at + (uint32_t)__popcll(am & ((1ull << lane) - 1));
-            const bool fits = at < ocap && mine < ocap;
-            if (ask && fits) open[mine] = path;
-            for (uint64_t left = __ballot(ask && !fits); left; left &= left - 1)
-                open_leaf(F, root, depth, base + (uint64_t)(__ffsll((unsigned long long)left) - 1));
+            if (ask) open[at + (uint32_t)__popcll(am & ((1ull << lane) - 1))] = path;
         }
         if (!__ballot(acc)) continue;
         const int bx = b.mx[0] - b.mn[0], by = b.mx[1] - b.mn[1], nrows = by * (b.mx[2] - b.mn[2]);
@@ -505,9 +521,9 @@ __global__ __launch_bounds__(256) void k_filter_leaves(BlockFilter F, FBlock roo
 
 __global__ __launch_bounds__(256) void k_filter_open(BlockFilter F, FBlock root, int depth,
                                                      const uint64_t *__restrict__ open,
-                                                     const uint32_t *__restrict__ nopen, uint32_t ocap) {
+                                                     const uint32_t *__restrict__ nopen) {
     const uint32_t wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6, nw = (gridDim.x * blockDim.x) >> 6;
-    const uint32_t n = min(*nopen, ocap);
+    const uint32_t n = *nopen;
     for (uint32_t i = wave; i < n; i += nw) open_leaf(F, root, depth, open[i]);
 }
 
@@ -556,9 +572,13 @@ hipError_t launch_table(uint32_t *t, const int *n, hipStream_t st) {
 
 hipError_t launch_block_filter(const BlockFilter &F, const FBlock &root, int depth, uint64_t *open, uint32_t *nopen,
                                uint32_t ocap, hipStream_t st) {
-    const uint64_t npath = 1ull << depth;
-    k_filter_leaves<<<grid_for(npath, 256, 1u << 16), 256, 0, st>>>(F, root, depth, npath, open, nopen, ocap);
-    k_filter_open<<<grid_for(std::min<uint64_t>(npath, ocap), 4, 2048), 256, 0, st>>>(F, root, depth, open, nopen, ocap);
+    const uint64_t npath = 1ull << depth, part = std::min<uint64_t>(npath, ocap);
+    for (uint64_t path0 = 0; path0 < npath; path0 += part) {
+        const hipError_t e = launch_zero(nopen, 16, st);
+        if (e != hipSuccess) return e;
+        k_filter_leaves<<<grid_for(part, 256, 1u << 16), 256, 0, st>>>(F, root, depth, path0, part, open, nopen);
+        k_filter_open<<<grid_for(part, 4, 2048), 256, 0, st>>>(F, root, depth, open, nopen);
+    }
     return hipGetLastError();
 }
 

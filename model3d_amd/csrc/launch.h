@@ -158,8 +158,8 @@ hipError_t launch_rgrid_fill(const RectGridDev &R, uint32_t *cursor, uint32_t *c
 hipError_t launch_vgrid(const RectGridDev &R, uint32_t *vsat, hipStream_t st);
 // cell counts t of an n[0] x n[1] x n[2] grid into their summed-volume table
 hipError_t launch_table(uint32_t *t, const int *n, hipStream_t st);
-// the recursion from root, at most `depth` halvings deep (open: ocap paths of
-// leaves; *nopen must start at zero)
+// the recursion from root, at most `depth` halvings deep, up to ocap (a multiple
+// of 64, or 2^depth) leaves at a time (open: as many entries; nopen: 16 bytes)
 hipError_t launch_block_filter(const BlockFilter &F, const FBlock &root, int depth, uint64_t *open, uint32_t *nopen,
                                uint32_t ocap, hipStream_t st);
 

@@ -1529,6 +1529,8 @@ int filter_depth(int lx, int ly, int lz) {
     }
 }
 
+constexpr uint32_t FILTER_LEAVES = 1u << 22;  // (a multiple of 64)
+
 // The block filter of job j on the device, into the cube mask `keep`
 // (after the upload: it reads the grid's axes there).  The collider's
 // triangles are binned in a grid over the search grid's bounds (cells of
@@ -1614,12 +1616,11 @@ int enqueue_block_filter(mc3d_ctx *ctx, const Job &j, const Upload &U, uint64_t 
     // the recursion from the root block (mc.go:712-716)
     const FBlock root{{0, 0, 0}, {j.g.nx - 1, j.g.ny - 1, j.g.nz - 1}};
     const int depth = filter_depth(root.mx[0], root.mx[1], root.mx[2]);
-    // room for a quarter of the leaves, at most 32 MiB (where the list is
-    // full, leaves are asked by the wave that found them)
-    const uint32_t ocap = (uint32_t)std::min<uint64_t>(std::max<uint64_t>((1ull << depth) / 4, 1024), 1u << 22);
+    // Room for all leaves, up to 4 M of them (32 MiB: a grid of about 730^3
+    // cubes), else that many at a time.
+    const uint32_t ocap = (uint32_t)std::min<uint64_t>(1ull << depth, FILTER_LEAVES);
     if ((rc = ctx->rf_open.ensure(ocap * sizeof(uint64_t))) || (rc = ctx->rf_nopen.ensure(16))) return rc;
     HIP_TRY(hipMemsetAsync(keep, 0, j.nwords * 8, st));
-    HIP_TRY(hipMemsetAsync(ctx->rf_nopen.p, 0, 4, st));
     const Grid &g = U.hsegs[0].g;
     const BlockFilter BF{R, g.xs, g.ys, g.zs, j.delta * 1e-3, F.extra, keep, g.W, g.ny};
     HIP_TRY(launch_block_filter(BF, root, depth, ctx->rf_open.as<uint64_t>(), ctx->rf_nopen.as<uint32_t>(), ocap, st));
