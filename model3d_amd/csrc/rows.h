@@ -47,36 +47,36 @@ MC3D_HD inline double recip(double x) {
 #endif
 }
 
-// ro >= sqrt(w') >= ri for every w' in [w - D, w + D] (w >= -D), with e0
-// more on each side; ri < 0: w' may be below zero.  (All in float64: D goes
-// down to 1e-219 over the coordinates that span_range admits.)
-MC3D_HD inline void span_root(double w, double D, double e0, double &ro, double &ri) {
+// ro >= sqrt(w') >= ri for every w' in [w - D, w + D] (w >= -D), with 1e-10 of
+// itself more on each side; ri < 0: w' may be below zero.  (All in float64: D goes
+// down to 1e-219 over the lengths that span_range admits.)
+MC3D_HD inline void span_root(double w, double D, double &ro, double &ri) {
     if (w <= 4 * D) {  // the line grazes the surface
-        ro = 5 * D * rsq_estimate(5 * D) * 1.001 + e0;
+        ro = 5 * D * rsq_estimate(5 * D) * 1.001;
         ri = -1;
         return;
     }
     const double y = rsq_estimate(w);
     double r = w * y;
     r = r + 0.5 * y * __builtin_fma(-r, r, w);
-    const double e = 1.1 * D * y + 1e-10 * r + e0;
+    const double e = 1.1 * D * y + 1e-10 * r;
     ro = r + e;
     ri = r - e;
 }
 
-// Coordinates that are neither so large nor so small that a square or a
-// product of two leaves the float64 range.
+// Lengths that are neither so large nor so small that a square or a product of
+// two leaves the float64 range.
 MC3D_HD inline bool span_range(double M) { return M > 1e-100 && M < 1e100; }
 
 // The axis of a line: known when the code is compiled (KX: the x axis), or
-// a lane's own, then as the unit vector e_k and 1 - e_k, so that picking a
+// a lane's own, then as the unit vector e_k, so that picking or leaving out a
 // component is three multiply-adds instead of selects of scalar operands.
 template <bool KX>
 struct LineAxis {
     int k = 0;
-    double v[3] = {1, 0, 0}, u[3] = {0, 1, 1};
+    double v[3] = {1, 0, 0};
     MC3D_HD explicit LineAxis(int axis) : k(axis) {
-        for (int a = 0; a < 3; a++) v[a] = a == axis ? 1.0 : 0.0, u[a] = a == axis ? 0.0 : 1.0;
+        for (int a = 0; a < 3; a++) v[a] = a == axis ? 1.0 : 0.0;
     }
     MC3D_HD double along(double x, double y, double z) const {
         if (KX) return x;
@@ -84,18 +84,37 @@ struct LineAxis {
     }
     MC3D_HD double across2(double x, double y, double z) const {  // the other components' squares
         if (KX) return __builtin_fma(z, z, y * y);
-        return __builtin_fma(z * z, u[2], __builtin_fma(y * y, u[1], x * x * u[0]));
+        const double a = __builtin_fma(-x, v[0], x), b = __builtin_fma(-y, v[1], y), c = __builtin_fma(-z, v[2], z);
+        return __builtin_fma(c, c, __builtin_fma(b, b, a * a));
     }
 };
 
-// Sphere with threshold T (s <= T) whose centre is p - d, M bounding every
-// coordinate and length.  Rounding moves s by far less than 1e-13 M^2.
+// A vector's square, its component along the line's axis and the square of the
+// rest, which rounding moves by a few half ulps of the whole square.
+struct LineVec {
+    double vv, along, across2;
+};
 template <bool KX>
-MC3D_HD inline Span sphere_span(const LineAxis<KX> &ax, double dx, double dy, double dz, double T, double M) {
-    const double D = 1e-13 * M * M, w = T - ax.across2(dx, dy, dz), m = -ax.along(dx, dy, dz);
+MC3D_HD inline LineVec line_vec(const LineAxis<KX> &ax, double x, double y, double z) {
+    LineVec r;
+    r.along = ax.along(x, y, z);
+    if (KX) {
+        r.across2 = __builtin_fma(z, z, y * y);
+        r.vv = __builtin_fma(x, x, r.across2);
+    } else {
+        r.vv = __builtin_fma(z, z, __builtin_fma(y, y, x * x));
+        r.across2 = __builtin_fma(-r.along, r.along, r.vv);
+    }
+    return r;
+}
+
+// Sphere with threshold T (s <= T) whose centre is p - d, its squared distance s
+// known to D.
+MC3D_HD inline Span sphere_span(const LineVec &d, double T, double D) {
+    const double w = T - d.across2, m = -d.along;
     if (w < -D) return span_none();
     double ro, ri;
-    span_root(w, D, 1e-14 * M, ro, ri);
+    span_root(w, D, ro, ri);
     Span s{m - ro, m + ro, INFINITY, -INFINITY};
     if (ri > 0) s.ai = m - ri, s.bi = m + ri;
     return s;
@@ -105,24 +124,26 @@ MC3D_HD inline Span sphere_span(const LineAxis<KX> &ax, double dx, double dy, do
 // c = v.d and n = v - c d, the squared distance from its axis is |n|^2 +
 // 2 s n_k + s^2 (1 - d_k^2), the position along it c + s d_k.  smax: the
 // largest |s| asked about (nearly parallel lines, where the roots or the end
-// planes are ill-defined, are bounded over that range instead).
+// planes are ill-defined, are bounded over that range instead).  M bounds the
+// lengths it is made of, D the rounding of the squared distance.
 template <bool KX>
-MC3D_HD inline Span cylinder_span(const LineAxis<KX> &ax, double vx, double vy, double vz, double dx, double dy, double dz,
-                                  double L, double T, double smax, double M) {
-    const double c = vx * dx + vy * dy + vz * dz;  // (atom64's own sum)
-    const double nx = __builtin_fma(-dx, c, vx), ny = __builtin_fma(-dy, c, vy), nz = __builtin_fma(-dz, c, vz);
-    const double nk = ax.along(nx, ny, nz), dk = ax.along(dx, dy, dz), A = ax.across2(dx, dy, dz);
-    const double w = T - __builtin_fma(nz, nz, __builtin_fma(ny, ny, nx * nx)), D = 1e-13 * M * M;
+MC3D_HD inline Span cylinder_span(const LineAxis<KX> &ax, const LineVec &v, double c, double dx, double dy, double dz, double L,
+                                  double T, double smax, double M, double D) {
+    const double dk = ax.along(dx, dy, dz), A = ax.across2(dx, dy, dz);
+    const double nk = __builtin_fma(-c, dk, v.along), w = T - __builtin_fma(-c, c, v.vv);
     Span s;
     if (A < 1e-6) {  // along the axis: the distance hardly changes
         const double D2 = D + 2 * fabs(nk) * smax + A * smax * smax;
         if (w < -D2) return span_none();
         s = w > D2 ? span_all() : span_unsure();
     } else {
-        const double disc = __builtin_fma(A, w, nk * nk), DD = A * D + 1e-14 * nk * nk;
+        // (n_k, at most |n| sqrt(A), carries a rounding of M: more than A D of
+        // its square where the line is nearly parallel)
+        const double disc = __builtin_fma(A, w, nk * nk);
+        const double DD = __builtin_fma(fabs(nk), __builtin_fma(1e-14, fabs(nk), 4e-15 * M), A * D);
         if (disc < -DD) return span_none();
         double ro, ri;
-        span_root(disc, DD, 0, ro, ri);
+        span_root(disc, DD, ro, ri);
         const double iA = recip(A), e = (1e-12 * (fabs(nk) + ro) + 1e-14 * M) * iA;
         s = Span{(-nk - ro) * iA - e, (-nk + ro) * iA + e, INFINITY, -INFINITY};
         if (ri > 0) s.ai = (-nk - ri) * iA + e, s.bi = (-nk + ri) * iA - e;
@@ -152,7 +173,6 @@ MC3D_HD inline Span cylinder_span(const LineAxis<KX> &ax, double vx, double vy, 
 template <bool KX, class F64P>
 MC3D_HD inline Span atom_span(uint32_t kind, F64P a, const LineAxis<KX> &ax, double x, double y, double z, double smax,
                               double mag) {
-    auto size = [&](int o) { return fabs(a[o]) + fabs(a[o + 1]) + fabs(a[o + 2]); };
     if (kind == A_RECT) {  // exact comparisons off the line's axis
         const int k = KX ? 0 : ax.k;
         const bool in = (int)(k == 0 || ((int)in_lo(x, a[0]) & (int)in_hi(x, a[3]))) &
@@ -166,27 +186,37 @@ MC3D_HD inline Span atom_span(uint32_t kind, F64P a, const LineAxis<KX> &ax, dou
         const double eh = fabs(hi) < INFINITY ? 1e-15 * (mag + fabs(a1)) : 0;
         return Span{lo - el, hi + eh, lo + el, hi - eh};
     }
+    // Rounding is bounded by the lengths that are computed with, not by the
+    // coordinates (a solid far from the origin has the same differences, each
+    // rounded once): the squared distance moves by far less than 1e-13 of the
+    // square of their sum, 3e-13 of the sum of three squares.
+    const double vx = x - a[0], vy = y - a[1], vz = z - a[2];
+    const LineVec v = line_vec(ax, vx, vy, vz);
     if (kind == A_SPHERE) {
-        const double M = 3 * mag + size(0) + a[3];
-        if (!span_range(M)) return span_unsure();
-        return sphere_span(ax, x - a[0], y - a[1], z - a[2], a[4], M);
+        const double q = v.vv + __builtin_fma(smax, smax, a[4]);
+        if (!(q > 1e-200 && q < 1e200)) return span_unsure();
+        return sphere_span(v, a[4], 3e-13 * q);
     }
-    if (kind == A_CYLINDER) {
-        const double M = 3 * mag + size(0) + a[6] + a[7];
-        if (!(span_range(M) && size(3) < 2)) return span_unsure();
-        return cylinder_span(ax, x - a[0], y - a[1], z - a[2], a[3], a[4], a[5], a[6], a[8], smax, M);
-    }
+    // Contains of the other two takes the difference from the axis's nearest
+    // point, rounded as a coordinate (at most G): 7 half ulps of G, at a distance
+    // of up to M, move the square by less than 1e-15 M G.
+    const bool cyl = kind == A_CYLINDER;
+    const double L = cyl ? a[6] : a[9], M = fabs(vx) + fabs(vy) + fabs(vz) + smax + L + (cyl ? a[7] : a[10]), G = mag + M;
+    const double D = __builtin_fma(1e-30 * G, G, M * __builtin_fma(1e-13, M, 4e-15 * G));
+    const int dir = cyl ? 3 : 6;
+    if (!(span_range(M) && G < 1e100 && fabs(a[dir]) + fabs(a[dir + 1]) + fabs(a[dir + 2]) < 2)) return span_unsure();
+    const double T = cyl ? a[8] : a[11];
+    const double c = vx * a[dir] + vy * a[dir + 1] + vz * a[dir + 2];  // (atom64's own sum)
+    Span s = cylinder_span(ax, v, c, a[dir], a[dir + 1], a[dir + 2], L, T, smax, M, D);
+    if (cyl) return s;
     // capsule: the cylinder between two spheres; it is convex, so the hull
-    // of their intervals (and of the certain parts of those) is its own
-    const double M = 3 * mag + size(0) + size(3) + a[9] + a[10];
-    if (!(span_range(M) && size(6) < 2)) return span_unsure();
-    const Span u = sphere_span(ax, x - a[0], y - a[1], z - a[2], a[11], M);
-    const Span v = sphere_span(ax, x - a[3], y - a[4], z - a[5], a[11], M);
-    Span s = cylinder_span(ax, x - a[0], y - a[1], z - a[2], a[6], a[7], a[8], a[9], a[11], smax, M);
+    // of their intervals (and of the certain parts of those, each by the margin
+    // of the points between the ends) is its own
+    const Span u = sphere_span(v, T, D), e = sphere_span(line_vec(ax, x - a[3], y - a[4], z - a[5]), T, D);
     if (!(s.ao <= s.bo)) s = span_none();
     if (!(s.ai <= s.bi)) s.ai = INFINITY, s.bi = -INFINITY;
-    s.ao = fmin(s.ao, fmin(u.ao, v.ao)), s.bo = fmax(s.bo, fmax(u.bo, v.bo));
-    s.ai = fmin(s.ai, fmin(u.ai, v.ai)), s.bi = fmax(s.bi, fmax(u.bi, v.bi));
+    s.ao = fmin(s.ao, fmin(u.ao, e.ao)), s.bo = fmax(s.bo, fmax(u.bo, e.bo));
+    s.ai = fmin(s.ai, fmin(u.ai, e.ai)), s.bi = fmax(s.bi, fmax(u.bi, e.bi));
     return s;
 }
 

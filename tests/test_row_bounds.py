@@ -59,3 +59,28 @@ def test_lines_in_a_cap_plane(kind, axis):
                 worst, inside = max(worst, opened), inside + n
     assert inside > 4000
     assert worst <= 2
+
+
+@pytest.mark.parametrize("kind", ["sphere", "cylinder", "capsule"])
+@pytest.mark.parametrize("far", [0.0, 1e3, 1e4, 1e5, 1e6])
+def test_lines_far_from_the_origin(kind, far):
+    """A solid's place costs its bounds nothing: rows and edges (spacing 0.01)
+    through solids of size one leave on average less than one point open, up to
+    10^8 spacings from the origin."""
+    rng = np.random.default_rng(int(far) + len(kind))
+    opened = inside = 0
+    lines = 400
+    for _ in range(lines):
+        c = [far + float(v) for v in rng.uniform(-1, 1, 3)]
+        d = rng.normal(size=3)
+        d /= np.linalg.norm(d)
+        e = [a + float(b) for a, b in zip(c, d)]
+        s = m3.Sphere(c, 0.5) if kind == "sphere" else (m3.Cylinder if kind == "cylinder" else m3.Capsule)(c, e, 0.4)
+        k, levels = int(rng.integers(3)), (0, 6)[int(rng.integers(2))]
+        t = float(rng.uniform(0.1, 0.9)) if kind != "sphere" else 0.0
+        p = [a + t * (b - a) + float(rng.uniform(-0.2, 0.2)) for a, b in zip(c, e)]
+        p[k] -= float(rng.uniform(0.0, 0.8))
+        o, n = _line(s, p, k, 0.01 if levels == 0 else 0.8, levels)
+        opened, inside = opened + o, inside + n
+    assert inside > 10 * lines
+    assert opened < lines
