@@ -215,9 +215,11 @@ struct Pool {
     std::vector<std::unique_ptr<B>> free;
     std::unique_ptr<B> take(size_t bytes) {
         std::lock_guard<std::mutex> lk(mu);
+        // (of equals the last given: calls of one shape then come back to the
+        // same few buffers, which their captured launches name)
         size_t best = free.size();
         for (size_t i = 0; i < free.size(); i++)
-            if (free[i]->cap >= bytes && (best == free.size() || free[i]->cap < free[best]->cap)) best = i;
+            if (free[i]->cap >= bytes && (best == free.size() || free[i]->cap <= free[best]->cap)) best = i;
         if (best < free.size()) {
             std::unique_ptr<B> b = std::move(free[best]);
             free.erase(free.begin() + best);
