@@ -240,6 +240,33 @@ struct Pool {
     }
 };
 
+// Device memory for one call's arrays of sizes not known beforehand, all in use
+// until the call ends: handed out of a few large buffers, which stay for the next
+// call (up to KEEP bytes of them; its calls run one after another on a context).
+struct DevArena {
+    static constexpr size_t CHUNK = 16u << 20, KEEP = 256u << 20;
+    std::vector<std::unique_ptr<DevBuf>> bufs;
+    size_t cur = 0, off = 0;
+    void start() { cur = off = 0; }
+    int take(size_t bytes, void **out) {
+        bytes = (bytes + 255) / 256 * 256;
+        if (cur < bufs.size() && off + bytes > bufs[cur]->cap) cur++, off = 0;
+        if (cur == bufs.size()) bufs.emplace_back(new DevBuf);
+        if (off == 0) {  // (this buffer holds nothing of the call yet)
+            const int rc = bufs[cur]->ensure(std::max(bytes, CHUNK));
+            if (rc) return rc;
+        }
+        *out = bufs[cur]->as<char>() + off;
+        off += bytes;
+        return MC3D_OK;
+    }
+    void trim() {
+        size_t kept = 0, n = 0;
+        while (n < bufs.size() && (kept += bufs[n]->cap) <= KEEP) n++;
+        bufs.resize(n);
+    }
+};
+
 // memcpy of large host buffers split over up to 16 threads (the first touch
 // of freshly allocated pages dominates a single-threaded copy).
 // Host threads kept for the library's parallel host loops (lowering a
@@ -470,6 +497,7 @@ struct mc3d_ctx {
     DevBuf keep;                         // block filter: cube mask
     // z slabs: a plane's vertex list and the stitch's per-vertex arrays
     DevBuf s_counts, s_keys[2], s_vals[2], s_ends, s_pieces;
+    DevArena s_ranks;
     // device block filter: triangles, their grid, the open leaves
     DevBuf rf_tris, rf_box, rf_counts, rf_start, rf_cursor, rf_cells, rf_tiles, rf_open, rf_nopen, rf_vsat;
     HostBuf rf_total;
@@ -2061,21 +2089,21 @@ int search_slabs(mc3d_ctx *ctx, Job &base, const mc3d_options &o, int planes, mc
     so.no_graph = 1;
     struct Piece {
         std::unique_ptr<mc3d_mesh, void (*)(mc3d_mesh *)> m{nullptr, mc3d_mesh_free};
-        std::unique_ptr<DevBuf> rank;
+        uint32_t *rank = nullptr;
     };
     const size_t npieces = (size_t)(ncube + planes - 1) / planes;
     std::vector<Piece> pieces;
     pieces.reserve(npieces);
     int table_bits[2] = {1, 1};  // of the top planes' edges, slabs in turn
-    // (the ranks' buffers go back to the pool however the call ends)
+    ctx->s_ranks.start();
+    // (the pieces' buffers are in use until the stream is done, however the call ends)
     struct Return {
         mc3d_ctx *ctx;
-        std::vector<Piece> &pieces;
         ~Return() {
             (void)hipStreamSynchronize(ctx->stream);
-            for (Piece &p : pieces) ctx->pool->give(std::move(p.rank));
+            ctx->s_ranks.trim();
         }
-    } on_return{ctx, pieces};
+    } on_return{ctx};
     int rc;
     for (int c0 = 0; c0 < ncube; c0 += planes) {
         const int c1 = std::min(ncube, c0 + planes);
@@ -2102,11 +2130,10 @@ int search_slabs(mc3d_ctx *ctx, Job &base, const mc3d_options &o, int planes, mc
         SlabPart S;
         S.vkeys = ctx->vkeys.as<uint64_t>();
         S.nv = nv;
-        pc.rank = ctx->pool->take(nv * 4 + 16);
-        if ((rc = pc.rank->ensure(nv * 4 + 16)) || (rc = ctx->s_counts.ensure((size_t)slab_tiles(nv) * 4)) ||
+        if ((rc = ctx->s_ranks.take(nv * 4 + 16, (void **)&pc.rank)) || (rc = ctx->s_counts.ensure((size_t)slab_tiles(nv) * 4)) ||
             (rc = ctx->s_ends.ensure(npieces * sizeof(SlabEnd))))
             return rc;
-        S.rank = pc.rank->as<uint32_t>();
+        S.rank = pc.rank;
         S.counts = ctx->s_counts.as<uint32_t>();
         S.end = ctx->s_ends.as<SlabEnd>() + k;
         if (c0 > 0) {
@@ -2169,7 +2196,7 @@ int search_slabs(mc3d_ctx *ctx, Job &base, const mc3d_options &o, int planes, mc
         P.v = m.buf->verts->as<double>() + 3 * m.voff;
         P.in = interior ? m.buf->interior->as<double>() + 3 * m.voff : nullptr;
         P.t = m.buf->tris->as<uint32_t>() + 3 * m.toff;
-        P.rank = pieces[k].rank->as<uint32_t>();
+        P.rank = pieces[k].rank;
         P.nv = m.nv, P.nt = m.nt, P.tbase = tbase;
         P.vbase = (uint32_t)vbase, P.pad = 0;
         vbase += m.nv - ends[k].bottom;

@@ -1,0 +1,73 @@
+"""Buffers kept between calls: a search in z slabs leaves later calls as they
+were -- their outputs come from the same few buffers, so that their captured
+launches are found again -- and its own repeat gives the same mesh."""
+import ctypes
+import time
+
+import numpy as np
+import pytest
+
+import model3d_amd as m3
+from model3d_amd import _lib
+from model3d_amd.solids import LibBackend
+from tests.helpers import same_triangles
+
+pytestmark = pytest.mark.gpu
+
+
+class _Calls:
+    def __init__(self, s):
+        self.b, self.L, self.ctx = LibBackend(), _lib.lib(), _lib.context(0)
+        self.h = s._build(self.b)
+
+    def run(self, entry, delta, iters, planes=0, fetch=False):
+        o = _lib.mc3d_options()
+        o.cull, o.device_only, o.slab_planes = 1, 1, planes
+        out = ctypes.c_void_p()
+        t = time.perf_counter()
+        _lib.check(getattr(self.L, entry)(self.ctx, self.h, delta, iters, ctypes.byref(o), ctypes.byref(out)))
+        t = time.perf_counter() - t
+        if fetch:
+            nv, nt = ctypes.c_size_t(), ctypes.c_size_t()
+            _lib.check(self.L.mc3d_mesh_counts(out, ctypes.byref(nv), ctypes.byref(nt)))
+            v, f = np.empty((nv.value, 3)), np.empty((nt.value, 3), dtype=np.uint32)
+            _lib.check(self.L.mc3d_mesh_copy(out, v.ctypes.data_as(ctypes.c_void_p), f.ctypes.data_as(ctypes.c_void_p)))
+        self.L.mc3d_mesh_free(out)
+        return (v, f) if fetch else t
+
+    def close(self):
+        self.b.release(self.h)
+        self.b.close()
+
+
+def _solid():
+    return m3.JoinedSolid([m3.Sphere((0.1, 0.0, -0.1), 0.8), m3.Cylinder((-0.6, -0.5, -0.4), (0.7, 0.6, 0.9), 0.3)])
+
+
+def test_calls_after_slabs():
+    c = _Calls(_solid())
+    for entry in ("mc3d_marching_cubes_interior", "mc3d_marching_cubes_search"):
+        best = []
+        for planes in (0, 5, 11, 23):  # before, and after slabs of several counts
+            if planes:
+                c.run("mc3d_marching_cubes_search", 0.03, 4, planes)
+            for _ in range(6):
+                c.run(entry, 0.05, 8)
+            best.append(min(c.run(entry, 0.05, 8) for _ in range(20)))
+        print(entry, [f"{1e6 * t:.1f} us" for t in best], flush=True)
+        assert max(best[1:]) < 1.4 * best[0] + 5e-6
+    c.close()
+
+
+@pytest.mark.parametrize("planes", [1, 2, 7, 64])
+def test_slabs_repeat(planes):
+    """More slabs than the pool keeps buffers, and few: twice the same mesh, the
+    whole grid's."""
+    s = _solid()
+    c = _Calls(s)
+    want = m3.MarchingCubesSearch(s, 0.025, 5)
+    for _ in range(2):
+        print(f"slabs of {planes}", flush=True)
+        v, f = c.run("mc3d_marching_cubes_search", 0.025, 5, planes, fetch=True)
+        assert same_triangles(v[f], want.triangles())
+    c.close()
