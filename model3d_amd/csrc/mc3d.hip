@@ -457,9 +457,10 @@ struct MeshBuffers {
     uint64_t nv = 0, nt = 0;  // of the whole call (the layout of `host`)
     ~MeshBuffers() {
         if (pool) {
-            pool->give(std::move(verts));
-            pool->give(std::move(tris));
+            // (the first taken last: the next call takes the same ones again)
             pool->give(std::move(interior));
+            pool->give(std::move(tris));
+            pool->give(std::move(verts));
         }
         if (hpool) hpool->give(std::move(host));
     }

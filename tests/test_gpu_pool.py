@@ -71,3 +71,20 @@ def test_slabs_repeat(planes):
         v, f = c.run("mc3d_marching_cubes_search", 0.025, 5, planes, fetch=True)
         assert same_triangles(v[f], want.triangles())
     c.close()
+
+
+def test_two_solids_in_turn():
+    """Two solids searched in turn, and with interior points: the outputs come
+    back to the same buffers each time, so a call takes what it takes alone."""
+    a, b = _Calls(_solid()), _Calls(m3.JoinedSolid([m3.Sphere((0.1, 0.0, -0.1), 0.8), m3.Capsule((-0.6, -0.5, -0.4), (0.7, 0.6, 0.9), 0.3)]))
+    for entry in ("mc3d_marching_cubes_interior", "mc3d_marching_cubes_search"):
+        def median(calls):
+            t = sorted(c.run(entry, 0.05, 8) for _ in range(20) for c in calls)
+            return t[len(t) // 2]
+
+        median([a, b])
+        alone, turns = max(median([a]), median([b])), median([a, b])
+        print(entry, f"alone {1e6 * alone:.1f} us, in turn {1e6 * turns:.1f} us", flush=True)
+        assert turns < 1.4 * alone + 5e-6
+    a.close()
+    b.close()
