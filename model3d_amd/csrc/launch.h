@@ -50,6 +50,7 @@ struct Pipe {
     bool scan_one_pass = false;  // classify scans its counts itself (at most SCAN_ONE_PASS blocks)
     bool rows = false;  // every atom has a row form: corners and bisection decide lines, not points
     int ray_rows = 0;   // the solid is a collider decided by rows, so many a wave (0: no)
+    bool ray_rest = false;  // its last halvings are lookups, a launch of their own
     int stack = 1;      // boolean stack entries of the call's programs
     uint32_t emit_div = 1024;  // emit blocks: occupancy words / emit_div, in [512, 4096]
 };

@@ -684,7 +684,7 @@ int prepare_job(Job &j, const mc3d_options &o, bool check = true) {
 // calls by points and by rows): edges of about 42 cells 124 and 213 us, 17
 // cells 133 and 149 us, 12 cells 334 and 207 us, 8 cells 262 and 124 us.
 bool ray_rows_pay(const RowScale &rs, double inv_cell) {
-    return rs.h > 0 && rs.eta < 0.01 && std::isfinite(rs.inv_h) && rs.h * inv_cell < 14;
+    return rs.h > 0 && rs.eta < RAY_ETA && std::isfinite(rs.inv_h) && rs.h * inv_cell < 14;
 }
 
 // The collider's triangles by planes, for rows of corners (k_rays.hip); none
@@ -1315,6 +1315,7 @@ Pipe make_pipe(const Call &c, const Upload &U) {
     p.wpb = c.wpb;
     p.rows = c.rows;
     p.ray_rows = c.nsegs == 1 && !c.stats && !c.host ? collider_rows(U) : 0;
+    p.ray_rest = p.ray_rows && !(bracket_eta(U.scale.mag, ldexp(U.scale.inv_h, U.hsegs[0].iters)) < RAY_ETA);
     p.stack = c.stack;
     p.plan_blocks = c.plan_blocks;
     // Launch shapes measured on MI355X.  A plan wave folds up to 64 bricks in

@@ -242,6 +242,9 @@ MC3D_HD inline void row_mask(const Span &s, double scale, double eta, int last, 
 MC3D_HD inline double row_eta(double mag, double inv_h) { return 1e-6 + 1e-11 * mag * inv_h; }
 MC3D_HD inline double bracket_eta(double mag, double scale) { return 1e-6 + 1e-15 * mag * scale; }
 
+// Bounds of a ray's interval are of use for points that stray less than this.
+constexpr double RAY_ETA = 0.01;
+
 // The point i / 2^levels of the bracket [a, b], as halvings reach it.
 MC3D_HD inline double bracket_point(double a, double b, int levels, int i) {
     double m = a;
