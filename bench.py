@@ -286,7 +286,9 @@ def algorithmic(stage, st):
               active brick and the 8 B occupancy words of the constant bricks
               (their share of the words taken as their share of the bricks)
     corners / bisect: the counted operations of every evaluated primitive,
-              transform and midpoint (float64, float32)
+              transform and midpoint (float64, float32) in a statistics run,
+              which evaluates point by point; the timed kernels decide whole
+              rows and edges, so this is no rate of theirs
     """
     n, v, t = st["corners"], st["vertices"], st["triangles"]
     words = st["words"]
@@ -310,8 +312,11 @@ def roofline_of(stage, ms, st):
         _, f64, f32 = kind
         # float64-equivalent rate: float32 runs at twice the float64 vector rate
         achieved = (f64 + f32 / 2) / (ms * 1e-3) / 1e12
-        r = {"bound": "valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s",
-             "frac": achieved / FP64_PEAK_TFLOPS, "flops64_per_launch": f64, "flops32_per_launch": f32}
+        # (the workloads' kernels decide whole lines: what is counted are the
+        # operations of evaluating each point, which they do not execute)
+        r = {"bound": "valu", "achieved": achieved, "peak": FP64_PEAK_TFLOPS, "unit": "TFLOP/s", "frac": None,
+             "achieved_of": "the operations of evaluating every point; the kernel decides lines with fewer",
+             "flops64_per_launch": f64, "flops32_per_launch": f32}
     else:
         achieved = kind[1] / (ms * 1e-3) / 1e9
         r = {"bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
@@ -521,7 +526,7 @@ def config_entry(name, steps=5, warmup=2):
 
 
 def sphere_batched(copies=64, steps=5):
-    """The north-star comparison on config 1: `copies` spheres (C1) meshed by
+    """`copies` unit spheres at delta 0.02 meshed by
     one batch call in float32 + guard, against the plain float64 GPU path
     (every atom at every corner, one call per sphere), corner evals/s."""
     c = dict(workload("sphere"))
@@ -625,7 +630,8 @@ def main():
         "tris_per_s": tris / (wall / args.steps),
         "ms_device": mean(st, "ms_device"),
     }
-    # The same steps in both precisions (bit-identical results).
+    # The same steps in both precisions (bit-identical results; solids with a row
+    # form, and a collider alone, run the same float64 kernels in both).
     other = "fp32_guard" if run["precision"] == "fp64" else "fp64"
     wall_o, _ = run_gpu(work, dict(run, precision=other), args.steps, args.warmup)
     result["precisions_ms_per_step"] = {run["precision"]: ms, other: 1e3 * wall_o / args.steps}
@@ -648,6 +654,7 @@ def main():
         _, gst = run_gpu(work, dict(run, precision="fp32_guard"), 1, 0, count_mismatch=True)
         g = gst[0]
     result["guard"] = {
+        "of": "a statistics run, point by point (timed calls of these solids decide lines in float64)",
         "fp32_atom_evals": g["guard_evals"],
         "fp64_rechecks": g["guard_rechecks"],
         "fp64_fallback_fraction": g["guard_rechecks"] / g["guard_evals"] if g["guard_evals"] else None,

@@ -130,8 +130,17 @@ mc3d_solid *mc3d_solid_retain(mc3d_solid *s);
 void mc3d_solid_release(mc3d_solid *s);
 /* Solid.Min() / Solid.Max() with the reference's float64 arithmetic. */
 int mc3d_solid_bounds(const mc3d_solid *s, double min[3], double max[3]);
+/* *row_form = 1 if every primitive is a sphere, box, capsule or cylinder in no
+ * transform's frame, so that searches decide whole rows of corners and whole
+ * edges at a time; else 0. */
+int mc3d_solid_row_form(const mc3d_solid *s, int32_t *row_form);
 
 /* ---- meshing ----------------------------------------------------------- */
+/* Solids with a row form (mc3d_solid_row_form) and searches of a mesh collider
+ * alone are decided line by line in float64: precision, rows_per_walk and
+ * waves_per_brick choose nothing for them, except in a statistics run
+ * (count_mismatch), which evaluates point by point.  The mesh is the same
+ * either way. */
 enum {
     MC3D_PREC_FP64 = 0,       /* every primitive evaluated in float64 */
     MC3D_PREC_FP32_GUARD = 1, /* float32 with an error band; in-band points re-decided in float64 */
@@ -143,8 +152,9 @@ typedef struct {
                           * (mc3d_mesh_host_ptrs), the triangles while the bisection runs */
     int32_t count_mismatch; /* 1: also count float32 sign mismatches (slower; statistics only) */
     int32_t brick;       /* culling brick: 64 x brick x brick corners (0: default 4) */
-    int32_t rows_per_walk; /* grid rows evaluated per walk of a brick program: 1, 2 or 4 (0: default 1) */
-    int32_t waves_per_brick; /* wavefronts sharing one brick: 1, 2 or 4 (0: default 4) */
+    int32_t rows_per_walk; /* point by point: grid rows evaluated per walk of a brick program: 1, 2 or 4
+                            * (0: default 1) */
+    int32_t waves_per_brick; /* point by point: wavefronts sharing one brick: 1, 2 or 4 (0: default 4) */
     int32_t no_graph;    /* 1: enqueue the stages one by one (per-stage timings in mc3d_stats); 0: a call
                           * left on the device runs its chain as one HIP graph launch, captured once per
                           * call shape and replayed (only ms_device is timed then) */

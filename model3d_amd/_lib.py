@@ -128,6 +128,7 @@ SIGNATURES = {
     "mc3d_solid_retain": (_P, [_P]),
     "mc3d_solid_release": (None, [_P]),
     "mc3d_solid_bounds": (ctypes.c_int, [_P, _D3, _D3]),
+    "mc3d_solid_row_form": (ctypes.c_int, [_P, ctypes.POINTER(ctypes.c_int32)]),
     "mc3d_marching_cubes_search": (
         ctypes.c_int,
         [_P, _P, ctypes.c_double, ctypes.c_int, ctypes.POINTER(mc3d_options), ctypes.POINTER(_P)],

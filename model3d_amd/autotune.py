@@ -1,13 +1,16 @@
 """Tile-shape autotuner for MarchingCubesSearch.
 
 Three shapes matter on the GPU: the culling brick (64 x B x B corners:
-smaller bricks fold programs tighter but cost more planning), how many grid
-rows one walk of a brick program evaluates (more rows amortise the walk,
-fewer keep register use and latency down) and how many wavefronts share a
-brick (fewer give each wave more rows behind one staging of the program,
-more put more waves on the brick's latency chain).  ``tune`` times each candidate on the
-actual solid and grid (results on the device, nothing copied back) and
-returns the fastest; every candidate produces the same triangles.
+smaller bricks fold programs tighter but cost more planning) and, where
+corners are evaluated point by point, how many grid rows one walk of a brick
+program evaluates (more rows amortise the walk, fewer keep register use and
+latency down) and how many wavefronts share a brick (fewer give each wave more
+rows behind one staging of the program, more put more waves on the brick's
+latency chain).  Solids with a row form (every primitive a sphere, box, capsule
+or cylinder, untransformed) decide whole rows instead, and only the brick is
+searched.  ``tune`` times each candidate on the actual solid and grid (results
+on the device, nothing copied back) and returns the fastest; every candidate
+produces the same triangles.
 """
 from __future__ import annotations
 
@@ -65,6 +68,13 @@ def tune(
     hs = [x._build(b) for x in solids]
     table = []
     try:
+        form = ctypes.c_int32()
+        by_rows = True
+        for h in hs:
+            _lib.check(L.mc3d_solid_row_form(h, ctypes.byref(form)))
+            by_rows = by_rows and form.value != 0
+        if by_rows:  # (of these two, any candidate: they choose nothing)
+            rows_per_walk, waves_per_brick = rows_per_walk[:1], waves_per_brick[-1:]
         for brick, rpw, wpb in itertools.product(bricks, rows_per_walk, waves_per_brick):
             o = _lib.mc3d_options()
             o.precision, o.cull, o.device_only = precision, 1, 1

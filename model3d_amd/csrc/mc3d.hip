@@ -2395,6 +2395,19 @@ int mc3d_marching_cubes_c2f(mc3d_ctx *ctx, const mc3d_solid *s, double big_delta
     });
 }
 
+int mc3d_solid_row_form(const mc3d_solid *s, int32_t *row_form) {
+    if (!s || !row_form) {
+        set_error("mc3d_solid_row_form: null argument");
+        return MC3D_E_INVALID_ARG;
+    }
+    return guarded([&]() -> int {
+        std::shared_ptr<const Lowered> low;
+        const int rc = lowered(s, low);
+        if (!rc) *row_form = low->rows && !low->host ? 1 : 0;
+        return rc;
+    });
+}
+
 int mc3d_marching_cubes_search(mc3d_ctx *ctx, const mc3d_solid *s, double delta, int iters,
                                const mc3d_options *opts, mc3d_mesh **out) {
     if (!ctx || !s || !out) {

@@ -176,3 +176,25 @@ def test_row_bounds_with_the_kernels_tolerances():
     assert L.mc3d_selftest_rows(91, 1000000, ctypes.byref(checked), ctypes.byref(opened), ctypes.byref(bad)) == 0
     assert checked.value > 1000000 * 32
     assert bad.value == 0
+
+
+def test_row_form():
+    """Which solids decide whole rows: the untransformed primitives with convex
+    quadric surfaces or flat sides, in any tree."""
+    import ctypes
+
+    from model3d_amd.solids import LibBackend
+
+    cat = solid_catalogue()
+    want = {"sphere", "rect", "capsule", "cylinder", "csg", "force_bounds", "clipped"}
+    b = LibBackend()
+    form = ctypes.c_int32()
+    got = set()
+    for name, s in cat.items():
+        h = s._build(b)
+        assert _lib.lib().mc3d_solid_row_form(h, ctypes.byref(form)) == 0
+        if form.value:
+            got.add(name)
+        b.release(h)
+    b.close()
+    assert got == want
