@@ -1,8 +1,9 @@
 """A mesh collider's triangles by planes: made for a search that decides its
 rows by them, and not before."""
+import ctypes
+
 import numpy as np
 import pytest
-import torch
 
 import model3d_amd as m3
 from model3d_amd import _lib
@@ -13,8 +14,14 @@ pytestmark = pytest.mark.gpu
 
 
 def _free():
-    torch.cuda.synchronize()
-    return torch.cuda.mem_get_info()[0]
+    """Free device memory, asked of the HIP runtime that the library links:
+    its symbols are found through the library, and no second runtime (torch
+    brings its own) comes into the process."""
+    L = _lib.lib()
+    free, total = ctypes.c_size_t(), ctypes.c_size_t()
+    assert L.hipDeviceSynchronize() == 0
+    assert L.hipMemGetInfo(ctypes.byref(free), ctypes.byref(total)) == 0
+    return free.value
 
 
 def test_planes_only_for_rows():
