@@ -164,7 +164,7 @@ __device__ __forceinline__ uint64_t bracket_bits(CodeP code, uint32_t n, F64P f6
 // Evaluating every halving is a chain of dependent program walks, bound by the
 // latency of its loads where few waves run (a small part) and by the walks'
 // scalar and vector issue where many do; one walk decides six halvings here.
-// Bound by vector issue now, at 3 waves per SIMD (144 registers; 168 for several
+// Bound by vector issue now, at 3 waves per SIMD (138 registers; 159 for several
 // solids).  UNI: one program for the wave.
 template <bool UNI>
 __device__ __forceinline__ void halve(const Insn *code, uint32_t n, const DevProg &P, const Grid &g, int k, double px, double py,
